@@ -161,14 +161,11 @@ void UNet3D::ensureTraining()
     ge3_.allocate(h * m2 * 64);
     gd2_.allocate(h * m1 * 32);
     gp_.allocate(h * std::max(m2 * 32, m1 * 16));
-    size_t wpart = 0, bpart = 0;
-    for (const Layer& L : layers_) {
-        const size_t chunks = (size_t)nn::wgrad_chunks(voxels(L.level));
-        wpart = std::max(wpart, chunks * 27 * L.cout * ((L.cin + 15) / 16 * 16));
-        bpart = std::max(bpart, chunks * L.cout);
-    }
+    size_t wpart = 0;
+    for (const Layer& L : layers_)
+        wpart = std::max(wpart, nn::wgrad_partial_floats(D_[L.level], H_[L.level], W_[L.level],
+                                                         std::max(L.cin, kInputChannels), L.cout));
     wpart_.allocate(sizeof(float) * wpart);
-    bpart_.allocate(sizeof(float) * bpart);
     hpart_.allocate(sizeof(float) * 1024 * 17);
     loss_.allocate(sizeof(double));
     lpart_.allocate(sizeof(double) * 1024);
@@ -183,9 +180,7 @@ void UNet3D::backward()
         const int D = D_[L.level], H = H_[L.level], W = W_[L.level];
         const size_t M = voxels(L.level);
         nn::relu_backward(gy, layerOutput(i), M * L.cout, stream_);
-        nn::conv3_weight_grad(layerInput(i), D, H, W, gy, L.cout, wpart_.as<float>(), stream_);
-        nn::conv3_weight_grad_reduce(wpart_.as<float>(), nn::wgrad_chunks(M), L.cout, L.cin, g + L.w, stream_);
-        nn::channel_sum(gy, M, L.cout, bpart_.as<float>(), g + L.b, stream_);
+        nn::conv3_weight_grad(layerInput(i), D, H, W, gy, L.cin, L.cout, wpart_.as<float>(), g + L.w, g + L.b, stream_);
         if (gx) {
             nn::ConvArgs a;
             a.src.a = gy;

@@ -62,7 +62,7 @@ private:
     std::vector<DeviceBuffer> act_;                 // output of each layer (bf16)
     // training buffers
     bool training_ = false;
-    DeviceBuffer gpred_, gd1_, gtmp_, gcat_, ge1_, ge2_, ge3_, gd2_, gp_, wpart_, bpart_, hpart_, loss_, lpart_;
+    DeviceBuffer gpred_, gd1_, gtmp_, gcat_, ge1_, ge2_, ge3_, gd2_, gp_, wpart_, hpart_, loss_, lpart_;
     int adam_t_ = 0;
 };
 

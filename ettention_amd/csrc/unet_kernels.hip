@@ -11,10 +11,9 @@
 // B[k][j] in lane j + 16 (k / 8); D[i][j] in lane j + 16 (i / 4), element i % 4.
 //
 // The weight gradient is the GEMM dW[co][(tap, ci)] = sum_m gy[m][co] x[m + d(tap)][ci]
-// with the voxels as the reduction: a workgroup takes one tap and a chunk of
-// voxels, stages gy and the tap-shifted input transposed in LDS (32 voxels at
-// a time) and accumulates all (co, ci) tiles; the per-chunk partials are then
-// summed in a fixed order, so every gradient is deterministic.
+// with the voxels as the reduction, over LDS-staged bricks read transposed
+// (conv3_wgrad_kernel); the workgroups' partial sums are added in a fixed
+// order, so every gradient is deterministic.
 #include <algorithm>
 
 #include "common.hpp"
@@ -273,146 +272,194 @@ void launch_conv(const ConvArgs& a, hipStream_t stream)
     conv3_fwd_kernel<NT, MT><<<grid, kThreads, 0, stream>>>(a);
 }
 
-// ---- weight gradient ----------------------------------------------------------
-constexpr int kLdsRow = 40;        // 32 voxels + 8 pad (bf16), 80-byte rows keep 16-byte alignment
+// ---- weight and bias gradient -------------------------------------------------
+// A workgroup takes 16 input channels, all output channels (NT tiles of 16),
+// all 27 taps and every chunk-th brick of kWZ x kWY x kWX voxels.  Both
+// operands of the GEMM need 8 voxels of one channel per lane while memory
+// holds 8 channels of one voxel: the input brick with its halo and the output
+// gradient's brick are staged as they are ([voxel][16 channels], 16-byte
+// cells) and read through ds_read_b64_tr_b16, which hands lane i of a 16-lane
+// group column i of 4 voxels x 16 channels.  A tap is then a row and column
+// offset into the halo, and the 27 taps read each staged voxel from LDS.  A
+// 32-wide k step is one x row of the brick; lane group kg holds voxels
+// 16 h + 4 kg + {0..3} (h = 0, 1) in both operands, so that one read of the
+// wave covers 512 contiguous bytes (the k order only has to agree between A
+// and B).  Wave w accumulates taps w, w + 4, ...; its slot past tap 26
+// multiplies the gradient by one: the bias gradient.
+// Bound by the LDS reads (two 8-byte reads a lane per MFMA and NT); the
+// version that staged one tap's transposed operands through 2-byte LDS writes
+// took 8.0 ms for the ten layers at 128^3, 27 passes over both operands.
+constexpr int kWZ = 4, kWY = 4, kWX = 32;
+constexpr int kWHZ = kWZ + 2, kWHY = kWY + 2, kWHX = kWX + 2;
+constexpr int kWVoxels = kWZ * kWY * kWX;                       // 512
+constexpr int kWHalo = kWHZ * kWHY * kWHX;                      // 1224
+constexpr int kWTaps = (27 + kConvWaves - 1) / kConvWaves;      // tap slots per wave
 constexpr int kMaxCout = 64;
-constexpr int kMaxCin = 96;
 
 struct WgradArgs {
     ConvSrc src;
     int D, H, W;
     const uint16_t* gy;
-    int cout;
-    int chunk;          // voxels per workgroup, multiple of 32
-    float* partial;     // [chunks][27][cout][cin16]
+    int cout, cin16;
+    int nbx, nby, bricks;
+    float* partial;     // [chunk][27 * cout * cin16 weights, then cout biases]
 };
 
-__global__ void __launch_bounds__(kThreads) conv3_wgrad_kernel(WgradArgs w)
-{
-    __shared__ __attribute__((aligned(16))) uint16_t gyT[kMaxCout * kLdsRow];
-    __shared__ __attribute__((aligned(16))) uint16_t xT[kMaxCin * kLdsRow];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = lane & 15, kg = lane >> 4;
-    const int t = blockIdx.y;
-    const int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
-    const size_t M = (size_t)w.D * w.H * w.W;
-    const int HW = w.H * w.W;
-    const int ca = w.src.ca, cin = w.src.ca + w.src.cb;
-    const int cin16 = (cin + 15) / 16 * 16;
-    const int nco = w.cout / 16, nci = cin16 / 16, ntiles = nco * nci;
-    const int Hh = w.H >> 1, Wh = w.W >> 1;
-    const size_t mbeg = (size_t)blockIdx.x * w.chunk;
-    floatx4 acc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+#ifdef __HIP_DEVICE_COMPILE__
+#define ETN_LDS __attribute__((address_space(3)))
+#else
+#define ETN_LDS
+#endif
 
-    for (int s = 0; s < w.chunk; s += 32) {
-        const size_t ms = mbeg + s;
-        // gy rows of 32 voxels, transposed: gyT[co][voxel]
-        const int gpv = w.cout / 8;
-        for (int g = threadIdx.x; g < 32 * gpv; g += kThreads) {
-            const int mi = g / gpv, c0 = (g - mi * gpv) * 8;
-            const size_t m = ms + mi;
-            u32x4 v = u32x4{0u, 0u, 0u, 0u};
-            if (m < M) v = load16(w.gy + m * w.cout + c0);
+// 8 voxels of one channel per lane (see above); cell: the lane's 8 bytes of
+// the first 16 voxels, the second 16 are 512 bytes on
+__device__ __forceinline__ bf16x8 load_voxels(const char* cell)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ETN_LDS i16x4*)(cell));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ETN_LDS i16x4*)(cell + 512));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#else
+    return as_bf16x8(*reinterpret_cast<const u32x4*>(cell));   // the host pass only parses this
+#endif
+}
+
+template <int NT>
+__global__ void __launch_bounds__(kThreads, NT == 4 ? 1 : 2) conv3_wgrad_kernel(WgradArgs w)
+{
+    __shared__ u32x4 xs[kWHalo * 2];          // [halo voxel][2 cells of 8 channels]
+    __shared__ u32x4 gs[NT * kWVoxels * 2];   // [channel tile][voxel][2 cells]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int col = lane & 15, kg = lane >> 4;
+    const int ci0 = blockIdx.y * 16;
+    const int ca = w.src.ca, cin = w.src.ca + w.src.cb;
+    const int Hh = w.H >> 1, Wh = w.W >> 1;
+    const u32x4 zero4 = u32x4{0u, 0u, 0u, 0u};
+    const bf16x8 ones = as_bf16x8(u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+
+    floatx4 acc[kWTaps][NT];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                gyT[(c0 + 2 * e) * kLdsRow + mi] = (uint16_t)(v[e] & 0xffffu);
-                gyT[(c0 + 2 * e + 1) * kLdsRow + mi] = (uint16_t)(v[e] >> 16);
-            }
-        }
-        // tap-shifted input, transposed: xT[ci][voxel]
-        {
-            const int gpx = cin / 8;
-            for (int g = threadIdx.x; g < 32 * gpx; g += kThreads) {
-                const int mi = g / gpx, c0 = (g - mi * gpx) * 8;
-                const size_t m = ms + mi;
-                u32x4 v = u32x4{0u, 0u, 0u, 0u};
-                if (m < M) {
-                    const int z = (int)(m / HW), r = (int)(m - (size_t)z * HW), y = r / w.W, x = r - y * w.W;
-                    const int zz = z + dz, yy = y + dy, xx = x + dx;
-                    if ((unsigned)zz < (unsigned)w.D && (unsigned)yy < (unsigned)w.H && (unsigned)xx < (unsigned)w.W) {
-                        if (c0 < ca) {
-                            const size_t vi = w.src.a_half ? ((size_t)(zz >> 1) * Hh + (yy >> 1)) * Wh + (xx >> 1)
-                                                           : ((size_t)zz * w.H + yy) * w.W + xx;
-                            v = load16(w.src.a + vi * ca + c0);
-                        } else {
-                            v = load16(w.src.b + (((size_t)zz * w.H + yy) * w.W + xx) * w.src.cb + (c0 - ca));
-                        }
-                    }
-                }
+    for (int i = 0; i < kWTaps; ++i)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    xT[(c0 + 2 * e) * kLdsRow + mi] = (uint16_t)(v[e] & 0xffffu);
-                    xT[(c0 + 2 * e + 1) * kLdsRow + mi] = (uint16_t)(v[e] >> 16);
-                }
-            }
-        }
-        __syncthreads();
+        for (int nt = 0; nt < NT; ++nt) acc[i][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // the lane's cell of a row's first 16 voxels: voxel 4 kg + (lane & 15) / 4,
+    // channels 4 (lane % 4) ..
+    const int lane_cell = (4 * kg + (col >> 2)) * 32 + (col & 3) * 8;
+    const char* xbase = reinterpret_cast<const char*>(xs) + lane_cell;
+    const char* gbase = reinterpret_cast<const char*>(gs) + lane_cell;
+    int tap_off[kWTaps];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int tile = wave + 4 * i;
-            if (tile < ntiles) {
-                const int ct = tile / nci, it = tile - ct * nci;
-                const bf16x8 A = as_bf16x8(*reinterpret_cast<const u32x4*>(&gyT[(ct * 16 + row) * kLdsRow + kg * 8]));
-                const bf16x8 B = as_bf16x8(*reinterpret_cast<const u32x4*>(&xT[(it * 16 + row) * kLdsRow + kg * 8]));
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[i], 0, 0, 0);
-            }
-        }
-        __syncthreads();
+    for (int i = 0; i < kWTaps; ++i) {
+        const int t = wave + kConvWaves * i;
+        tap_off[i] = (((t / 9) * kWHY + (t / 3) % 3) * kWHX + t % 3) * 32;
     }
+
+    for (int b = blockIdx.x; b < w.bricks; b += gridDim.x) {
+        const int bxi = b % w.nbx, rest = b / w.nbx, byi = rest % w.nby, bzi = rest / w.nby;
+        const int x0 = bxi * kWX, y0 = byi * kWY, z0 = bzi * kWZ;
+        __syncthreads();   // the previous brick's reads are done
+        for (int e = tid; e < kWHalo * 2; e += kThreads) {
+            const int v = e >> 1, c = ci0 + (e & 1) * 8;
+            const int hz = v / (kWHY * kWHX), r2 = v - hz * (kWHY * kWHX), hy = r2 / kWHX, hx = r2 - hy * kWHX;
+            const int zz = z0 - 1 + hz, yy = y0 - 1 + hy, xx = x0 - 1 + hx;
+            u32x4 cell = zero4;
+            if (c < cin && (unsigned)zz < (unsigned)w.D && (unsigned)yy < (unsigned)w.H && (unsigned)xx < (unsigned)w.W) {
+                if (c < ca) {
+                    const size_t vi = w.src.a_half ? ((size_t)(zz >> 1) * Hh + (yy >> 1)) * Wh + (xx >> 1)
+                                                   : ((size_t)zz * w.H + yy) * w.W + xx;
+                    cell = load16(w.src.a + vi * ca + c);
+                } else {
+                    cell = load16(w.src.b + (((size_t)zz * w.H + yy) * w.W + xx) * w.src.cb + (c - ca));
+                }
+            }
+            xs[e] = cell;
+        }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int tile = wave + 4 * i;
-        if (tile < ntiles) {
-            const int ct = tile / nci, it = tile - ct * nci;
+        for (int k = 0; k < NT * kWVoxels * 2 / kThreads; ++k) {
+            const int e = k * kThreads + tid;
+            const int v = e / (2 * NT), c = e - v * (2 * NT);
+            const int z = z0 + v / (kWY * kWX), y = y0 + (v / kWX) % kWY, x = x0 + v % kWX;
+            u32x4 cell = zero4;
+            if (z < w.D && y < w.H && x < w.W) cell = load16(w.gy + (((size_t)z * w.H + y) * w.W + x) * w.cout + c * 8);
+            gs[((c >> 1) * kWVoxels + v) * 2 + (c & 1)] = cell;
+        }
+        __syncthreads();
+#pragma unroll 2
+        for (int row = 0; row < kWZ * kWY; ++row) {
+            bf16x8 A[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) A[nt] = load_voxels(gbase + (nt * kWVoxels + row * kWX) * 32);
+            const char* xrow = xbase + (((row / kWY) * kWHY + row % kWY) * kWHX) * 32;
+#pragma unroll
+            for (int i = 0; i < kWTaps; ++i) {
+                const bool tap = i + 1 < kWTaps || wave + kConvWaves * i < 27;   // uniform in the wave
+                const bf16x8 B = tap ? load_voxels(xrow + tap_off[i]) : ones;
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    acc[i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[nt], B, acc[i][nt], 0, 0, 0);
+            }
+        }
+    }
+    float* out = w.partial + (size_t)blockIdx.x * ((size_t)27 * w.cout * w.cin16 + w.cout);
+#pragma unroll
+    for (int i = 0; i < kWTaps; ++i) {
+        const int t = wave + kConvWaves * i;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int co = ct * 16 + kg * 4 + r, ci = it * 16 + row;
-                w.partial[(((size_t)blockIdx.x * 27 + t) * w.cout + co) * cin16 + ci] = acc[i][r];
+                const int co = nt * 16 + kg * 4 + r;
+                if (t < 27) out[((size_t)t * w.cout + co) * w.cin16 + ci0 + col] = acc[i][nt][r];
+                else if (ci0 == 0 && col == 0) out[(size_t)27 * w.cout * w.cin16 + co] = acc[i][nt][r];
             }
-        }
     }
 }
 
-__global__ void wgrad_reduce_kernel(const float* partial, int chunks, int cout, int cin, int cin16, float* dw)
-{
-    const int n = cout * 27 * cin;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int co = i / (27 * cin), r = i - co * 27 * cin, t = r / cin, ci = r - t * cin;
-    const size_t stride = (size_t)27 * cout * cin16;
-    const float* p = partial + ((size_t)t * cout + co) * cin16 + ci;
-    float s = 0.0f;
-    for (int c = 0; c < chunks; ++c) s += p[c * stride];
-    dw[i] = s;
-}
-
-__global__ void channel_sum_partial_kernel(const uint16_t* g, size_t voxels, int C, int chunk, float* partial)
+// Sum of `chunks` rows of n partial sums, rows `stride` apart: kSumLanes
+// threads share a column, each adding every kSumLanes-th row in order, then
+// the lanes are added in order (deterministic).  One thread per column left
+// the few columns of a bias waiting on thousands of dependent loads: 3.0 ms
+// of a 128^3 gradient, and 6.6 ms for the weights.
+constexpr int kSumColumns = 32, kSumLanes = kThreads / kSumColumns;
+template <typename Store>
+__device__ __forceinline__ void sum_rows(const float* partial, int chunks, size_t stride, int n, Store&& store)
 {
     __shared__ float red[kThreads];
-    const int lanes = kThreads / C;   // voxel lanes per channel
-    const int ch = threadIdx.x % C, j = threadIdx.x / C;
-    const size_t beg = (size_t)blockIdx.x * chunk, end = std::min(voxels, beg + chunk);
+    const int c = threadIdx.x % kSumColumns, l = threadIdx.x / kSumColumns;
+    const int i = blockIdx.x * kSumColumns + c;
     float s = 0.0f;
-    if (j < lanes)
-        for (size_t m = beg + j; m < end; m += lanes) s += bf2f(g[m * C + ch]);
+    if (i < n) {
+#pragma unroll 8
+        for (int k = l; k < chunks; k += kSumLanes) s += partial[(size_t)k * stride + i];
+    }
     red[threadIdx.x] = s;
     __syncthreads();
-    if (threadIdx.x < C) {
+    if (l == 0 && i < n) {
         float t = 0.0f;
-        for (int q = 0; q < lanes; ++q) t += red[q * C + threadIdx.x];
-        partial[(size_t)blockIdx.x * C + threadIdx.x] = t;
+        for (int q = 0; q < kSumLanes; ++q) t += red[q * kSumColumns + c];
+        store(i, t);
     }
 }
 
-__global__ void sum_partials_kernel(const float* partial, int chunks, int C, float* out)
+__global__ void __launch_bounds__(kThreads) wgrad_reduce_kernel(const float* partial, int chunks, int cout, int cin,
+                                                                int cin16, float* dw, float* db)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    float s = 0.0f;
-    for (int k = 0; k < chunks; ++k) s += partial[(size_t)k * C + c];
-    out[c] = s;
+    const int nw = 27 * cout * cin16;
+    sum_rows(partial, chunks, (size_t)nw + cout, nw + cout, [&](int i, float v) {
+        if (i >= nw) {
+            db[i - nw] = v;
+            return;
+        }
+        const int t = i / (cout * cin16), r = i - t * cout * cin16, co = r / cin16, ci = r - co * cin16;
+        if (ci < cin) dw[((size_t)co * 27 + t) * cin + ci] = v;
+    });
+}
+
+__global__ void __launch_bounds__(kThreads) sum_partials_kernel(const float* partial, int chunks, int C, float* out)
+{
+    sum_rows(partial, chunks, (size_t)C, C, [&](int i, float v) { out[i] = v; });
 }
 
 __global__ void pack_weights_kernel(const float* w, int cout, int cin, int cin_pad, uint16_t* wt, int kpad,
@@ -547,13 +594,18 @@ __global__ void mse_partial_kernel(const float* pred, const float* target, float
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-__global__ void mse_final_kernel(const double* partial, int blocks, size_t n, double* loss)
+__global__ void __launch_bounds__(kThreads) mse_final_kernel(const double* partial, int blocks, size_t n, double* loss)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (int b = 0; b < blocks; ++b) s += partial[b];
-        *loss = s / (double)n;
+    __shared__ double red[kThreads];
+    double s = 0.0;
+    for (int b = threadIdx.x; b < blocks; b += kThreads) s += partial[b];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = kThreads / 2; w > 0; w /= 2) {
+        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        __syncthreads();
     }
+    if (threadIdx.x == 0) *loss = red[0] / (double)n;
 }
 
 __global__ void head_backward_kernel(const uint16_t* d1, const float* gp, const float* hw, size_t n, uint16_t* gd1,
@@ -620,33 +672,37 @@ void conv3_forward(const ConvArgs& a, hipStream_t stream)
     hip_check(hipGetLastError(), "conv3 forward launch");
 }
 
-void conv3_weight_grad(const ConvSrc& src, int D, int H, int W, const uint16_t* gy, int cout, float* partial,
-                       hipStream_t stream)
+int wgrad_chunks(int D, int H, int W, int cin)
 {
-    if (cout % 16 || cout > kMaxCout || src.ca + src.cb > kMaxCin || src.ca % 8 || src.cb % 8)
+    // two workgroups per CU over all channel chunks, at most one per brick:
+    // more only adds partial sums to write and read back
+    const int bricks = ((W + kWX - 1) / kWX) * ((H + kWY - 1) / kWY) * ((D + kWZ - 1) / kWZ);
+    return std::min(bricks, std::max(1, 512 / ((cin + 15) / 16)));
+}
+
+size_t wgrad_partial_floats(int D, int H, int W, int cin, int cout)
+{
+    return (size_t)wgrad_chunks(D, H, W, cin) * ((size_t)27 * cout * ((cin + 15) / 16 * 16) + cout);
+}
+
+void conv3_weight_grad(const ConvSrc& src, int D, int H, int W, const uint16_t* gy, int cin, int cout, float* partial,
+                       float* dw, float* db, hipStream_t stream)
+{
+    if (cout % 16 || cout > kMaxCout || cout == 48 || src.ca % 8 || src.cb % 8 || cin > src.ca + src.cb)
         fail("conv3 weight gradient: channel counts");
-    WgradArgs w{src, D, H, W, gy, cout, kWgradChunk, partial};
-    const size_t M = (size_t)D * H * W;
-    const dim3 grid((unsigned)wgrad_chunks(M), 27);
-    conv3_wgrad_kernel<<<grid, kThreads, 0, stream>>>(w);
+    const int cin16 = (src.ca + src.cb + 15) / 16 * 16, chunks = wgrad_chunks(D, H, W, src.ca + src.cb);
+    const int nbx = (W + kWX - 1) / kWX, nby = (H + kWY - 1) / kWY, nbz = (D + kWZ - 1) / kWZ;
+    WgradArgs w{src, D, H, W, gy, cout, cin16, nbx, nby, nbx * nby * nbz, partial};
+    const dim3 grid((unsigned)chunks, (unsigned)(cin16 / 16));
+    switch (cout / 16) {
+        case 1: conv3_wgrad_kernel<1><<<grid, kThreads, 0, stream>>>(w); break;
+        case 2: conv3_wgrad_kernel<2><<<grid, kThreads, 0, stream>>>(w); break;
+        default: conv3_wgrad_kernel<4><<<grid, kThreads, 0, stream>>>(w); break;
+    }
+    const int n = 27 * cout * cin16 + cout;
+    wgrad_reduce_kernel<<<(n + kSumColumns - 1) / kSumColumns, kThreads, 0, stream>>>(partial, chunks, cout, cin, cin16,
+                                                                                     dw, db);
     hip_check(hipGetLastError(), "conv3 weight gradient launch");
-}
-
-void conv3_weight_grad_reduce(const float* partial, int chunks, int cout, int cin, float* dw, hipStream_t stream)
-{
-    const int n = cout * 27 * cin;
-    const int cin16 = (cin + 15) / 16 * 16;
-    wgrad_reduce_kernel<<<(n + kThreads - 1) / kThreads, kThreads, 0, stream>>>(partial, chunks, cout, cin, cin16, dw);
-    hip_check(hipGetLastError(), "weight gradient reduction launch");
-}
-
-void channel_sum(const uint16_t* g, size_t voxels, int channels, float* partial, float* out, hipStream_t stream)
-{
-    if (channels > kThreads || kThreads % channels) fail("channel_sum: channel count");
-    const int chunks = wgrad_chunks(voxels);
-    channel_sum_partial_kernel<<<chunks, kThreads, 0, stream>>>(g, voxels, channels, kWgradChunk, partial);
-    sum_partials_kernel<<<1, 128, 0, stream>>>(partial, chunks, channels, out);
-    hip_check(hipGetLastError(), "channel sum launch");
 }
 
 void pack_weights(const float* w, int cout, int cin, int cin_pad, uint16_t* wt, uint16_t* wb, hipStream_t stream)
@@ -709,14 +765,14 @@ void mse_loss(const float* pred, const float* target, float scale, size_t voxels
               double* loss, hipStream_t stream)
 {
     mse_partial_kernel<<<kRedBlocks, kThreads, 0, stream>>>(pred, target, scale, voxels, g_pred, partial);
-    mse_final_kernel<<<1, 64, 0, stream>>>(partial, kRedBlocks, voxels, loss);
+    mse_final_kernel<<<1, kThreads, 0, stream>>>(partial, kRedBlocks, voxels, loss);
 }
 
 void head_backward(const uint16_t* d1, const float* g_pred, const float* hw, size_t voxels, uint16_t* g_d1,
                    float* partial, float* ghw_ghb, hipStream_t stream)
 {
     head_backward_kernel<<<kRedBlocks, kThreads, 0, stream>>>(d1, g_pred, hw, voxels, g_d1, partial);
-    sum_partials_kernel<<<1, 64, 0, stream>>>(partial, kRedBlocks, 17, ghw_ghb);
+    sum_partials_kernel<<<1, kThreads, 0, stream>>>(partial, kRedBlocks, 17, ghw_ghb);
 }
 
 void adam_step(float* p, const float* g, float* m, float* v, size_t count, float lr, float beta1, float beta2,

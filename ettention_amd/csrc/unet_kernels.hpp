@@ -35,21 +35,16 @@ struct ConvArgs {
     uint16_t* out = nullptr;      // [D][H][W][cout] bf16
 };
 
-// Columns of the weight-gradient GEMM per workgroup.
-constexpr int kWgradChunk = 512;
-
 inline int kpad_for(int cin) { return (27 * cin + 31) / 32 * 32; }
-inline int wgrad_chunks(size_t voxels) { return (int)((voxels + kWgradChunk - 1) / kWgradChunk); }
 
 // y = act(conv3(src) + bias)
 void conv3_forward(const ConvArgs& a, hipStream_t stream);
-// partial[c][tap][co][ci16] = sum over voxels of chunk c of gy[m][co] * x[m + d(tap)][ci]
-void conv3_weight_grad(const ConvSrc& src, int D, int H, int W, const uint16_t* gy, int cout, float* partial,
-                       hipStream_t stream);
-// dw[co][tap][ci] (fp32, scaled by `scale` and added to dw when accumulate) from the partials
-void conv3_weight_grad_reduce(const float* partial, int chunks, int cout, int cin, float* dw, hipStream_t stream);
-// partial[c][ch] = sum over the voxels of chunk c; then out[ch] = sum of partials
-void channel_sum(const uint16_t* g, size_t voxels, int channels, float* partial, float* out, hipStream_t stream);
+// dw[co][tap][ci] = sum over voxels of gy[m][co] x[m + d(tap)][ci] for the
+// first cin input channels, db[co] = sum over voxels of gy[m][co] (fp32);
+// partial: wgrad_partial_floats(..., src.ca + src.cb, cout) floats of scratch
+size_t wgrad_partial_floats(int D, int H, int W, int cin, int cout);
+void conv3_weight_grad(const ConvSrc& src, int D, int H, int W, const uint16_t* gy, int cin, int cout, float* partial,
+                       float* dw, float* db, hipStream_t stream);
 
 // packing of fp32 master weights [cout][27][cin] into the forward layout
 // (wt[co][tap * cin_pad + ci], zero for ci >= cin) and the flipped, transposed

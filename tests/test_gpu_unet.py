@@ -85,6 +85,13 @@ def test_scale_only_rescales():
     assert err < 3e-2, err
 
 
+# (the brick kernels' edges: rows of 68 voxels are two bricks and a remainder of
+# 4 at full resolution, 34 and 17 at the lower ones, 12 slices one and a half
+# weight-gradient bricks at half resolution; the same bounds)
+def test_gradient_matches_oracle_at_brick_edges():
+    test_gradient_matches_oracle((12, 8, 68))
+
+
 @pytest.mark.parametrize("shape", [(16, 16, 16), (8, 12, 20)])
 def test_gradient_matches_oracle(shape):
     params, x, d, target = setup_case(shape, 13)
