@@ -20,6 +20,8 @@ constexpr LayerSpec kLayers[] = {
 constexpr int kLayerCount = 10;
 constexpr int kHead = 16;
 constexpr int kInputChannels = 8;   // (x, d) padded to one 16-byte channel group
+// upsampled input channels of a layer (they come first)
+constexpr int upsampled(int i) { return i == 6 ? 64 : i == 8 ? 32 : 0; }
 
 }  // namespace
 
@@ -50,14 +52,13 @@ UNet3D::UNet3D(int nx, int ny, int nz, hipStream_t stream) : stream_(stream)
     params_.allocate(sizeof(float) * P);
     ETN_HIP(hipMemsetAsync(params_.get(), 0, sizeof(float) * P, stream_));
     for (const Layer& L : layers_) {
-        wt_.emplace_back(sizeof(uint16_t) * L.cout * nn::kpad_for(std::max(L.cin, kInputChannels)));
-        wb_.emplace_back(L.cin >= 8 ? sizeof(uint16_t) * L.cin * nn::kpad_for(L.cout) : 0);
+        // the first layer reads the fp32 volumes and has no input gradient
+        wt_.emplace_back(sizeof(uint16_t) * (L.cin < 16 ? (size_t)nn::kFirstWeights : nn::conv_weight_count(L.cin, L.cout)));
+        wb_.emplace_back(L.cin < 16 ? 0 : sizeof(uint16_t) * nn::conv_weight_count(L.cout, L.cin));
         act_.emplace_back(sizeof(uint16_t) * voxels(L.level) * L.cout);
     }
-    xin_.allocate(sizeof(uint16_t) * voxels(0) * kInputChannels);
     pool1_.allocate(sizeof(uint16_t) * voxels(1) * 16);
     pool2_.allocate(sizeof(uint16_t) * voxels(2) * 32);
-    pred_.allocate(sizeof(float) * voxels(0));
     packAll();
 }
 
@@ -85,8 +86,17 @@ void UNet3D::packAll()
 {
     for (int i = 0; i < kLayerCount; ++i) {
         const Layer& L = layers_[i];
-        nn::pack_weights(params_.as<float>() + L.w, L.cout, L.cin, std::max(L.cin, kInputChannels),
-                         wt_[i].as<uint16_t>(), L.cin >= 8 ? wb_[i].as<uint16_t>() : nullptr, stream_);
+        const float* w = params_.as<float>() + L.w;
+        if (L.cin < 16) {
+            nn::pack_first_weights(w, wt_[i].as<uint16_t>(), stream_);
+            continue;
+        }
+        nn::pack_weights(w, L.cin, L.cin, L.cout, false, wt_[i].as<uint16_t>(), stream_);
+        // the decoder's first layers: the upsampled channels' part, then the skip's
+        const int up = upsampled(i);
+        if (up) nn::pack_weights(w, L.cin, L.cout, up, true, wb_[i].as<uint16_t>(), stream_);
+        nn::pack_weights(w + up, L.cin, L.cout, L.cin - up, true,
+                         wb_[i].as<uint16_t>() + nn::conv_weight_count(L.cout, up), stream_);
     }
 }
 
@@ -110,35 +120,44 @@ nn::ConvSrc UNet3D::layerInput(int i) const
     return s;
 }
 
-void UNet3D::forward(const float* x, const float* d, float scale, float dscale)
+void UNet3D::forward(const float* x, const float* d, float scale, float dscale, float* pred, bool predict)
 {
-    nn::pack_input(x, scale, d, dscale, voxels(0), xin_.as<uint16_t>(), stream_);
+    const float* p = params_.as<float>();
     for (int i = 0; i < kLayerCount; ++i) {
         const Layer& L = layers_[i];
-        if (i == 2) nn::pool2(layerOutput(1), D_[0], H_[0], W_[0], 16, pool1_.as<uint16_t>(), stream_);
-        if (i == 4) nn::pool2(layerOutput(3), D_[1], H_[1], W_[1], 32, pool2_.as<uint16_t>(), stream_);
+        if (i == 0) {
+            nn::conv3_first(x, scale, d, dscale, D_[0], H_[0], W_[0], wt_[0].as<uint16_t>(), p + L.b,
+                            act_[0].as<uint16_t>(), stream_);
+            continue;
+        }
         nn::ConvArgs a;
         a.src = layerInput(i);
         a.D = D_[L.level];
         a.H = H_[L.level];
         a.W = W_[L.level];
         a.wt = wt_[i].as<uint16_t>();
-        a.kpad = nn::kpad_for(std::max(L.cin, kInputChannels));
-        a.bias = params_.as<float>() + L.b;
+        a.bias = p + L.b;
         a.cout = L.cout;
         a.relu = 1;
         a.out = act_[i].as<uint16_t>();
+        if (i == 1) a.pool = pool1_.as<uint16_t>();
+        if (i == 3) a.pool = pool2_.as<uint16_t>();
+        if (i == kLayerCount - 1) {
+            if (predict) a.out = nullptr;   // only the backward pass reads it
+            a.head = p + head_;
+            a.x = x;
+            a.scale = scale;
+            a.pred = pred;
+            a.unscale = predict;
+        }
         nn::conv3_forward(a, stream_);
     }
-    const float* p = params_.as<float>();
-    nn::head_forward(layerOutput(9), x, scale, p + head_, p + head_ + kHead, voxels(0), pred_.as<float>(), stream_);
 }
 
 void UNet3D::predict(const float* x, const float* d, float scale, float dscale, float* out)
 {
     if (!(scale > 0.0f) || !std::isfinite(scale) || !std::isfinite(dscale)) fail("scales must be finite, scale > 0");
-    forward(x, d, scale, dscale);
-    nn::unscale_prediction(pred_.as<float>(), x, scale, voxels(0), out, stream_);
+    forward(x, d, scale, dscale, out, true);
 }
 
 void UNet3D::ensureTraining()
@@ -152,10 +171,11 @@ void UNet3D::ensureTraining()
     ETN_HIP(hipMemsetAsync(adam_v_.get(), 0, adam_v_.bytes(), stream_));
     const size_t m0 = voxels(0), m1 = voxels(1), m2 = voxels(2);
     const size_t h = sizeof(uint16_t);
+    xin_.allocate(h * m0 * kInputChannels);
+    pred_.allocate(sizeof(float) * m0);
     gpred_.allocate(sizeof(float) * m0);
     gd1_.allocate(h * m0 * 16);
     gtmp_.allocate(h * std::max({m0 * 16, m1 * 32, m2 * 64}));
-    gcat_.allocate(h * std::max(m0 * 48, m1 * 96));
     ge1_.allocate(h * m0 * 16);
     ge2_.allocate(h * m1 * 32);
     ge3_.allocate(h * m2 * 64);
@@ -175,60 +195,73 @@ void UNet3D::ensureTraining()
 void UNet3D::backward()
 {
     float* g = grads_.as<float>();
-    auto layer_back = [&](int i, uint16_t* gy, uint16_t* gx) {
+    // layer i from its output's gradient gy (already zero where the ReLU is):
+    // the parameters' gradients, and the input's in gx, zero where gate's ReLU
+    // is; of a layer on upsampled channels, gx takes the skip's and gx_up the
+    // upsampled volume's at its own resolution
+    auto layer_back = [&](int i, const uint16_t* gy, uint16_t* gx, const uint16_t* gate, uint16_t* gx_up = nullptr,
+                          const uint16_t* gate_up = nullptr) {
         const Layer& L = layers_[i];
         const int D = D_[L.level], H = H_[L.level], W = W_[L.level];
-        const size_t M = voxels(L.level);
-        nn::relu_backward(gy, layerOutput(i), M * L.cout, stream_);
         nn::conv3_weight_grad(layerInput(i), D, H, W, gy, L.cin, L.cout, wpart_.as<float>(), g + L.w, g + L.b, stream_);
-        if (gx) {
-            nn::ConvArgs a;
-            a.src.a = gy;
-            a.src.ca = L.cout;
-            a.D = D;
-            a.H = H;
-            a.W = W;
-            a.wt = wb_[i].as<uint16_t>();
-            a.kpad = nn::kpad_for(L.cout);
-            a.cout = L.cin;
-            a.out = gx;
+        if (!gx) return;
+        nn::ConvArgs a;
+        a.src.a = gy;
+        a.src.ca = L.cout;
+        a.D = D;
+        a.H = H;
+        a.W = W;
+        a.wt = wb_[i].as<uint16_t>();
+        const int up = upsampled(i);
+        if (up) {
+            a.cout = up;
+            a.out = gx_up;
+            a.gate = gate_up;
+            a.children = 1;
             nn::conv3_forward(a, stream_);
+            a.children = 0;
+            a.wt += nn::conv_weight_count(L.cout, up);
         }
+        a.cout = L.cin - up;
+        a.out = gx;
+        a.gate = gate;
+        nn::conv3_forward(a, stream_);
     };
     uint16_t* gtmp = gtmp_.as<uint16_t>();
-    uint16_t* gcat = gcat_.as<uint16_t>();
     uint16_t* gp = gp_.as<uint16_t>();
+    uint16_t* gd1 = gd1_.as<uint16_t>();
+    uint16_t* gd2 = gd2_.as<uint16_t>();
+    uint16_t* ge1 = ge1_.as<uint16_t>();
+    uint16_t* ge2 = ge2_.as<uint16_t>();
+    uint16_t* ge3 = ge3_.as<uint16_t>();
     const float* p = params_.as<float>();
-    nn::head_backward(layerOutput(9), gpred_.as<float>(), p + head_, voxels(0), gd1_.as<uint16_t>(), hpart_.as<float>(),
-                      g + head_, stream_);
-    // decoder, full resolution
-    layer_back(9, gd1_.as<uint16_t>(), gtmp);
-    layer_back(8, gtmp, gcat);
-    nn::up2_backward(gcat, 48, 0, D_[0], H_[0], W_[0], 32, gd2_.as<uint16_t>(), stream_);
-    nn::take_channels(gcat, 48, 32, voxels(0), 16, ge1_.as<uint16_t>(), 0, stream_);
-    // decoder, half resolution
-    layer_back(7, gd2_.as<uint16_t>(), gtmp);
-    layer_back(6, gtmp, gcat);
-    nn::up2_backward(gcat, 96, 0, D_[1], H_[1], W_[1], 64, ge3_.as<uint16_t>(), stream_);
-    nn::take_channels(gcat, 96, 64, voxels(1), 32, ge2_.as<uint16_t>(), 0, stream_);
+    nn::head_backward(layerOutput(9), gpred_.as<float>(), p + head_, voxels(0), gd1, hpart_.as<float>(), g + head_,
+                      stream_);
+    // decoder, full and half resolution (the skips' gradients stay without
+    // their ReLU until the encoder's own arrive)
+    layer_back(9, gd1, gtmp, layerOutput(8));
+    layer_back(8, gtmp, ge1, nullptr, gd2, layerOutput(7));
+    layer_back(7, gd2, gtmp, layerOutput(6));
+    layer_back(6, gtmp, ge2, nullptr, ge3, layerOutput(5));
     // bottleneck
-    layer_back(5, ge3_.as<uint16_t>(), gtmp);
-    layer_back(4, gtmp, gp);
-    nn::pool2_backward(gp, D_[1], H_[1], W_[1], 32, ge2_.as<uint16_t>(), 1, stream_);
-    // encoder, half resolution
-    layer_back(3, ge2_.as<uint16_t>(), gtmp);
-    layer_back(2, gtmp, gp);
-    nn::pool2_backward(gp, D_[0], H_[0], W_[0], 16, ge1_.as<uint16_t>(), 1, stream_);
-    // encoder, full resolution
-    layer_back(1, ge1_.as<uint16_t>(), gtmp);
-    layer_back(0, gtmp, nullptr);
+    layer_back(5, ge3, gtmp, layerOutput(4));
+    layer_back(4, gtmp, gp, nullptr);
+    nn::join_gradients(gp, D_[1], H_[1], W_[1], 32, layerOutput(3), ge2, stream_);
+    // encoder, half and full resolution
+    layer_back(3, ge2, gtmp, layerOutput(2));
+    layer_back(2, gtmp, gp, nullptr);
+    nn::join_gradients(gp, D_[0], H_[0], W_[0], 16, layerOutput(1), ge1, stream_);
+    layer_back(1, ge1, gtmp, layerOutput(0));
+    layer_back(0, gtmp, nullptr, nullptr);
 }
 
 double UNet3D::gradient(const float* x, const float* d, const float* target, float scale, float dscale)
 {
     if (!(scale > 0.0f) || !std::isfinite(scale) || !std::isfinite(dscale)) fail("scales must be finite, scale > 0");
     ensureTraining();
-    forward(x, d, scale, dscale);
+    // the first layer's weight gradient reads its input as channels
+    nn::pack_input(x, scale, d, dscale, voxels(0), xin_.as<uint16_t>(), stream_);
+    forward(x, d, scale, dscale, pred_.as<float>(), false);
     nn::mse_loss(pred_.as<float>(), target, scale, voxels(0), gpred_.as<float>(), lpart_.as<double>(),
                  loss_.as<double>(), stream_);
     backward();
@@ -264,11 +297,12 @@ double UNet3D::timeForward(const float* x, float scale, double* flops)
     for (const Layer& L : layers_) f += 2.0 * 27.0 * L.cin * L.cout * (double)voxels(L.level);
     f += 2.0 * kHead * (double)voxels(0);
     if (flops) *flops = f;
+    if (!pred_.get()) pred_.allocate(sizeof(float) * voxels(0));
     hipEvent_t a, b;
     ETN_HIP(hipEventCreate(&a));
     ETN_HIP(hipEventCreate(&b));
     ETN_HIP(hipEventRecord(a, stream_));
-    forward(x, nullptr, scale, 0.0f);
+    forward(x, nullptr, scale, 0.0f, pred_.as<float>(), true);
     ETN_HIP(hipEventRecord(b, stream_));
     ETN_HIP(hipEventSynchronize(b));
     float ms = 0.0f;

@@ -44,7 +44,8 @@ public:
     double timeForward(const float* x, float scale, double* flops);
 
 private:
-    void forward(const float* x, const float* d, float scale, float dscale);
+    // pred = x scale + delta, or (predict) x + delta / scale without the last activation kept
+    void forward(const float* x, const float* d, float scale, float dscale, float* pred, bool predict);
     void backward();
     void packAll();
     void ensureTraining();
@@ -58,11 +59,11 @@ private:
     size_t head_;                                   // offset of the head weights
     DeviceBuffer params_, grads_, adam_m_, adam_v_;
     std::vector<DeviceBuffer> wt_, wb_;             // packed bf16 weights per layer
-    DeviceBuffer xin_, pool1_, pool2_, pred_;
+    DeviceBuffer pool1_, pool2_;
     std::vector<DeviceBuffer> act_;                 // output of each layer (bf16)
     // training buffers
     bool training_ = false;
-    DeviceBuffer gpred_, gd1_, gtmp_, gcat_, ge1_, ge2_, ge3_, gd2_, gp_, wpart_, hpart_, loss_, lpart_;
+    DeviceBuffer xin_, pred_, gpred_, gd1_, gtmp_, ge1_, ge2_, ge3_, gd2_, gp_, wpart_, hpart_, loss_, lpart_;
     int adam_t_ = 0;
 };
 

@@ -1,12 +1,8 @@
 // Learned correction network kernels (see unet_kernels.hpp).
 //
-// The 3x3x3 convolution is an implicit GEMM on the matrix cores: output
-// voxels are the GEMM rows, output channels the columns, and the reduction
-// runs over k = tap * cin + ci.  Each wave owns MT tiles of 16 voxels and all
-// cout channels (NT tiles of 16); per 32-wide k step a lane loads its 8
-// channels of one tap for each voxel tile (one 16-byte load from the
-// channels-last activation, or zeros outside the volume) and 8 weights per
-// channel tile, then issues MT x NT v_mfma_f32_16x16x32_bf16.  Lane layouts
+// The 3x3x3 convolutions are implicit GEMMs on the matrix cores
+// (v_mfma_f32_16x16x32_bf16, FP32 accumulation): output channels are the rows,
+// voxels the columns, taps x input channels the reduction.  Lane layouts
 // (checked on the device): A[i][k] in lane i + 16 (k / 8), element k % 8;
 // B[k][j] in lane j + 16 (k / 8); D[i][j] in lane j + 16 (i / 4), element i % 4.
 //
@@ -29,7 +25,6 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ uint16_t f2bf(float f) { return dev::BF16::pack(f); }
 
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
@@ -38,238 +33,335 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast
 constexpr int kConvWaves = 4;
 constexpr int kThreads = 256;
 
-// ---- 3x3x3 convolution, implicit GEMM ---------------------------------------
-template <int NT, int MT>
-__global__ void __launch_bounds__(kThreads) conv3_fwd_kernel(ConvArgs a)
+// 1 where a stored activation is positive: the derivative of the ReLU behind it
+__device__ __forceinline__ bool positive(uint16_t h) { return !(h & 0x8000u) && (h & 0x7fffu) != 0; }
+// a pair of bf16 values with the ones whose activation is not positive set to zero
+__device__ __forceinline__ uint32_t gated(uint32_t pair, uint32_t act)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = lane & 15, kg = lane >> 4;
-    const size_t M = (size_t)a.D * a.H * a.W;
-    const size_t m0 = ((size_t)blockIdx.x * kConvWaves + wave) * (MT * 16);
-    if (m0 >= M) return;   // the whole wave is past the volume (no barriers below)
-    const int HW = a.H * a.W;
-    int vz[MT], vy[MT], vx[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const size_t m = m0 + mt * 16 + row;
-        if (m < M) {
-            vz[mt] = (int)(m / HW);
-            const int r = (int)(m - (size_t)vz[mt] * HW);
-            vy[mt] = r / a.W;
-            vx[mt] = r - vy[mt] * a.W;
-        } else {
-            vz[mt] = -4;   // every tap falls outside
-            vy[mt] = 0;
-            vx[mt] = 0;
-        }
-    }
-    floatx4 acc[MT][NT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    const int ca = a.src.ca, cin = a.src.ca + a.src.cb;
-    const int Hh = a.H >> 1, Wh = a.W >> 1;
-    const bf16x8 zero = as_bf16x8(u32x4{0u, 0u, 0u, 0u});
-    for (int k0 = kg * 8; k0 < a.kpad; k0 += 32) {
-        bf16x8 B[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) B[nt] = as_bf16x8(load16(a.wt + (size_t)(nt * 16 + row) * a.kpad + k0));
-        bf16x8 A[MT];
-        {
-            const int t = k0 / cin, ci = k0 - t * cin;
-            const int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const int zz = vz[mt] + dz, yy = vy[mt] + dy, xx = vx[mt] + dx;
-                A[mt] = zero;
-                if (t < 27 && (unsigned)zz < (unsigned)a.D && (unsigned)yy < (unsigned)a.H &&
-                    (unsigned)xx < (unsigned)a.W) {
-                    const uint16_t* p;
-                    if (ci < ca) {
-                        const size_t v = a.src.a_half ? ((size_t)(zz >> 1) * Hh + (yy >> 1)) * Wh + (xx >> 1)
-                                                      : ((size_t)zz * a.H + yy) * a.W + xx;
-                        p = a.src.a + v * ca + ci;
-                    } else {
-                        p = a.src.b + (((size_t)zz * a.H + yy) * a.W + xx) * a.src.cb + (ci - ca);
-                    }
-                    A[mt] = as_bf16x8(load16(p));
-                }
-            }
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt], B[nt], acc[mt][nt], 0, 0, 0);
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int co = nt * 16 + row;
-            const float b = a.bias ? a.bias[co] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const size_t m = m0 + mt * 16 + kg * 4 + r;
-                if (m < M) {
-                    float v = acc[mt][nt][r] + b;
-                    if (a.relu) v = fmaxf(v, 0.0f);
-                    a.out[m * a.cout + co] = f2bf(v);
-                }
-            }
-        }
+    return (positive((uint16_t)(act & 0xffffu)) ? pair & 0xffffu : 0u) |
+           (positive((uint16_t)(act >> 16)) ? pair & 0xffff0000u : 0u);
 }
 
-// ---- 3x3x3 convolution to 16 or 32 channels, LDS-staged bricks ----------
-// A workgroup computes a kBZ x kBY x kBX brick of output voxels, all
-// NT x 16 output channels.  Its input halo (kBZ + 2) x (kBY + 2) x (kBX + 2)
-// is staged in LDS eight input channels at a time (one 16-byte cell per halo
-// voxel), so that the 27 taps read each staged voxel from LDS instead of from
-// memory.  An MFMA k step takes four taps of the chunk: lane group kg's A
-// operand is its voxel's 8 channels at tap 4 s + kg, and its B operand the 8
-// weights wt[co][tap * cin + ci ..] of the same tap, contiguous in the forward
-// weight layout (the k order inside a step only has to agree between A and
-// B).  The next chunk's weights and halo are loaded into registers while the
-// current chunk's MFMAs run.  Wave w owns the brick's output rows
-// (z = w, y = 0..7), two 16-voxel tiles each: the LDS reads of a step share one
-// base address and differ by constant offsets.  The result goes through LDS
-// (one 16-channel slice at a time) so that each voxel's channels leave in
-// 16-byte stores.
-constexpr int kBZ = kConvWaves, kBY = 8, kBX = 32;
+// ---- 3x3x3 convolution on LDS-staged bricks -------------------------------
+// A workgroup computes a kBZ x kBY x kBX brick of output voxels and NC x 16
+// output channels (blockIdx.y: which); each of its 8 NC waves owns 4 z x 2 y
+// rows of 16 voxels and 16 channels, whose sums stay in registers.  The input
+// brick with its halo is staged in LDS 16 channels at a time as two arrays of
+// 16-byte cells (channels 0-7 and 8-15), with the chunk's weights behind it.
+// The weights are the GEMM's rows and the voxels its columns, so that a lane
+// ends with 4 consecutive channels of one voxel and stores 8 bytes without a
+// pass through LDS.
+// A 32-wide k step holds two taps of 16 channels (lane group kg: tap kg / 2,
+// channels 8 (kg % 2) ..), chosen so that a voxel operand depends only on the
+// input row it starts at and serves every output row whose taps it holds:
+//   F1(r): taps dx = 0 and 1 of input row r,     used with dy = 0, 1, 2;
+//   F2(r): tap dx = 2 of input rows r and r + 1, used with dy = 0 and 1 (P)
+//          and, its first row weighted 0, with dy = 2 (Q).
+// That is 5 steps per dz and output row (15 for the 27 taps, 0.9 of the
+// products wanted) and 7 LDS reads for 10 MFMAs; a step of four arbitrary taps
+// of 8 channels took one read per MFMA.  What bounds it besides the MFMAs is
+// everything around them: a wave has 120 MFMAs a chunk (1920 cycles), so the
+// halo's addresses are scalars (a wave stages whole rows; per-cell indices cost
+// more VALU time than the MFMAs take), and 128 VGPRs keep four waves a SIMD,
+// two workgroups a CU, for one to load while the other computes.  Measured at
+// 256^3 (prediction 4.08 -> 2.27 ms): 48 to 16 channels 1.13 -> 0.80 ms (875
+// TFLOP/s of its 27 taps), 16 to 16 with the pooling in the epilogue 0.35 ms
+// (1.2 GB, 3.4 TB/s).
+constexpr int kBZ = 4, kBY = 8, kBX = 32;
 constexpr int kHZ = kBZ + 2, kHY = kBY + 2, kHX = kBX + 2;
-constexpr int kHaloCells = kHZ * kHY * kHX;                    // 2040
-constexpr int kBrickVoxels = kBZ * kBY * kBX;                  // 1024
-constexpr int kBrickTiles = kBrickVoxels / 16 / kConvWaves;    // 16 tiles of 16 voxels per wave
-constexpr int kStage = (kHaloCells + kThreads - 1) / kThreads; // halo cells per thread
-constexpr int kChunkSteps = (27 + 3) / 4;                      // k steps per 8-channel chunk
-constexpr int kBrickLds = 2 * kBrickVoxels;                    // cells: >= the halo, = one output slice
+constexpr int kHaloRows = kHZ * kHY;          // 60
+constexpr int kHaloCells = kHaloRows * kHX;   // 2040
+// Cells between the two channel halves.  A multiple of 16: lane groups 0 and 1
+// (2 and 3) of a read are served together, and with the same position modulo
+// the 256 bytes of the banks they do not collide (4.1 cycles a read of the
+// wave, 8.0 with any other distance, 2040 among them).
+constexpr int kPlane = (kHaloCells + 15) / 16 * 16;
+constexpr int kConvThreads = 512;
+constexpr int kXcds = 8;
 
-template <int NT>
-__global__ void __launch_bounds__(kThreads) conv3_brick_kernel(ConvArgs a, int nbx, int nby)
+// What a convolution does with its sums (besides bias and activation).
+enum Epilogue {
+    kStore,      // out, optionally gated
+    kPool,       // out, and its 2 x 2 x 2 averages
+    kChildren,   // the sums over 2 x 2 x 2 voxels, gated, instead of out
+    kHead        // the 1 x 1 x 1 head's prediction; out only where it is wanted
+};
+
+// Brick of workgroup b of `groups` (a multiple of kXcds): the bricks of an XCD
+// are consecutive (workgroup b runs on XCD b mod 8), so that neighbours read
+// their shared halo from one L2.
+__device__ __forceinline__ int brick_of(int b, int groups) { return b % kXcds * (groups / kXcds) + b / kXcds; }
+
+template <int NC, Epilogue kEpi>
+__global__ void __launch_bounds__(kConvThreads * NC, 4) conv3_brick_kernel(ConvArgs a, int nbx, int nby, int bricks)
 {
-    static_assert(kBrickLds >= kHaloCells, "the output slice reuses the halo's LDS");
-    __shared__ u32x4 lds[kBrickLds];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row = lane & 15, kg = lane >> 4;
-    const int bxi = blockIdx.x % nbx, rest = blockIdx.x / nbx;
-    const int byi = rest % nby, bzi = rest / nby;
+    constexpr int kT = kConvThreads * NC, kWaves = kT / 64;
+    __shared__ u32x4 lds[2 * kPlane];
+    __shared__ u32x4 wlds[NC * kConvFrags * 64];   // the chunk's weights
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, kg = lane >> 4;
+    const int brick = brick_of(blockIdx.x, gridDim.x);
+    if (brick >= bricks) return;
+    const int bxi = brick % nbx, rest = brick / nbx, byi = rest % nby, bzi = rest / nby;
     const int x0 = bxi * kBX, y0 = byi * kBY, z0 = bzi * kBZ;
+    const int wx = (wave & 1) * 16, wy = (wave >> 1 & 3) * 2;   // the wave's voxels and rows in the brick
     const int ca = a.src.ca, cin = a.src.ca + a.src.cb;
     const int Hh = a.H >> 1, Wh = a.W >> 1;
     const u32x4 zero4 = u32x4{0u, 0u, 0u, 0u};
+    const int tiles = a.cout / 16, tile = blockIdx.y * NC + (wave >> 3);
 
-    floatx4 acc[kBrickTiles][NT];
+    // the lane's first channel and its bias (the sums start there)
+    const int c = tile * 16 + kg * 4;
+    floatx4 acc[kBZ][2];
+    {
+        floatx4 bias = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (a.bias) {
 #pragma unroll
-    for (int t = 0; t < kBrickTiles; ++t)
+            for (int r = 0; r < 4; ++r) bias[r] = a.bias[c + r];
+        }
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[t][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int z = 0; z < kBZ; ++z) acc[z][0] = acc[z][1] = bias;
+    }
 
-    // one chunk's weights (step st, tap 4 st + kg, output channel nt * 16 + row)
-    // and halo cells, loaded into registers; the next chunk's loads are in
-    // flight while the current chunk's MFMAs run
-    u32x4 B[kChunkSteps][NT], cell[kStage];
+    // A wave stages halo rows wave, wave + kWaves, ...: lanes take the cells of
+    // voxels 0 .. 31 (voxel lane / 2, channel half lane % 2), whose addresses are
+    // the row's scalar one and the lane's offset; threads 0 .. 239 take voxels
+    // 32 and 33 of the 60 rows.  Cells outside the volume read a valid address
+    // and are zeroed on their way to LDS: a branch or a select at the load would
+    // wait for it on the spot.
+    constexpr int kRows = (kHaloRows + kWaves - 1) / kWaves;
+    constexpr int kWStage = (NC * kConvFrags * 64 + kT - 1) / kT;
+    u32x4 cell[kRows], edge, wcell[kWStage];
+    const int hx = x0 - 1 + (lane >> 1), erow = tid >> 2, ehx = x0 + 31 + (tid >> 1 & 1);
+    const int ehy = y0 - 1 + erow % kHY, ehz = z0 - 1 + erow / kHY;
+    const bool hx_in = (unsigned)hx < (unsigned)a.W;
+    const bool edge_in = erow < kHaloRows && ehx < a.W && (unsigned)ehy < (unsigned)a.H && (unsigned)ehz < (unsigned)a.D;
+    auto row_y = [&](int k) { return y0 - 1 + (wave + k * kWaves) % kHY; };
+    auto row_z = [&](int k) { return z0 - 1 + (wave + k * kWaves) / kHY; };
     auto load_chunk = [&](int c0) {
+        const bool from_a = c0 < ca;
+        const int cs = (from_a ? ca : a.src.cb) / 8;   // cells per voxel
+        const u32x4* src = reinterpret_cast<const u32x4*>(from_a ? a.src.a + c0 : a.src.b + (c0 - ca));
+        const int shift = from_a && a.src.a_half ? 1 : 0;
+        const int Hs = shift ? Hh : a.H, Ws = shift ? Wh : a.W;
+        const uint32_t at = (uint32_t)((hx_in ? hx >> shift : 0) * cs + (lane & 1));
 #pragma unroll
-        for (int st = 0; st < kChunkSteps; ++st) {
-            const int tap = 4 * st + kg;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                B[st][nt] = tap < 27 ? load16(a.wt + (size_t)(nt * 16 + row) * a.kpad + tap * cin + c0) : zero4;
+        for (int k = 0; k < kRows; ++k) {
+            const int y = min(max(row_y(k), 0), a.H - 1) >> shift, z = min(max(row_z(k), 0), a.D - 1) >> shift;
+            cell[k] = (src + ((size_t)z * Hs + y) * Ws * cs)[at];
         }
+        const size_t ev = edge_in ? ((size_t)(ehz >> shift) * Hs + (ehy >> shift)) * Ws + (ehx >> shift) : 0;
+        edge = src[ev * cs + (tid & 1)];
+        const u32x4* w = reinterpret_cast<const u32x4*>(a.wt) +
+                         ((size_t)(c0 / 16) * tiles + blockIdx.y * NC) * (kConvFrags * 64);
 #pragma unroll
-        for (int k = 0; k < kStage; ++k) {
-            const int e = k * kThreads + tid;
-            cell[k] = zero4;
-            if (e < kHaloCells) {
-                const int hz = e / (kHY * kHX), r2 = e - hz * (kHY * kHX), hy = r2 / kHX, hx = r2 - hy * kHX;
-                const int zz = z0 - 1 + hz, yy = y0 - 1 + hy, xx = x0 - 1 + hx;
-                if ((unsigned)zz < (unsigned)a.D && (unsigned)yy < (unsigned)a.H && (unsigned)xx < (unsigned)a.W) {
-                    const uint16_t* p;
-                    if (c0 < ca) {
-                        const size_t vi = a.src.a_half ? ((size_t)(zz >> 1) * Hh + (yy >> 1)) * Wh + (xx >> 1)
-                                                       : ((size_t)zz * a.H + yy) * a.W + xx;
-                        p = a.src.a + vi * ca + c0;
-                    } else {
-                        p = a.src.b + (((size_t)zz * a.H + yy) * a.W + xx) * a.src.cb + (c0 - ca);
-                    }
-                    cell[k] = load16(p);
-                }
-            }
-        }
+        for (int k = 0; k < kWStage; ++k) wcell[k] = w[min(k * kT + tid, NC * kConvFrags * 64 - 1)];
     };
     load_chunk(0);
-    for (int c0 = 0; c0 < cin; c0 += 8) {
-        __syncthreads();   // the previous chunk's reads of lds are done
+    // the lane's cell of F1(row 0) and F2(row 0) in halo slice 0, its weights
+    const u32x4* half = lds + (kg & 1) * kPlane + wy * kHX + wx + col;
+    const u32x4* f1 = half + (kg >> 1);
+    const u32x4* f2 = half + (kg >> 1) * kHX + 2;
+    const u32x4* wf = wlds + (wave >> 3) * (kConvFrags * 64) + lane;
+    for (int c0 = 0; c0 < cin; c0 += 16) {
+        __syncthreads();   // the previous chunk's reads are done
+        u32x4* to = lds + (lane & 1) * kPlane + (lane >> 1) + wave * kHX;
 #pragma unroll
-        for (int k = 0; k < kStage; ++k) {
-            const int e = k * kThreads + tid;
-            if (e < kHaloCells) lds[e] = cell[k];
+        for (int k = 0; k < kRows; ++k) {
+            const bool in = (unsigned)row_y(k) < (unsigned)a.H && (unsigned)row_z(k) < (unsigned)a.D && hx_in;
+            if (wave + k * kWaves < kHaloRows) to[k * kWaves * kHX] = in ? cell[k] : zero4;
         }
-        u32x4 Bc[kChunkSteps][NT];
+        if (erow < kHaloRows) lds[(tid & 1) * kPlane + erow * kHX + 32 + (tid >> 1 & 1)] = edge_in ? edge : zero4;
 #pragma unroll
-        for (int st = 0; st < kChunkSteps; ++st)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) Bc[st][nt] = B[st][nt];
+        for (int k = 0; k < kWStage; ++k) {
+            const int e = k * kT + tid;
+            if (e < NC * kConvFrags * 64) wlds[e] = wcell[k];
+        }
         __syncthreads();
-        if (c0 + 8 < cin) load_chunk(c0 + 8);
+        if (c0 + 16 < cin) load_chunk(c0 + 16);
+#pragma unroll 1
+        for (int dz = 0; dz < 3; ++dz) {
+            bf16x8 w[kConvFrags / 3];
 #pragma unroll
-        for (int st = 0; st < kChunkSteps; ++st) {
-            const int tap = 4 * st + kg;
-            const bool live = tap < 27;
-            const int tc = live ? tap : 0;   // a valid address for the padding taps (B is zero there)
-            const int dz = tc / 9, dy = (tc / 3) % 3, dx = tc % 3;
-            const u32x4* base = lds + ((wave + dz) * kHY + dy) * kHX + dx + row;
+            for (int f = 0; f < kConvFrags / 3; ++f) w[f] = as_bf16x8(wf[(dz * (kConvFrags / 3) + f) * 64]);
 #pragma unroll
-            for (int t = 0; t < kBrickTiles; ++t) {
-                u32x4 av = base[(t >> 1) * kHX + (t & 1) * 16];
-                if (!live) av = zero4;
+            for (int z = 0; z < kBZ; ++z) {
+                const u32x4* r1 = f1 + (z + dz) * (kHY * kHX);
+                const u32x4* r2 = f2 + (z + dz) * (kHY * kHX);
+                bf16x8 F1[4], F2[3];
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                    acc[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(av), as_bf16x8(Bc[st][nt]),
-                                                                         acc[t][nt], 0, 0, 0);
+                for (int r = 0; r < 4; ++r) F1[r] = as_bf16x8(r1[r * kHX]);
+#pragma unroll
+                for (int r = 0; r < 3; ++r) F2[r] = as_bf16x8(r2[r * kHX]);
+#pragma unroll
+                for (int f = 0; f < kConvFrags / 3; ++f)
+#pragma unroll
+                    for (int y = 0; y < 2; ++y)
+                        acc[z][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[f], f < 3 ? F1[y + f] : F2[y + f - 3],
+                                                                            acc[z][y], 0, 0, 0);
             }
         }
     }
-    // epilogue, one 16-channel slice at a time: bias, activation, bf16 into
-    // LDS as [brick voxel][16 channels], then 16-byte stores of 8 channels
-    uint16_t* slice = reinterpret_cast<uint16_t*>(lds);
+
+    // rows are uniform in the wave: a row's address is a scalar plus the lane's
+    // offset
+    const int x = x0 + wx + col;
+    const bool xin = x < a.W;
+    const uint32_t at = (uint32_t)(x * a.cout + c), at_low = (uint32_t)((x >> 1) * a.cout + c);
+    auto row = [&](int z, int y) { return ((size_t)(z0 + z) * a.H + (y0 + wy + y)) * a.W; };
+    auto row_low = [&](int z) { return ((size_t)((z0 + z) >> 1) * Hh + ((y0 + wy) >> 1)) * Wh; };
+    auto row_in = [&](int z, int y) { return z0 + z < a.D && y0 + wy + y < a.H; };
+    // the gates of all the lane's voxels, in flight together
+    [[maybe_unused]] uint2 gate[kEpi == kStore ? kBZ * 2 : kEpi == kChildren ? kBZ / 2 : 1];
+    if constexpr (kEpi == kStore) {
+        if (a.gate && xin) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const int co = nt * 16 + row;
-        const float b = a.bias ? a.bias[co] : 0.0f;
-        __syncthreads();   // the last chunk's reads (or the previous slice's copy) are done
+            for (int i = 0; i < kBZ * 2; ++i)
+                if (row_in(i / 2, i % 2))
+                    gate[i] = *reinterpret_cast<const uint2*>(a.gate + row(i / 2, i % 2) * a.cout + at);
+        }
+    }
+    if constexpr (kEpi == kChildren) {
+        if (a.gate && xin) {
 #pragma unroll
-        for (int t = 0; t < kBrickTiles; ++t) {
-            const int v0 = (wave * kBY + (t >> 1)) * kBX + (t & 1) * 16 + kg * 4;
+            for (int i = 0; i < kBZ / 2; ++i)
+                if (row_in(2 * i, 0)) gate[i] = *reinterpret_cast<const uint2*>(a.gate + row_low(2 * i) * a.cout + at_low);
+        }
+    }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float v = acc[t][nt][e] + b;
-                if (a.relu) v = fmaxf(v, 0.0f);
-                slice[(v0 + e) * 16 + row] = f2bf(v);
+    for (int z = 0; z < kBZ; ++z)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+            floatx4& v = acc[z][y];
+            if (a.relu) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.0f);
+            }
+            if constexpr (kEpi == kChildren) continue;
+            uint2 p = make_uint2(dev::BF16::pack2(v[0], v[1]), dev::BF16::pack2(v[2], v[3]));
+            if constexpr (kEpi == kStore) {
+                if (a.gate) p = make_uint2(gated(p.x, gate[z * 2 + y].x), gated(p.y, gate[z * 2 + y].y));
+            }
+            if (row_in(z, y) && xin && (kEpi != kHead || a.out))
+                *reinterpret_cast<uint2*>(a.out + row(z, y) * a.cout + at) = p;
+            if constexpr (kEpi == kPool || kEpi == kHead) {
+                // what follows reads the stored (rounded) values
+                float t[4];
+                dev::BF16::unpack2(p.x, t[0], t[1]);
+                dev::BF16::unpack2(p.y, t[2], t[3]);
+                v = floatx4{t[0], t[1], t[2], t[3]};
             }
         }
-        __syncthreads();
+    if constexpr (kEpi == kHead) {
+        const bool mine = xin && kg == 0;
+        float xv[kBZ * 2];
 #pragma unroll
-        for (int k = 0; k < kBrickLds / kThreads; ++k) {
-            const int c = k * kThreads + tid;         // cell: voxel c / 2, channels 8 (c % 2) ..
-            const int bv = c >> 1, bz = bv / (kBY * kBX), by = (bv / kBX) % kBY, bx = bv % kBX;
-            const int z = z0 + bz, y = y0 + by, x = x0 + bx;
-            if (z < a.D && y < a.H && x < a.W)
-                *reinterpret_cast<u32x4*>(a.out + (((size_t)z * a.H + y) * a.W + x) * a.cout + nt * 16 + (c & 1) * 8) =
-                    lds[c];
+        for (int i = 0; i < kBZ * 2; ++i)
+            if (mine && row_in(i / 2, i % 2)) xv[i] = (a.x + row(i / 2, i % 2))[(uint32_t)x];
+#pragma unroll
+        for (int i = 0; i < kBZ * 2; ++i) {
+            const floatx4 v = acc[i / 2][i % 2];
+            float s = a.head[c] * v[0];
+#pragma unroll
+            for (int r = 1; r < 4; ++r) s = fmaf(a.head[c + r], v[r], s);
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            if (mine && row_in(i / 2, i % 2)) {
+                const float xs = xv[i] * a.scale;
+                const float pred = xs + (s + a.head[16]);
+                (a.pred + row(i / 2, i % 2))[(uint32_t)x] = a.unscale ? xv[i] + (pred - xs) / a.scale : pred;
+            }
+        }
+    }
+    if constexpr (kEpi == kPool || kEpi == kChildren) {
+        uint16_t* low = kEpi == kPool ? a.pool : a.out;
+#pragma unroll
+        for (int z = 0; z < kBZ; z += 2) {
+            floatx4 s = (acc[z][0] + acc[z][1]) + (acc[z + 1][0] + acc[z + 1][1]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] += __shfl_xor(s[r], 1);
+            if (kEpi == kPool) s *= 0.125f;
+            if (row_in(z, 0) && xin && (col & 1) == 0) {   // (z, y and the sizes are even)
+                uint2 p = make_uint2(dev::BF16::pack2(s[0], s[1]), dev::BF16::pack2(s[2], s[3]));
+                if constexpr (kEpi == kChildren) {
+                    if (a.gate) p = make_uint2(gated(p.x, gate[z / 2].x), gated(p.y, gate[z / 2].y));
+                }
+                *reinterpret_cast<uint2*>(low + row_low(z) * a.cout + at_low) = p;
+            }
         }
     }
 }
 
-template <int NT, int MT>
-void launch_conv(const ConvArgs& a, hipStream_t stream)
+// ---- first layer: (x, d) to 16 channels -----------------------------------
+// Reads the fp32 volumes themselves and keeps the halo in LDS as one 4-byte
+// bf16 pair per voxel.  A lane's 8 operands are 4 consecutive voxels of one
+// input row, the fourth and the rows past the ninth zero: 3 k steps for the 27
+// taps of 2 channels, where the two channels padded to 8 took 7 and a 16-byte
+// cell per voxel written and read back first (pack_input).  Bound by its
+// 32-byte output per voxel: 0.20 ms at 256^3, 3.4 TB/s.
+__global__ void __launch_bounds__(kThreads, 4) conv3_first_kernel(const float* __restrict__ xv, float scale,
+                                                                  const float* __restrict__ dv, float dscale, int D,
+                                                                  int H, int W, const uint16_t* __restrict__ wt,
+                                                                  const float* __restrict__ bias, uint16_t* out, int nbx,
+                                                                  int nby, int bricks)
 {
-    const size_t M = (size_t)a.D * a.H * a.W;
-    const size_t per_block = (size_t)kConvWaves * MT * 16;
-    const dim3 grid((unsigned)((M + per_block - 1) / per_block));
-    conv3_fwd_kernel<NT, MT><<<grid, kThreads, 0, stream>>>(a);
+    __shared__ uint32_t lds[kHaloCells];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int col = lane & 15, kg = lane >> 4;
+    const int brick = brick_of(blockIdx.x, gridDim.x);
+    if (brick >= bricks) return;
+    const int bxi = brick % nbx, rest = brick / nbx, byi = rest % nby, bzi = rest / nby;
+    const int x0 = bxi * kBX, y0 = byi * kBY, z0 = bzi * kBZ;
+    const int wy = (wave >> 1) * 4, wx = (wave & 1) * 16;
+#pragma unroll
+    for (int k = 0; k < (kHaloCells + kThreads - 1) / kThreads; ++k) {
+        const int v = k * kThreads + tid;
+        const int hz = v / (kHY * kHX), r2 = v - hz * (kHY * kHX), hy = r2 / kHX, hx = r2 - hy * kHX;
+        const int zz = z0 - 1 + hz, yy = y0 - 1 + hy, xx = x0 - 1 + hx;
+        uint32_t pair = 0u;
+        if ((unsigned)zz < (unsigned)D && (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W) {
+            const size_t m = ((size_t)zz * H + yy) * W + xx;
+            pair = dev::BF16::pack2(xv[m] * scale, dv ? dv[m] * dscale : 0.0f);
+        }
+        if (v < kHaloCells) lds[v] = pair;
+    }
+    bf16x8 w[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) w[s] = as_bf16x8(load16(wt + (s * 64 + lane) * 8));
+    float b[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) b[r] = bias[kg * 4 + r];
+    __syncthreads();
+    // step s, lane group kg: input row (dz, dy) = row 4 s + kg of the 3 x 3
+    int row_off[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+        const int g = min(4 * s + kg, 8);
+        row_off[s] = ((g / 3) * kHY + g % 3) * kHX;
+    }
+    const int x = x0 + wx + col;
+#pragma unroll
+    for (int z = 0; z < kBZ; ++z)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const uint32_t* at = lds + (z * kHY + wy + y) * kHX + wx + col;
+            floatx4 acc = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                const uint32_t* p = at + row_off[s];
+                u32x4 f = u32x4{p[0], p[1], p[2], 0u};
+                if (4 * s + kg > 8) f = u32x4{0u, 0u, 0u, 0u};
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s], as_bf16x8(f), acc, 0, 0, 0);
+            }
+            const int zz = z0 + z, yy = y0 + wy + y;
+            if (zz < D && yy < H && x < W) {
+                float v[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = fmaxf(acc[r] + b[r], 0.0f);
+                *reinterpret_cast<uint2*>(out + (((size_t)zz * H + yy) * W + x) * 16 + kg * 4) =
+                    make_uint2(dev::BF16::pack2(v[0], v[1]), dev::BF16::pack2(v[2], v[3]));
+            }
+        }
 }
 
 // ---- weight and bias gradient -------------------------------------------------
@@ -356,36 +448,57 @@ __global__ void __launch_bounds__(kThreads, NT == 4 ? 1 : 2) conv3_wgrad_kernel(
         tap_off[i] = (((t / 9) * kWHY + (t / 3) % 3) * kWHX + t % 3) * 32;
     }
 
-    for (int b = blockIdx.x; b < w.bricks; b += gridDim.x) {
+    // the thread's share of a brick, loaded into registers while the brick
+    // before it is worked on (cells outside the volume: a valid address, zeroed
+    // on their way to LDS)
+    const bool from_a = ci0 < ca;
+    const int cs = from_a ? ca : w.src.cb;
+    const uint16_t* src = from_a ? w.src.a + ci0 : w.src.b + (ci0 - ca);
+    const int shift = from_a && w.src.a_half ? 1 : 0;
+    const int Hs = shift ? Hh : w.H, Ws = shift ? Wh : w.W;
+    constexpr int kWStage = (kWHalo * 2 + kThreads - 1) / kThreads, kGStage = NT * kWVoxels * 2 / kThreads;
+    u32x4 xcell[kWStage], gcell[kGStage];
+    uint32_t xin = 0u, gin = 0u;   // bit k: cell k lies in the volume
+    auto load_brick = [&](int b) {
+        xin = gin = 0u;
         const int bxi = b % w.nbx, rest = b / w.nbx, byi = rest % w.nby, bzi = rest / w.nby;
         const int x0 = bxi * kWX, y0 = byi * kWY, z0 = bzi * kWZ;
-        __syncthreads();   // the previous brick's reads are done
-        for (int e = tid; e < kWHalo * 2; e += kThreads) {
-            const int v = e >> 1, c = ci0 + (e & 1) * 8;
+#pragma unroll
+        for (int k = 0; k < kWStage; ++k) {
+            const int e = k * kThreads + tid, v = e >> 1;
             const int hz = v / (kWHY * kWHX), r2 = v - hz * (kWHY * kWHX), hy = r2 / kWHX, hx = r2 - hy * kWHX;
             const int zz = z0 - 1 + hz, yy = y0 - 1 + hy, xx = x0 - 1 + hx;
-            u32x4 cell = zero4;
-            if (c < cin && (unsigned)zz < (unsigned)w.D && (unsigned)yy < (unsigned)w.H && (unsigned)xx < (unsigned)w.W) {
-                if (c < ca) {
-                    const size_t vi = w.src.a_half ? ((size_t)(zz >> 1) * Hh + (yy >> 1)) * Wh + (xx >> 1)
-                                                   : ((size_t)zz * w.H + yy) * w.W + xx;
-                    cell = load16(w.src.a + vi * ca + c);
-                } else {
-                    cell = load16(w.src.b + (((size_t)zz * w.H + yy) * w.W + xx) * w.src.cb + (c - ca));
-                }
-            }
-            xs[e] = cell;
+            const bool in = ci0 + (e & 1) * 8 < cin && (unsigned)zz < (unsigned)w.D && (unsigned)yy < (unsigned)w.H &&
+                            (unsigned)xx < (unsigned)w.W;
+            const size_t at = in ? (((size_t)(zz >> shift) * Hs + (yy >> shift)) * Ws + (xx >> shift)) * cs + (e & 1) * 8 : 0;
+            xcell[k] = load16(src + at);
+            xin |= in ? 1u << k : 0u;
         }
 #pragma unroll
-        for (int k = 0; k < NT * kWVoxels * 2 / kThreads; ++k) {
+        for (int k = 0; k < kGStage; ++k) {
             const int e = k * kThreads + tid;
             const int v = e / (2 * NT), c = e - v * (2 * NT);
             const int z = z0 + v / (kWY * kWX), y = y0 + (v / kWX) % kWY, x = x0 + v % kWX;
-            u32x4 cell = zero4;
-            if (z < w.D && y < w.H && x < w.W) cell = load16(w.gy + (((size_t)z * w.H + y) * w.W + x) * w.cout + c * 8);
-            gs[((c >> 1) * kWVoxels + v) * 2 + (c & 1)] = cell;
+            const bool in = z < w.D && y < w.H && x < w.W;
+            const size_t at = in ? (((size_t)z * w.H + y) * w.W + x) * w.cout + c * 8 : 0;
+            gcell[k] = load16(w.gy + at);
+            gin |= in ? 1u << k : 0u;
+        }
+    };
+    load_brick(blockIdx.x);   // the host launches at most one workgroup per brick
+    for (int b = blockIdx.x; b < w.bricks; b += gridDim.x) {
+        __syncthreads();   // the previous brick's reads are done
+#pragma unroll
+        for (int k = 0; k < kWStage; ++k)
+            if (k * kThreads + tid < kWHalo * 2) xs[k * kThreads + tid] = xin >> k & 1u ? xcell[k] : zero4;
+#pragma unroll
+        for (int k = 0; k < kGStage; ++k) {
+            const int e = k * kThreads + tid;
+            const int v = e / (2 * NT), c = e - v * (2 * NT);
+            gs[((c >> 1) * kWVoxels + v) * 2 + (c & 1)] = gin >> k & 1u ? gcell[k] : zero4;
         }
         __syncthreads();
+        if (b + (int)gridDim.x < w.bricks) load_brick(b + gridDim.x);
 #pragma unroll 2
         for (int row = 0; row < kWZ * kWY; ++row) {
             bf16x8 A[NT];
@@ -462,84 +575,57 @@ __global__ void __launch_bounds__(kThreads) sum_partials_kernel(const float* par
     sum_rows(partial, chunks, (size_t)C, C, [&](int i, float v) { out[i] = v; });
 }
 
-__global__ void pack_weights_kernel(const float* w, int cout, int cin, int cin_pad, uint16_t* wt, int kpad,
-                                    uint16_t* wb, int kpad_b)
+// Weights in the order conv3_brick_kernel's lanes read them: per 16 input
+// channels, 16 output channels and step (dz, f) the 64 lanes' 8 values.
+// transposed: the flipped, transposed weights of the backward-data pass (w
+// stays [wco][27][wci], input channels are its wco).
+__global__ void pack_weights_kernel(const float* w, int wci, int cin, int cout, int transposed, uint16_t* wt)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < cout * kpad) {
-        const int co = i / kpad, k = i - co * kpad, t = k / cin_pad, ci = k - t * cin_pad;
-        wt[i] = (t < 27 && ci < cin) ? f2bf(w[((size_t)co * 27 + t) * cin + ci]) : (uint16_t)0;
-    }
-    if (wb && i < cin * kpad_b) {
-        const int ci = i / kpad_b, k = i - ci * kpad_b, t = k / cout, co = k - t * cout;
-        wb[i] = t < 27 ? f2bf(w[((size_t)co * 27 + (26 - t)) * cin + ci]) : (uint16_t)0;
-    }
+    if (i >= cin / 16 * (cout / 16) * kConvFrags * 512) return;
+    const int e = i & 7, lane = (i >> 3) & 63, frag = (i >> 9) % kConvFrags, tile = (i >> 9) / kConvFrags;
+    const int co = tile % (cout / 16) * 16 + (lane & 15), kg = lane >> 4;
+    const int ci = tile / (cout / 16) * 16 + (kg & 1) * 8 + e;
+    const int dz = frag / 5, f = frag % 5, second = kg >> 1;
+    // F1: row f, dx 0 or 1; P: dx 2, rows 0 and 1; Q: dx 2, row 2 from the second
+    const int dy = f < 3 ? f : f == 3 ? second : 2, dx = f < 3 ? second : 2;
+    const int tap = (dz * 3 + dy) * 3 + dx;
+    float v = transposed ? w[((size_t)ci * 27 + (26 - tap)) * wci + co] : w[((size_t)co * 27 + tap) * wci + ci];
+    if (f == 4 && !second) v = 0.0f;
+    wt[i] = f2bf(v);
 }
 
-__global__ void relu_backward_kernel(uint16_t* g, const uint16_t* y, size_t n)
+// The first layer's [16][27][2] weights in conv3_first_kernel's order.
+__global__ void pack_first_weights_kernel(const float* w, uint16_t* wt)
 {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const uint16_t v = y[i];
-        if ((v & 0x8000u) || (v & 0x7fffu) == 0) g[i] = 0;
-    }
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 3 * 512) return;
+    const int e = i & 7, lane = (i >> 3) & 63, row = (i >> 9) * 4 + (lane >> 4), dx = e >> 1;
+    wt[i] = row < 9 && dx < 3 ? f2bf(w[((lane & 15) * 27 + row * 3 + dx) * 2 + (e & 1)]) : (uint16_t)0;
 }
 
-__global__ void pool2_kernel(const uint16_t* x, int D, int H, int W, int C, uint16_t* y)
+// g = (g + its parent's g_low / 8) where the activation y is positive, eight
+// channels a thread
+__global__ void join_gradients_kernel(const uint16_t* gl, int D, int H, int W, int C, const uint16_t* y, uint16_t* g)
 {
-    const int Dl = D / 2, Hl = H / 2, Wl = W / 2;
-    const size_t n = (size_t)Dl * Hl * Wl * C;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const size_t p = i / C;
-        const int xl = (int)(p % Wl), yl = (int)((p / Wl) % Hl), zl = (int)(p / ((size_t)Wl * Hl));
-        float s = 0.0f;
-        for (int a = 0; a < 2; ++a)
-            for (int b = 0; b < 2; ++b)
-                for (int e = 0; e < 2; ++e)
-                    s += bf2f(x[((((size_t)(2 * zl + a) * H) + 2 * yl + b) * W + 2 * xl + e) * C + c]);
-        y[i] = f2bf(s * 0.125f);
-    }
-}
-
-__global__ void pool2_backward_kernel(const uint16_t* gl, int D, int H, int W, int C, uint16_t* g, int accumulate)
-{
-    const size_t n = (size_t)D * H * W * C;
+    const int groups = C / 8;
+    const size_t n = (size_t)D * H * W * groups;
     const int Hl = H / 2, Wl = W / 2;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const size_t m = i / C;
-        const int x = (int)(m % W), y = (int)((m / W) % H), z = (int)(m / ((size_t)W * H));
-        const float v = bf2f(gl[(((size_t)(z / 2) * Hl + y / 2) * Wl + x / 2) * C + c]) * 0.125f;
-        g[i] = f2bf(accumulate ? bf2f(g[i]) + v : v);
-    }
-}
-
-__global__ void up2_backward_kernel(const uint16_t* g, int stride, int c0, int D, int H, int W, int C, uint16_t* gl)
-{
-    const int Dl = D / 2, Hl = H / 2, Wl = W / 2;
-    const size_t n = (size_t)Dl * Hl * Wl * C;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const size_t p = i / C;
-        const int xl = (int)(p % Wl), yl = (int)((p / Wl) % Hl), zl = (int)(p / ((size_t)Wl * Hl));
-        float s = 0.0f;
-        for (int a = 0; a < 2; ++a)
-            for (int b = 0; b < 2; ++b)
-                for (int e = 0; e < 2; ++e)
-                    s += bf2f(g[((((size_t)(2 * zl + a) * H) + 2 * yl + b) * W + 2 * xl + e) * stride + c0 + c]);
-        gl[i] = f2bf(s);
-    }
-}
-
-__global__ void take_channels_kernel(const uint16_t* g, int stride, int c0, size_t voxels, int C, uint16_t* dst,
-                                     int accumulate)
-{
-    const size_t n = voxels * C;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const size_t m = i / C;
-        const int c = (int)(i - m * C);
-        const float v = bf2f(g[m * stride + c0 + c]);
-        dst[i] = f2bf(accumulate ? bf2f(dst[i]) + v : v);
+        const size_t m = i / groups;
+        const int c = (int)(i - m * groups) * 8;
+        const int z = (int)(m / ((size_t)W * H)), r = (int)(m - (size_t)z * W * H), yy = r / W, x = r - yy * W;
+        const u32x4 low = load16(gl + (((size_t)(z / 2) * Hl + yy / 2) * Wl + x / 2) * C + c);
+        const u32x4 act = load16(y + m * C + c);
+        u32x4 v = load16(g + m * C + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float a, b, la, lb;
+            dev::BF16::unpack2(v[e], a, b);
+            dev::BF16::unpack2(low[e], la, lb);
+            v[e] = gated(dev::BF16::pack2(a + la * 0.125f, b + lb * 0.125f), act[e]);
+        }
+        *reinterpret_cast<u32x4*>(g + m * C + c) = v;
     }
 }
 
@@ -549,27 +635,6 @@ __global__ void pack_input_kernel(const float* x, float scale, const float* d, f
         const uint32_t a = f2bf(x[i] * scale), b = d ? f2bf(d[i] * dscale) : 0u;
         *reinterpret_cast<u32x4*>(y + 8 * i) = u32x4{a | (b << 16), 0u, 0u, 0u};
     }
-}
-
-__global__ void head_forward_kernel(const uint16_t* d1, const float* x, float scale, const float* hw, const float* hb,
-                                    size_t n, float* pred)
-{
-    for (size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x; m < n; m += (size_t)gridDim.x * blockDim.x) {
-        const u32x4 a = load16(d1 + m * 16), b = load16(d1 + m * 16 + 8);
-        float s = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            s += hw[2 * e] * bf2f((uint16_t)(a[e] & 0xffffu)) + hw[2 * e + 1] * bf2f((uint16_t)(a[e] >> 16));
-            s += hw[8 + 2 * e] * bf2f((uint16_t)(b[e] & 0xffffu)) + hw[9 + 2 * e] * bf2f((uint16_t)(b[e] >> 16));
-        }
-        pred[m] = x[m] * scale + (s + hb[0]);
-    }
-}
-
-__global__ void unscale_kernel(const float* pred, const float* x, float scale, size_t n, float* out)
-{
-    for (size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x; m < n; m += (size_t)gridDim.x * blockDim.x)
-        out[m] = x[m] + (pred[m] - x[m] * scale) / scale;
 }
 
 constexpr int kRedBlocks = 1024;
@@ -608,28 +673,47 @@ __global__ void __launch_bounds__(kThreads) mse_final_kernel(const double* parti
     if (threadIdx.x == 0) *loss = red[0] / (double)n;
 }
 
-__global__ void head_backward_kernel(const uint16_t* d1, const float* gp, const float* hw, size_t n, uint16_t* gd1,
-                                     float* partial)
+// g_d1 = g_pred hw where d1 is positive; per block the sums of g_pred d1[c] and
+// of g_pred: over each wave's lanes, then over its waves, in a fixed order
+__global__ void __launch_bounds__(kThreads) head_backward_kernel(const uint16_t* d1, const float* gp, const float* hw,
+                                                                 size_t n, uint16_t* gd1, float* partial)
 {
-    __shared__ float red[kThreads * 17];
-    float s[17];
+    __shared__ float red[kThreads / 64][17];
+    float s[17], h[16];
 #pragma unroll
     for (int c = 0; c < 17; ++c) s[c] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) h[c] = hw[c];
     for (size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x; m < n; m += (size_t)gridDim.x * blockDim.x) {
         const float g = gp[m];
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            s[c] += g * bf2f(d1[m * 16 + c]);
-            gd1[m * 16 + c] = f2bf(g * hw[c]);
+        for (int half = 0; half < 2; ++half) {
+            const u32x4 act = load16(d1 + m * 16 + half * 8);
+            u32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int c = half * 8 + 2 * e;
+                float a, b;
+                dev::BF16::unpack2(act[e], a, b);
+                s[c] += g * a;
+                s[c + 1] += g * b;
+                v[e] = gated(dev::BF16::pack2(g * h[c], g * h[c + 1]), act[e]);
+            }
+            *reinterpret_cast<u32x4*>(gd1 + m * 16 + half * 8) = v;
         }
         s[16] += g;
     }
 #pragma unroll
-    for (int c = 0; c < 17; ++c) red[c * kThreads + threadIdx.x] = s[c];
+    for (int c = 0; c < 17; ++c) {
+        float t = s[c];
+#pragma unroll
+        for (int w = 32; w > 0; w /= 2) t += __shfl_xor(t, w);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64][c] = t;
+    }
     __syncthreads();
     if (threadIdx.x < 17) {
         float t = 0.0f;
-        for (int q = 0; q < kThreads; ++q) t += red[threadIdx.x * kThreads + q];
+        for (int q = 0; q < kThreads / 64; ++q) t += red[q][threadIdx.x];
         partial[(size_t)blockIdx.x * 17 + threadIdx.x] = t;
     }
 }
@@ -654,22 +738,59 @@ unsigned grid_for(size_t n)
 
 }  // namespace
 
+namespace {
+int conv_bricks(int D, int H, int W, int* nbx, int* nby)
+{
+    *nbx = (W + kBX - 1) / kBX;
+    *nby = (H + kBY - 1) / kBY;
+    return *nbx * *nby * ((D + kBZ - 1) / kBZ);
+}
+
+// one workgroup per brick, as many on every XCD
+unsigned brick_groups(int bricks) { return (unsigned)((bricks + kXcds - 1) / kXcds * kXcds); }
+
+template <Epilogue kEpi>
+void launch_conv(const ConvArgs& a, hipStream_t stream)
+{
+    int nbx, nby;
+    const int bricks = conv_bricks(a.D, a.H, a.W, &nbx, &nby);
+    const unsigned groups = brick_groups(bricks);
+    // 32 channels a workgroup share one halo, 16 give twice the workgroups:
+    // those where 32 would leave CUs idle
+    if (a.cout % 32 == 0 && bricks * (a.cout / 32) >= 512)
+        conv3_brick_kernel<2, kEpi><<<dim3(groups, a.cout / 32), kConvThreads * 2, 0, stream>>>(a, nbx, nby, bricks);
+    else
+        conv3_brick_kernel<1, kEpi><<<dim3(groups, a.cout / 16), kConvThreads, 0, stream>>>(a, nbx, nby, bricks);
+}
+}  // namespace
+
 void conv3_forward(const ConvArgs& a, hipStream_t stream)
 {
-    if (a.src.ca < 8 || (a.src.ca % 8) || (a.src.cb % 8)) fail("conv3: input channels must be multiples of 8");
-    if (a.kpad != kpad_for(a.src.ca + a.src.cb)) fail("conv3: weight row length mismatch");
-    if (a.src.a_half && ((a.D | a.H | a.W) & 1)) fail("conv3: upsampled input needs even sizes");
-    const int nbx = (a.W + kBX - 1) / kBX, nby = (a.H + kBY - 1) / kBY, nbz = (a.D + kBZ - 1) / kBZ;
-    const unsigned bricks = (unsigned)(nbx * nby * nbz);
-    switch (a.cout) {
-        case 16: conv3_brick_kernel<1><<<bricks, kThreads, 0, stream>>>(a, nbx, nby); break;
-        case 32: conv3_brick_kernel<2><<<bricks, kThreads, 0, stream>>>(a, nbx, nby); break;
-        case 48: launch_conv<3, 2>(a, stream); break;
-        case 64: launch_conv<4, 2>(a, stream); break;
-        case 96: launch_conv<6, 2>(a, stream); break;
-        default: fail("conv3: output channels must be 16, 32, 48, 64 or 96");
+    if (a.src.ca < 16 || (a.src.ca % 16) || (a.src.cb % 16)) fail("conv3: input channels must be multiples of 16");
+    if (a.cout < 16 || a.cout % 16) fail("conv3: output channels must be a multiple of 16");
+    if ((a.src.a_half || a.pool || a.children) && ((a.D | a.H | a.W) & 1)) fail("conv3: halved volumes need even sizes");
+    if (a.head && a.cout != 16) fail("conv3: the head follows 16 channels");
+    if (a.head) {
+        int nbx, nby;
+        const int bricks = conv_bricks(a.D, a.H, a.W, &nbx, &nby);
+        conv3_brick_kernel<1, kHead><<<brick_groups(bricks), kConvThreads, 0, stream>>>(a, nbx, nby, bricks);
+    } else if (a.pool) {
+        launch_conv<kPool>(a, stream);
+    } else if (a.children) {
+        launch_conv<kChildren>(a, stream);
+    } else {
+        launch_conv<kStore>(a, stream);
     }
     hip_check(hipGetLastError(), "conv3 forward launch");
+}
+
+void conv3_first(const float* x, float scale, const float* d, float dscale, int D, int H, int W, const uint16_t* wt,
+                 const float* bias, uint16_t* out, hipStream_t stream)
+{
+    int nbx, nby;
+    const int bricks = conv_bricks(D, H, W, &nbx, &nby);
+    conv3_first_kernel<<<brick_groups(bricks), kThreads, 0, stream>>>(x, scale, d, dscale, D, H, W, wt, bias, out, nbx, nby, bricks);
+    hip_check(hipGetLastError(), "conv3 first layer launch");
 }
 
 int wgrad_chunks(int D, int H, int W, int cin)
@@ -705,60 +826,30 @@ void conv3_weight_grad(const ConvSrc& src, int D, int H, int W, const uint16_t* 
     hip_check(hipGetLastError(), "conv3 weight gradient launch");
 }
 
-void pack_weights(const float* w, int cout, int cin, int cin_pad, uint16_t* wt, uint16_t* wb, hipStream_t stream)
+void pack_weights(const float* w, int wci, int cin, int cout, bool transposed, uint16_t* wt, hipStream_t stream)
 {
-    const int kpad = kpad_for(cin_pad), kpad_b = kpad_for(cout);
-    const int n = std::max(cout * kpad, wb ? cin * kpad_b : 0);
-    pack_weights_kernel<<<(n + kThreads - 1) / kThreads, kThreads, 0, stream>>>(w, cout, cin, cin_pad, wt, kpad, wb,
-                                                                               kpad_b);
+    const size_t n = conv_weight_count(cin, cout);
+    pack_weights_kernel<<<(unsigned)((n + kThreads - 1) / kThreads), kThreads, 0, stream>>>(w, wci, cin, cout, transposed,
+                                                                                           wt);
     hip_check(hipGetLastError(), "weight packing launch");
 }
 
-void relu_backward(uint16_t* g, const uint16_t* y, size_t count, hipStream_t stream)
+void pack_first_weights(const float* w, uint16_t* wt, hipStream_t stream)
 {
-    relu_backward_kernel<<<grid_for(count), kThreads, 0, stream>>>(g, y, count);
+    pack_first_weights_kernel<<<(kFirstWeights + kThreads - 1) / kThreads, kThreads, 0, stream>>>(w, wt);
+    hip_check(hipGetLastError(), "weight packing launch");
 }
 
-void pool2(const uint16_t* x, int D, int H, int W, int C, uint16_t* y, hipStream_t stream)
-{
-    pool2_kernel<<<grid_for((size_t)D * H * W * C / 8), kThreads, 0, stream>>>(x, D, H, W, C, y);
-}
-
-void pool2_backward(const uint16_t* g_low, int D, int H, int W, int C, uint16_t* g_full, int accumulate,
+void join_gradients(const uint16_t* g_low, int D, int H, int W, int C, const uint16_t* y, uint16_t* g,
                     hipStream_t stream)
 {
-    pool2_backward_kernel<<<grid_for((size_t)D * H * W * C), kThreads, 0, stream>>>(g_low, D, H, W, C, g_full,
-                                                                                    accumulate);
-}
-
-void up2_backward(const uint16_t* g, int stride, int c0, int D, int H, int W, int C, uint16_t* g_low,
-                  hipStream_t stream)
-{
-    up2_backward_kernel<<<grid_for((size_t)D * H * W * C / 8), kThreads, 0, stream>>>(g, stride, c0, D, H, W, C,
-                                                                                      g_low);
-}
-
-void take_channels(const uint16_t* g, int stride, int c0, size_t voxels, int C, uint16_t* dst, int accumulate,
-                   hipStream_t stream)
-{
-    take_channels_kernel<<<grid_for(voxels * C), kThreads, 0, stream>>>(g, stride, c0, voxels, C, dst, accumulate);
+    join_gradients_kernel<<<grid_for((size_t)D * H * W * C / 8), kThreads, 0, stream>>>(g_low, D, H, W, C, y, g);
 }
 
 void pack_input(const float* x, float scale, const float* d, float dscale, size_t count, uint16_t* y,
                 hipStream_t stream)
 {
     pack_input_kernel<<<grid_for(count), kThreads, 0, stream>>>(x, scale, d, dscale, count, y);
-}
-
-void head_forward(const uint16_t* d1, const float* x, float scale, const float* hw, const float* hb, size_t voxels,
-                  float* pred, hipStream_t stream)
-{
-    head_forward_kernel<<<grid_for(voxels), kThreads, 0, stream>>>(d1, x, scale, hw, hb, voxels, pred);
-}
-
-void unscale_prediction(const float* pred, const float* x, float scale, size_t voxels, float* out, hipStream_t stream)
-{
-    unscale_kernel<<<grid_for(voxels), kThreads, 0, stream>>>(pred, x, scale, voxels, out);
 }
 
 void mse_loss(const float* pred, const float* target, float scale, size_t voxels, float* g_pred, double* partial,

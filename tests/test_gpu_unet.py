@@ -85,6 +85,22 @@ def test_scale_only_rescales():
     assert err < 3e-2, err
 
 
+def test_large_volume_equals_its_crop():
+    """A volume large enough for the workgroups of 32 channels (512 bricks at
+    half resolution) against a crop of it that takes 16-channel ones: the sums
+    run in the same order, and voxels further from the crop's faces than the
+    network sees (22 voxels, 24 here) read the same inputs, so they are equal."""
+    shape, at, n, margin = (128, 128, 256), (32, 36, 100), 64, 24
+    params, x, d, _ = setup_case(shape, 17)
+    xd, dd = torch.from_numpy(x).cuda(), torch.from_numpy(d).cuda()
+    whole = Lrn.CorrectionNet(shape, params).predict(xd, dd, 1.0)
+    crop = tuple(slice(a, a + n) for a in at)
+    part = Lrn.CorrectionNet((n, n, n), params).predict(xd[crop].contiguous(), dd[crop].contiguous(), 1.0)
+    inner = (slice(margin, n - margin),) * 3
+    torch.cuda.synchronize()
+    assert torch.equal(whole[crop][inner], part[inner])
+
+
 # (the brick kernels' edges: rows of 68 voxels are two bricks and a remainder of
 # 4 at full resolution, 34 and 17 at the lower ones, 12 slices one and a half
 # weight-gradient bricks at half resolution; the same bounds)
