@@ -22,6 +22,7 @@ OBJ = os.path.join(PKG, "_build")
 
 SOURCES = [
     "projectors.hip",
+    "plane_projectors.hip",
     "fused.hip",
     "fused_inst.hip",
     "unet_kernels.hip",

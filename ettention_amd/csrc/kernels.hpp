@@ -41,6 +41,13 @@ void launch_forward_project(const SlabParams& s, const RayParams& r, etn_voxel_t
                             const uint8_t* mask, float* projection, float* traversal_length, hipStream_t stream);
 void launch_back_project(const SlabParams& s, const BpParams& b, etn_voxel_type vt, void* volume,
                          const uint8_t* mask, const float* residual, const float* ray_length, hipStream_t stream);
+// The same for one single-axis tilt projection with one sample and no mask
+// (plane_projectors.hip); false, with nothing launched, where the geometry is
+// another one.
+bool plane_forward_project(const SlabParams& s, const RayParams& r, etn_voxel_type vt, const void* volume,
+                           float* projection, float* traversal_length, hipStream_t stream);
+bool plane_back_project(const SlabParams& s, const BpParams& b, etn_voxel_type vt, void* volume, const float* residual,
+                        const float* ray_length, hipStream_t stream);
 void launch_compare(uint32_t n, const float* real, const float* virt, float* residual, hipStream_t stream);
 // real in its storage type (measured projections stored as f16 or bf16)
 void launch_compare(uint32_t n, const void* real, etn_voxel_type real_type, const float* virt, float* residual,
