@@ -481,9 +481,9 @@ def run_wbp(args):
     """Weighted back projection: a step is one whole WBP reconstruction (every
     projection filtered, its ray length computed and back-projected with
     lambda / N).  GUPS = V x N / seconds per reconstruction.  The dominant
-    kernel is the fused back projection (eight projections per volume sweep),
-    timed with HIP events around its launches in one more run; its
-    algorithmic bytes are those of one sweep for B = 8 projections, 2 s V + 8 P B
+    kernel is the back projection sweep (up to 64 projections per volume
+    sweep), timed with HIP events around its launches in one more run; its
+    algorithmic bytes are those of one sweep for its B projections, 2 s V + 8 P B
     (the volume read and written once, residual and length images read)."""
     import torch
     import ettention_amd as E
@@ -533,8 +533,10 @@ def run_wbp(args):
     del r
     torch.cuda.empty_cache()
     if kernel == 0:
-        B = 8
-        name = "fused_plane_kernel (back projections only, %d projections per launch)" % B
+        # a sweep carries up to 64 projections; launches of the fused kernels eight
+        B = N / launches if launches * 8 < N else 8
+        name = "%s (back projections only, %g projections per launch)" % (
+            "sweep_back_kernel" if launches * 8 < N else "fused_plane_kernel", B)
     else:
         B = 1
         name = "back_project_kernel (generic, one projection with lambda / N)"

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 #include "etn/etn.h"
 
@@ -48,6 +49,35 @@ bool plane_forward_project(const SlabParams& s, const RayParams& r, etn_voxel_ty
                            float* projection, float* traversal_length, hipStream_t stream);
 bool plane_back_project(const SlabParams& s, const BpParams& b, etn_voxel_type vt, void* volume, const float* residual,
                         const float* ray_length, hipStream_t stream);
+// One projection of sweep_back_project (device table entries): the matrix
+// entries of a single-axis tilt (u = m0 x + m8 z + m12, v = m5 y + m13), the
+// sample's offset and lambda times its chord, the images.
+struct BackView {
+    float m0, m8, m12, m5, m13;
+    float sx, sy, sz, weight;
+    const float* residual;
+    const float* length;
+};
+// The table entry for a projection with one sample; false where its geometry
+// is another one or a tile's columns would not fit.
+bool make_back_view(const SlabParams& s, const BpParams& b, const float* residual, const float* length, BackView* out);
+// Detector rows whose rays have equal lengths, column by column: 1 for rows of
+// rays inside the volume in y, 0 for the others (whose lengths are not known
+// to be equal).
+std::vector<uint8_t> row_classes(const SlabParams& s, const RayParams& r);
+// Plane groups of a sweep of the n projections (host entries), and the run of
+// them whose planes read rows of class 1; count 0 where the projections do not
+// agree on a plane's rows (no sweep then).
+struct SweepGroups {
+    int count = 0, begin = 0, end = 0;
+};
+SweepGroups sweep_groups(const SlabParams& s, const BackView* views, int n, uint32_t nv,
+                         const std::vector<uint8_t>& row_class);
+// Back-projects views[0 .. n) (device memory) in order in one sweep of the
+// volume with the fused kernels' fast arithmetic, operation for operation,
+// rounding to the storage type after each.
+void sweep_back_project(const SlabParams& s, const SweepGroups& g, const BackView* views, int n, uint32_t nu,
+                        uint32_t nv, etn_voxel_type vt, void* volume, hipStream_t stream);
 void launch_compare(uint32_t n, const float* real, const float* virt, float* residual, hipStream_t stream);
 // real in its storage type (measured projections stored as f16 or bf16)
 void launch_compare(uint32_t n, const void* real, etn_voxel_type real_type, const float* virt, float* residual,

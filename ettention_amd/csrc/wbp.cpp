@@ -93,10 +93,42 @@ WeightedBackProjection::WeightedBackProjection(const etn_reconstruction_desc& d,
     taps_.allocate(k.size() * sizeof(float));
     ETN_HIP(hipMemcpyAsync(taps_.get(), k.data(), taps_.bytes(), hipMemcpyHostToDevice, stream_));
     ETN_HIP(hipStreamSynchronize(stream_));
-    if ((d.flags & (ETN_RECON_FLAG_GENERIC_KERNELS | ETN_RECON_FLAG_EXACT_ARITHMETIC)) == 0)
-        fused_ = FusedBackProjector::create(volume_.get(), geometries_, nu, nv, d.bp_samples ? d.bp_samples : 1,
-                                            (d.flags & ETN_RECON_FLAG_LDS_BACK_PROJECTION) != 0, stream_);
-    if (fused_) {
+    if ((d.flags & (ETN_RECON_FLAG_GENERIC_KERNELS | ETN_RECON_FLAG_EXACT_ARITHMETIC)) == 0) {
+        // the sweep takes every projection or none; the whole volume is one slab
+        const uint32_t samples = d.bp_samples ? d.bp_samples : 1;
+        std::vector<dev::BackView> views(geometries_.size());
+        const VolumeProperties whole = wholeVolume();
+        bool sweep = samples == 1 && (d.flags & ETN_RECON_FLAG_LDS_BACK_PROJECTION) == 0;
+        const uint32_t slots = std::min(count_, kChunk);
+        if (sweep) chunk_.allocate(sizeof(float) * 2 * pixels_ * slots);
+        for (size_t i = 0; sweep && i < views.size(); ++i) {
+            const float* image = chunk_.as<float>() + 2 * pixels_ * (i % kChunk);
+            sweep = dev::make_back_view(make_slab_params(whole, 0),
+                                        make_bp_params(geometries_[i], whole, samples, lambda_ / (float)count_), image,
+                                        image + pixels_, &views[i]);
+        }
+        if (sweep) {
+            const dev::SlabParams slab = make_slab_params(whole, 0);
+            // rows whose rays lie inside the volume in y at every tilt
+            std::vector<uint8_t> rows(nv, 1);
+            for (const ParallelScannerGeometry& g : geometries_) {
+                const std::vector<uint8_t> one = dev::row_classes(slab, make_ray_params(g, 1));
+                for (uint32_t r = 0; r < nv; ++r) rows[r] = rows[r] && one[r];
+            }
+            groups_ = dev::sweep_groups(slab, views.data(), (int)views.size(), nv, rows);
+            sweep = groups_.count > 0;
+        }
+        if (sweep) {
+            views_.allocate(sizeof(dev::BackView) * views.size());
+            ETN_HIP(hipMemcpyAsync(views_.get(), views.data(), views_.bytes(), hipMemcpyHostToDevice, stream_));
+            ETN_HIP(hipStreamSynchronize(stream_));
+        } else {
+            chunk_.release();
+            fused_ = FusedBackProjector::create(volume_.get(), geometries_, nu, nv, samples,
+                                                (d.flags & ETN_RECON_FLAG_LDS_BACK_PROJECTION) != 0, stream_);
+        }
+    }
+    if (usesFusedPath()) {
         std::vector<dev::RayParams> geo;
         for (const ParallelScannerGeometry& g : geometries_) geo.push_back(make_ray_params(g, 1));
         rays_.allocate(sizeof(dev::RayParams) * std::max<size_t>(geo.size(), 1));
@@ -117,34 +149,76 @@ void WeightedBackProjection::filter(const float* src, float* dst)
     dev::launch_ramp_filter(params_, taps_.as<float>(), src, dst, stream_);
 }
 
+// The volume as one slab: its slabs are contiguous in z, and a back projection
+// treats every voxel alone.
+VolumeProperties WeightedBackProjection::wholeVolume() const
+{
+    etn_volume_geometry g{};
+    const VolumeProperties& v = volume_->properties();
+    g.resolution[0] = v.nx();
+    g.resolution[1] = v.ny();
+    g.resolution[2] = v.nz();
+    v.bbox_min().store(g.bbox_min);
+    v.bbox_max().store(g.bbox_max);
+    g.subvolume_count = 1;
+    return VolumeProperties(g);
+}
+
+// Filtered images and ray lengths of projections first .. first + count - 1
+// into the slots of chunk_, one launch each (one launch per image had cost 13
+// and 4 us each, most of it launch and ramp-up).
+void WeightedBackProjection::filterChunk(uint32_t first, uint32_t count)
+{
+    const VolumeProperties& vp = setup_->getVolume();
+    float bmin[3], bmax[3];
+    vp.bbox_min().store(bmin);
+    vp.bbox_max().store(bmax);
+    dev::launch_ramp_filter_batch(params_, taps_.as<float>(), projections_ + (size_t)first * pixels_, pixels_,
+                                  chunk_.as<float>(), 2 * pixels_, count, stream_);
+    dev::launch_ray_length_batch(bmin, bmax, rays_.as<dev::RayParams>() + first, count, params_.nu, params_.nv,
+                                 chunk_.as<float>() + pixels_, 2 * pixels_, stream_);
+}
+
 void WeightedBackProjection::run() { runNiterations(count_); }
 
 void WeightedBackProjection::runNiterations(uint32_t n)
 {
     if (n > count_) fail("WBP: more projections requested than the stack holds");
+    if (views_.get()) {
+        // filtered images and ray lengths of up to kChunk projections, then
+        // their back projections in stack order in one sweep of the volume
+        const dev::SlabParams slab = make_slab_params(wholeVolume(), 0);
+        for (uint32_t i0 = 0; i0 < n; i0 += kChunk) {
+            const uint32_t k = std::min(n - i0, kChunk);
+            filterChunk(i0, k);
+            hipEvent_t ev[2] = {nullptr, nullptr};
+            if (launch_ms_) {
+                for (auto& e : ev) ETN_HIP(hipEventCreate(&e));
+                ETN_HIP(hipEventRecord(ev[0], stream_));
+            }
+            dev::sweep_back_project(slab, groups_, views_.as<dev::BackView>() + i0, (int)k, params_.nu, params_.nv,
+                                    volume_->voxel_type(), volume_->data(), stream_);
+            if (launch_ms_) {
+                ETN_HIP(hipEventRecord(ev[1], stream_));
+                ETN_HIP(hipEventSynchronize(ev[1]));
+                float ms = 0.0f;
+                ETN_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
+                launch_ms_->push_back(ms);
+                for (auto& e : ev) (void)hipEventDestroy(e);
+            }
+        }
+        return;
+    }
     if (fused_) {
-        // filtered images and ray lengths of up to 64 projections, then their
-        // back projections in stack order, eight per volume sweep
-        constexpr uint32_t kChunk = 64;
-        DeviceBuffer chunk(sizeof(float) * 2 * pixels_ * std::min(n, kChunk));
-        const VolumeProperties& vp = setup_->getVolume();
-        float bmin[3], bmax[3];
-        vp.bbox_min().store(bmin);
-        vp.bbox_max().store(bmax);
+        // the same chunks, eight projections per volume sweep
+        if (!chunk_.get()) chunk_.allocate(sizeof(float) * 2 * pixels_ * std::min(count_, kChunk));
         for (uint32_t i0 = 0; i0 < n; i0 += kChunk) {
             std::vector<uint32_t> idx;
             std::vector<const float*> res, len;
             const uint32_t i1 = std::min(n, i0 + kChunk);
-            // the chunk's projections filtered in one launch and their ray
-            // lengths in another (one launch per image had cost 13 and 4 us
-            // each, most of it launch and ramp-up)
-            dev::launch_ramp_filter_batch(params_, taps_.as<float>(), projections_ + (size_t)i0 * pixels_, pixels_,
-                                          chunk.as<float>(), 2 * pixels_, i1 - i0, stream_);
-            dev::launch_ray_length_batch(bmin, bmax, rays_.as<dev::RayParams>() + i0, i1 - i0,
-                                         geometries_[i0].nu(), geometries_[i0].nv(),
-                                         chunk.as<float>() + pixels_, 2 * pixels_, stream_);
+            filterChunk(i0, i1 - i0);
             for (uint32_t i = i0; i < i1; ++i) {
-                float* f = chunk.as<float>() + 2 * pixels_ * (i - i0);
+                float* f = chunk_.as<float>() + 2 * pixels_ * (i - i0);
                 idx.push_back(i);
                 res.push_back(f);
                 len.push_back(f + pixels_);
@@ -170,7 +244,7 @@ void WeightedBackProjection::synchronize() { ETN_HIP(hipStreamSynchronize(stream
 double WeightedBackProjection::timeKernels(int* kernel, uint32_t* launches)
 {
     std::vector<float> ms;
-    if (fused_) {
+    if (usesFusedPath()) {
         *kernel = 0;
         launch_ms_ = &ms;
         try {

@@ -30,13 +30,14 @@ public:
     GpuVolume* getReconstructedVolume() override { return volume_.get(); }
     void synchronize() override;
     hipStream_t stream() const override { return stream_; }
-    // Single-axis tilt geometries back-project on the fused kernels, eight
-    // projections per volume sweep (fast arithmetic), unless the generic
-    // kernels or exact arithmetic are asked for.
-    bool usesFusedPath() const override { return fused_ != nullptr; }
+    // Single-axis tilt geometries back-project up to kChunk projections per
+    // volume sweep, or on the fused kernels eight (oversampled, the LDS back
+    // projection), with fast arithmetic, unless the generic kernels or exact
+    // arithmetic are asked for.
+    bool usesFusedPath() const override { return fused_ != nullptr || views_.get() != nullptr; }
     // One more run() with HIP events around the back projections: the average
-    // fused launch carrying eight projections (*kernel = 0), or the generic
-    // back projection (*kernel = 2).  Adds to the volume.
+    // sweep, or fused launch carrying eight projections (*kernel = 0), or the
+    // generic back projection (*kernel = 2).  Adds to the volume.
     double timeKernels(int* kernel, uint32_t* launches) override;
 
     // GenerateRamLakKernel.cl: value at position p = i - resolution / 2 is 1/4
@@ -49,6 +50,10 @@ public:
     void filter(const float* src, float* dst);
 
 private:
+    static constexpr uint32_t kChunk = 64;
+    void filterChunk(uint32_t first, uint32_t count);
+    VolumeProperties wholeVolume() const;
+
     hipStream_t stream_ = nullptr;
     bool own_stream_ = false;
     uint32_t count_;
@@ -66,7 +71,10 @@ private:
     DeviceBuffer taps_;
     dev::RampFilterParams params_;
     std::unique_ptr<FusedBackProjector> fused_;
-    DeviceBuffer rays_;   // fused path: every projection's ray geometry, for the batched ray lengths
+    DeviceBuffer rays_;   // fused paths: every projection's ray geometry, for the batched ray lengths
+    DeviceBuffer views_;  // sweep path: every projection's table entry (its images: a slot of chunk_)
+    dev::SweepGroups groups_;
+    DeviceBuffer chunk_;  // filtered images and ray lengths of up to kChunk projections
     std::vector<float>* launch_ms_ = nullptr;    // set while timeKernels runs
 };
 
