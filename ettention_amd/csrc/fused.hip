@@ -540,6 +540,24 @@ private:
     size_t passCount() const;
     void tuneTiles(hipStream_t stream);
     float timeSchedule(const Schedule& s, hipStream_t stream) const;
+    void plan_split(hipStream_t stream);
+    void enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* ev) const;
+
+    // An iteration as separate sweeps (blocks of several projections): per block
+    // the back projections of the block before it, all in one sweep, then the
+    // block's forward projections, up to kSweepForward a sweep.
+    struct ForwardSweep {
+        int first, count, zdir;
+    };
+    struct SplitBlock {
+        int back_first, back_count;
+        std::vector<ForwardSweep> forward;
+    };
+    std::vector<SplitBlock> split_;     // empty: the fused passes
+    bool split_off_ = false;            // a tile or workgroup shape was asked for
+    dev::SlabParams split_slab_;
+    dev::SweepGroups split_groups_;
+    DeviceBuffer split_back_, split_forward_;
 
     std::vector<MemberPlan> members_;
     etn_voxel_type vt_;
@@ -566,6 +584,105 @@ FusedEngineImpl::FusedEngineImpl(std::vector<MemberPlan> members, etn_voxel_type
     ETN_HIP(hipGetDevice(&dev));
     ETN_HIP(hipDeviceGetAttribute(&dev_cus_, hipDeviceAttributeMultiprocessorCount, dev));
     upload(stream);
+    plan_split(stream);
+}
+
+// The fused pass reads the volume once for a block's back and forward
+// projections, but works out every voxel's column and every ray's steps in
+// every plane: with several projections a pass it is bound by that (512 x 512 x
+// 256, blocks of 8: 0.61 ms a pass, 0.1 ms of memory traffic).  Separate sweeps
+// share them among planes and read the volume once more (0.21 ms back, 0.17 ms
+// forward a block).  One projection a pass (SART) is bound by the traffic (512^3:
+// 0.21 ms a pass, the time of a copy of the volume) and stays fused.
+void FusedEngineImpl::plan_split(hipStream_t stream)
+{
+    split_.clear();
+    if (members_.size() != 1 || exact_ || mask_ || over_ || sr_ || cap_ || !reg_bp_) return;
+    const MemberPlan& m = members_[0];
+    if (m.bmax < 2) return;
+    BlockIterativeReconstructionOperator& op = *m.op;
+    GpuVolume* vol = op.getReconstructedVolume();
+    const VolumeProperties vp = whole_volume(vol->properties());
+    const dev::SlabParams slab = make_slab_params(vp, 0);
+    auto image = [&](uint32_t parity, uint32_t slot, int which) {
+        return m.images.as<float>() + m.pixels * ((((size_t)parity * m.bmax + slot) * 2) + which);
+    };
+    std::vector<SplitBlock> blocks;
+    std::vector<dev::BackView> back;
+    std::vector<dev::ForwardView> forward;
+    std::vector<uint8_t> rows(m.nv, 1);
+    int back_first = 0, back_count = 0;
+    const uint32_t nb = op.GetBlockCount();
+    for (uint32_t b = 0; b < nb; ++b) {
+        const uint32_t bs = op.getBlockSize(b), parity = b & 1u;
+        SplitBlock block{back_first, back_count, {}};
+        back_first = (int)back.size();
+        back_count = (int)bs;
+        // long-object compensation uses the block's last geometry (compensateLongObject)
+        const ParallelScannerGeometry& last = op.geometry(op.getPhysicalProjectionIndex(b, bs - 1));
+        const float loc_c = m.use_loc ? last.traversal_length_through(vp.bbox_min(), vp.bbox_max()) : 0.0f;
+        for (const int zdir : {-1, 1}) {
+            const int first = (int)forward.size();
+            for (uint32_t p = 0; p < bs; ++p) {
+                const uint32_t phys = op.getPhysicalProjectionIndex(b, p);
+                const ParallelScannerGeometry& g = op.geometry(phys);
+                dev::ForwardView f{};
+                g.ray_direction().store(f.ray);
+                if ((f.ray[2] > 0.0f) != (zdir > 0)) continue;
+                g.source_base().store(f.source);
+                g.horizontal_pitch().store(f.h);
+                g.vertical_pitch().store(f.v);
+                f.measured = op.realProjection(phys);
+                f.measured_type = op.projectionType();
+                f.residual = image(parity, p, 0);
+                f.length = image(parity, p, 1);
+                f.loc_c = loc_c;
+                f.use_loc = m.use_loc ? 1 : 0;
+                if (!dev::forward_view_fits(slab, f, (uint32_t)m.nu, (uint32_t)m.nv)) return;
+                // (a row lies in one plane for every projection: plan_member)
+                const std::vector<uint8_t> one = dev::row_classes(slab, make_ray_params(g, 1));
+                for (int r = 0; r < m.nv; ++r) rows[r] = rows[r] && one[r];
+                forward.push_back(f);
+            }
+            for (int i = first; i < (int)forward.size(); i += dev::kSweepForward)
+                block.forward.push_back({i, std::min(dev::kSweepForward, (int)forward.size() - i), zdir});
+        }
+        for (uint32_t p = 0; p < bs; ++p) {
+            dev::BackView v;
+            const dev::BpParams bp = make_bp_params(op.geometry(op.getPhysicalProjectionIndex(b, p)), vp, 1,
+                                                    m.lambda / (float)bs);
+            if (!dev::make_back_view(slab, bp, image(parity, p, 0), image(parity, p, 1), &v)) return;
+            back.push_back(v);
+        }
+        blocks.push_back(std::move(block));
+    }
+    blocks.push_back({back_first, back_count, {}});
+    const dev::SweepGroups groups = dev::sweep_groups(slab, back.data(), (int)back.size(), (uint32_t)m.nv, rows);
+    if (groups.count == 0) return;
+    split_back_.allocate(sizeof(dev::BackView) * back.size());
+    split_forward_.allocate(sizeof(dev::ForwardView) * forward.size());
+    ETN_HIP(hipMemcpyAsync(split_back_.get(), back.data(), split_back_.bytes(), hipMemcpyHostToDevice, stream));
+    ETN_HIP(hipMemcpyAsync(split_forward_.get(), forward.data(), split_forward_.bytes(), hipMemcpyHostToDevice, stream));
+    ETN_HIP(hipStreamSynchronize(stream));
+    split_slab_ = slab;
+    split_groups_ = groups;
+    split_ = std::move(blocks);
+}
+
+void FusedEngineImpl::enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* ev) const
+{
+    const MemberPlan& m = members_[0];
+    void* volume = m.op->getReconstructedVolume()->data();
+    for (size_t k = 0; k < split_.size(); ++k) {
+        const SplitBlock& b = split_[k];
+        if (ev) ETN_HIP(hipEventRecord((*ev)[2 * k], stream));
+        dev::sweep_back_project(split_slab_, split_groups_, split_back_.as<dev::BackView>() + b.back_first, b.back_count,
+                                (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
+        for (const ForwardSweep& f : b.forward)
+            dev::sweep_forward_project(split_slab_, split_forward_.as<dev::ForwardView>() + f.first, f.count, f.zdir,
+                                       (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
+        if (ev) ETN_HIP(hipEventRecord((*ev)[2 * k + 1], stream));
+    }
 }
 
 // Passes and volume descriptors of every member under the current tiles, and
@@ -786,7 +903,11 @@ void FusedEngineImpl::enqueue(const Schedule& s, size_t first, size_t last, hipS
     }
 }
 
-void FusedEngineImpl::enqueueIteration(hipStream_t stream) { enqueue(sched_, 0, sched_.launches.size(), stream, nullptr); }
+void FusedEngineImpl::enqueueIteration(hipStream_t stream)
+{
+    if (!split_.empty() && !split_off_) enqueueSplit(stream, nullptr);
+    else enqueue(sched_, 0, sched_.launches.size(), stream, nullptr);
+}
 
 double FusedEngineImpl::residualNorm(size_t member, double* scratch, hipStream_t stream)
 {
@@ -876,17 +997,20 @@ void FusedEngineImpl::check(hipStream_t stream)
 
 std::vector<FusedPlaneEngine::LaunchTime> FusedEngineImpl::timeIteration(hipStream_t stream)
 {
-    const size_t n = sched_.launches.size();
+    const bool split = !split_.empty() && !split_off_;
+    const size_t n = split ? split_.size() : sched_.launches.size();
     std::vector<hipEvent_t> ev(2 * n);
     for (auto& e : ev) ETN_HIP(hipEventCreate(&e));
-    enqueue(sched_, 0, n, stream, &ev);
+    if (split) enqueueSplit(stream, &ev);
+    else enqueue(sched_, 0, n, stream, &ev);
     ETN_HIP(hipStreamSynchronize(stream));
     std::vector<LaunchTime> out;
     for (size_t k = 0; k < n; ++k) {
-        if (sched_.launches[k].groups == 0) continue;
+        if (!split && sched_.launches[k].groups == 0) continue;
         float ms = 0.0f;
         ETN_HIP(hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]));
-        out.push_back({ms, sched_.launches[k].steady});
+        // (a block's sweeps count as one launch)
+        out.push_back({ms, split ? split_[k].back_count > 0 && !split_[k].forward.empty() : sched_.launches[k].steady});
     }
     for (auto& e : ev) (void)hipEventDestroy(e);
     return out;
@@ -898,6 +1022,7 @@ void FusedEngineImpl::setTile(size_t member, int planes, int band, hipStream_t s
     const Tile t{planes, band};
     if (!tile_fits(members_[member], t)) fail("tile does not fit this volume (planes must divide ny, LDS limit)");
     members_[member].tile = t;
+    split_off_ = true;   // a tile is one of the fused passes
     upload(stream);
 }
 
@@ -943,6 +1068,7 @@ size_t FusedEngineImpl::passCount() const
 void FusedEngineImpl::setThreads(int threads, hipStream_t stream)
 {
     if (!threadsFit(threads)) fail("workgroup size must be 256 or 512 threads and fit every member");
+    split_off_ = true;   // a workgroup shape is the fused passes'
     useThreads(threads);
     upload(stream);
 }
@@ -1007,6 +1133,7 @@ void FusedEngineImpl::tuneTiles(hipStream_t stream)
 // the engine's whole schedule; keep the fastest shape with its tiles.
 void FusedEngineImpl::autotune(hipStream_t stream)
 {
+    if (!split_.empty() && !split_off_) return;   // the sweeps have no tiles
     // Candidates: workgroup shape x cap on the rays per thread.  A lower cap
     // needs fewer registers per thread (more waves per SIMD: two rays take
     // about 120 VGPRs, eight about 190) but splits a block's forward

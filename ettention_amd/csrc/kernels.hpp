@@ -78,6 +78,27 @@ SweepGroups sweep_groups(const SlabParams& s, const BackView* views, int n, uint
 // rounding to the storage type after each.
 void sweep_back_project(const SlabParams& s, const SweepGroups& g, const BackView* views, int n, uint32_t nu,
                         uint32_t nv, etn_voxel_type vt, void* volume, hipStream_t stream);
+// One forward projection of sweep_forward_project (device table entries); the
+// residual measured - line integral (with long-object compensation when
+// use_loc) and the ray length are written.
+struct ForwardView {
+    float source[3], h[3], v[3], ray[3];
+    const void* measured;       // nv x nu in measured_type
+    int measured_type;
+    float* residual;
+    float* length;
+    float loc_c;
+    int use_loc;
+};
+constexpr int kSweepForward = 8;    // projections of a sweep
+// Whether sweep_forward_project takes a projection (a plane per detector row,
+// the same steps in every row, rays below the 2048-step limit).
+bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, uint32_t nv);
+// Forward-projects n <= kSweepForward views (device memory) whose rays move in
+// the z direction zdir (or stay in z) in one sweep of the volume, with the fused
+// kernels' fast arithmetic, operation for operation.
+void sweep_forward_project(const SlabParams& s, const ForwardView* views, int n, int zdir, uint32_t nu, uint32_t nv,
+                           etn_voxel_type vt, const void* volume, hipStream_t stream);
 void launch_compare(uint32_t n, const float* real, const float* virt, float* residual, hipStream_t stream);
 // real in its storage type (measured projections stored as f16 or bf16)
 void launch_compare(uint32_t n, const void* real, etn_voxel_type real_type, const float* virt, float* residual,

@@ -144,3 +144,27 @@ def test_wbp_register_back_projection_equals_lds():
             vols.append(r.get_reconstructed_volume().cpu().numpy())
     np.testing.assert_array_equal(vols[0], vols[2])
     np.testing.assert_array_equal(vols[1], vols[3])
+
+
+# blocks as separate sweeps (the default) against the fused passes on the LDS
+# back projection: nx off a multiple of 4, rows beside the volume, one, two and
+# four planes a workgroup, several rays a thread, both z directions, more
+# projections in a block than in a sweep
+SWEEPS = [((61, 20, 33), 17, 4, 60.0, "float"), ((64, 70, 40), 23, 8, 60.0, "float"), ((64, 520, 12), 9, 3, 60.0, "float"),
+          ((520, 9, 16), 11, 8, 60.0, "bfloat16"), ((48, 33, 30), 40, 0, 60.0, "half"), ((40, 130, 24), 30, 5, 150.0, "float")]
+
+
+@pytest.mark.parametrize("shape,ntilts,block,reach,voxel", SWEEPS)
+@pytest.mark.parametrize("loc", [False, True])
+def test_block_sweeps_equal_the_fused_passes(shape, ntilts, block, reach, voxel, loc):
+    nx, ny, nz = shape
+    rng = np.random.default_rng(ntilts)
+    case = dict(volume=E.VolumeGeometry.make(shape), base_geometry=E.ScannerGeometry.mrc_base(nx, ny),
+                tilt_angles=np.linspace(-reach, reach, ntilts).astype(np.float32),
+                projections=torch.from_numpy(rng.normal(1.0, 0.3, (ntilts, ny, nx)).astype(np.float32)).cuda(),
+                algorithm="blockiterative" if block else "sirt", block_size=block, lam=0.3, voxel_type=voxel,
+                use_long_object_compensation=loc)
+    v, norm = run(case)
+    w, ref = run(case, flags=LDS)
+    np.testing.assert_array_equal(v, w)
+    assert norm == ref
