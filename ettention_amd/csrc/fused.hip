@@ -597,9 +597,24 @@ FusedEngineImpl::FusedEngineImpl(std::vector<MemberPlan> members, etn_voxel_type
 void FusedEngineImpl::plan_split(hipStream_t stream)
 {
     split_.clear();
-    if (members_.size() != 1 || exact_ || mask_ || over_ || sr_ || cap_ || !reg_bp_) return;
+    if (members_.size() != 1 || exact_ || sr_ || cap_ || !reg_bp_) return;
     const MemberPlan& m = members_[0];
-    if (m.bmax < 2) return;
+    const bool plain = !over_ && !m.mask;
+    // Where the sweeps are the faster (fused passes against sweeps, 31 tilts, n^3
+    // f32 voxels).  They are two launches a block, of fewer workgroups:
+    //   blocks of 8: 96^3 318 / 326 us, 128^3 356 / 348, 256^3 928 / 697
+    //   blocks of 4: 128^3 387 / 455, 256^3 1000 / 889;  of 2: 256^3 1115 / 1328
+    //   masked, 8: 96^3 408 / 279, 256^3 1053 / 937;  masked, 4: 128^3 409 / 430
+    //   2 x 2 sub-rays, 4 samples: 64^3 587 / 637, 80^3 730 / 699, 96^3 841 / 788
+    //   4 x 4 sub-rays, 1 sample: 96^3 684 / 718
+    const size_t voxels = (size_t)m.nx * m.ny * m.nz;
+    if (over_) {
+        if (voxels < (m.bp_samples > 1 ? (size_t)500000 : (size_t)1 << 23)) return;
+    } else if (m.mask) {
+        if (m.bmax < 8 || voxels < (size_t)1 << 19) return;
+    } else {
+        if (m.bmax < 4 || voxels < (size_t)1 << (m.bmax < 8 ? 23 : 21)) return;
+    }
     BlockIterativeReconstructionOperator& op = *m.op;
     GpuVolume* vol = op.getReconstructedVolume();
     const VolumeProperties vp = whole_volume(vol->properties());
@@ -609,6 +624,7 @@ void FusedEngineImpl::plan_split(hipStream_t stream)
     };
     std::vector<SplitBlock> blocks;
     std::vector<dev::BackView> back;
+    std::vector<dev::SampleView> samples;
     std::vector<dev::ForwardView> forward;
     std::vector<uint8_t> rows(m.nv, 1);
     int back_first = 0, back_count = 0;
@@ -616,7 +632,7 @@ void FusedEngineImpl::plan_split(hipStream_t stream)
     for (uint32_t b = 0; b < nb; ++b) {
         const uint32_t bs = op.getBlockSize(b), parity = b & 1u;
         SplitBlock block{back_first, back_count, {}};
-        back_first = (int)back.size();
+        back_first += back_count;
         back_count = (int)bs;
         // long-object compensation uses the block's last geometry (compensateLongObject)
         const ParallelScannerGeometry& last = op.geometry(op.getPhysicalProjectionIndex(b, bs - 1));
@@ -638,7 +654,7 @@ void FusedEngineImpl::plan_split(hipStream_t stream)
                 f.length = image(parity, p, 1);
                 f.loc_c = loc_c;
                 f.use_loc = m.use_loc ? 1 : 0;
-                if (!dev::forward_view_fits(slab, f, (uint32_t)m.nu, (uint32_t)m.nv)) return;
+                if (!dev::forward_view_fits(slab, f, (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, m.mask != nullptr)) return;
                 // (a row lies in one plane for every projection: plan_member)
                 const std::vector<uint8_t> one = dev::row_classes(slab, make_ray_params(g, 1));
                 for (int r = 0; r < m.nv; ++r) rows[r] = rows[r] && one[r];
@@ -648,24 +664,33 @@ void FusedEngineImpl::plan_split(hipStream_t stream)
                 block.forward.push_back({i, std::min(dev::kSweepForward, (int)forward.size() - i), zdir});
         }
         for (uint32_t p = 0; p < bs; ++p) {
-            dev::BackView v;
-            const dev::BpParams bp = make_bp_params(op.geometry(op.getPhysicalProjectionIndex(b, p)), vp, 1,
-                                                    m.lambda / (float)bs);
-            if (!dev::make_back_view(slab, bp, image(parity, p, 0), image(parity, p, 1), &v)) return;
-            back.push_back(v);
+            const dev::BpParams bp = make_bp_params(op.geometry(op.getPhysicalProjectionIndex(b, p)), vp,
+                                                    (uint32_t)m.bp_samples, m.lambda / (float)bs);
+            if (plain) {
+                dev::BackView v;
+                if (!dev::make_back_view(slab, bp, image(parity, p, 0), image(parity, p, 1), &v)) return;
+                back.push_back(v);
+            } else {
+                dev::SampleView v;
+                if (!dev::make_sample_view(slab, bp, image(parity, p, 0), image(parity, p, 1), &v)) return;
+                samples.push_back(v);
+            }
         }
         blocks.push_back(std::move(block));
     }
     blocks.push_back({back_first, back_count, {}});
-    const dev::SweepGroups groups = dev::sweep_groups(slab, back.data(), (int)back.size(), (uint32_t)m.nv, rows);
-    if (groups.count == 0) return;
-    split_back_.allocate(sizeof(dev::BackView) * back.size());
+    if (plain) {
+        split_groups_ = dev::sweep_groups(slab, back.data(), (int)back.size(), (uint32_t)m.nv, rows);
+        if (split_groups_.count == 0) return;
+    }
+    const size_t back_bytes = plain ? sizeof(dev::BackView) * back.size() : sizeof(dev::SampleView) * samples.size();
+    split_back_.allocate(back_bytes);
     split_forward_.allocate(sizeof(dev::ForwardView) * forward.size());
-    ETN_HIP(hipMemcpyAsync(split_back_.get(), back.data(), split_back_.bytes(), hipMemcpyHostToDevice, stream));
+    ETN_HIP(hipMemcpyAsync(split_back_.get(), plain ? (const void*)back.data() : (const void*)samples.data(), back_bytes,
+                           hipMemcpyHostToDevice, stream));
     ETN_HIP(hipMemcpyAsync(split_forward_.get(), forward.data(), split_forward_.bytes(), hipMemcpyHostToDevice, stream));
     ETN_HIP(hipStreamSynchronize(stream));
     split_slab_ = slab;
-    split_groups_ = groups;
     split_ = std::move(blocks);
 }
 
@@ -676,11 +701,15 @@ void FusedEngineImpl::enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* 
     for (size_t k = 0; k < split_.size(); ++k) {
         const SplitBlock& b = split_[k];
         if (ev) ETN_HIP(hipEventRecord((*ev)[2 * k], stream));
-        dev::sweep_back_project(split_slab_, split_groups_, split_back_.as<dev::BackView>() + b.back_first, b.back_count,
-                                (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
+        if (!over_ && !m.mask)
+            dev::sweep_back_project(split_slab_, split_groups_, split_back_.as<dev::BackView>() + b.back_first,
+                                    b.back_count, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
+        else
+            dev::sweep_samples_project(split_slab_, split_back_.as<dev::SampleView>() + b.back_first, b.back_count,
+                                       m.rowsets, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, m.mask, stream);
         for (const ForwardSweep& f : b.forward)
             dev::sweep_forward_project(split_slab_, split_forward_.as<dev::ForwardView>() + f.first, f.count, f.zdir,
-                                       (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
+                                       (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, vt_, volume, m.mask, stream);
         if (ev) ETN_HIP(hipEventRecord((*ev)[2 * k + 1], stream));
     }
 }

@@ -92,13 +92,29 @@ struct ForwardView {
 };
 constexpr int kSweepForward = 8;    // projections of a sweep
 // Whether sweep_forward_project takes a projection (a plane per detector row,
-// the same steps in every row, rays below the 2048-step limit).
-bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, uint32_t nv);
+// the same steps in every row, rays below the 2048-step limit); sub: sub-rays
+// along each pixel axis.
+bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, uint32_t nv, int sub, bool masked);
 // Forward-projects n <= kSweepForward views (device memory) whose rays move in
 // the z direction zdir (or stay in z) in one sweep of the volume, with the fused
-// kernels' fast arithmetic, operation for operation.
+// kernels' fast arithmetic, operation for operation.  mask: prior-knowledge mask
+// or null.
 void sweep_forward_project(const SlabParams& s, const ForwardView* views, int n, int zdir, uint32_t nu, uint32_t nv,
-                           etn_voxel_type vt, const void* volume, hipStream_t stream);
+                           int sub, etn_voxel_type vt, const void* volume, const uint8_t* mask, hipStream_t stream);
+// One back projection of sweep_samples_project (device table entries): a
+// per_dir x per_dir sample pattern, sx, sz, sw the offsets and in-voxel chords
+// along a pattern row, sy the rows' offsets.
+struct SampleView {
+    float m0, m8, m12, m5, m13, lambda;
+    float sx[4], sz[4], sw[4], sy[4];
+    const float* residual;
+    const float* length;
+};
+bool make_sample_view(const SlabParams& s, const BpParams& b, const float* residual, const float* length, SampleView* out);
+// Back-projects views[0 .. n) (device memory) in order, with a sample pattern, a
+// mask or both, rounding to the storage type after each.
+void sweep_samples_project(const SlabParams& s, const SampleView* views, int n, int per_dir, uint32_t nu, uint32_t nv,
+                           etn_voxel_type vt, void* volume, const uint8_t* mask, hipStream_t stream);
 void launch_compare(uint32_t n, const float* real, const float* virt, float* residual, hipStream_t stream);
 // real in its storage type (measured projections stored as f16 or bf16)
 void launch_compare(uint32_t n, const void* real, etn_voxel_type real_type, const float* virt, float* residual,

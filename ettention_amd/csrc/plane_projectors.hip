@@ -297,7 +297,8 @@ void launch_forward_typed(const SlabParams& s, const RayParams& r, const void* v
 }
 
 // Whether a geometry's rows lie in planes and take the same steps in each.
-bool plane_geometry_fits(const SlabParams& s, const RayParams& r)
+// (sub: the rows are sub-ray rows, so many a pixel)
+bool plane_geometry_fits(const SlabParams& s, const RayParams& r, int sub = 1)
 {
     if (r.nu == 0 || r.nv == 0 || s.res[0] > kFpLds) return false;
     if (r.ray[1] != 0.0f || r.h[1] != 0.0f || r.v[0] != 0.0f || r.v[2] != 0.0f) return false;
@@ -315,8 +316,9 @@ bool plane_geometry_fits(const SlabParams& s, const RayParams& r)
     }
     if (!(size > 0.5f)) return false;   // (a unit vector without y) the larger of x and z bounds the times
     const float inv = -FLT_MAX;
-    for (uint32_t y = 0; y < r.nv; ++y) {
-        const float fy = (float)y + 0.5f + 1.0f * 0.0f;
+    const float sd = 1.0f / (float)sub, off = sd / 2.0f;
+    for (uint32_t y = 0; y < r.nv * (uint32_t)sub; ++y) {
+        const float fy = (float)(y / sub) + off + sd * (float)(y % sub);
         const float rv = r.v[1] * fy;
         const float src = r.source[1] + 0.0f + rv;
         const float t0 = (s.bmin[1] - src) * inv, t1 = (s.bmax[1] - src) * inv;
@@ -695,28 +697,52 @@ __global__ void __launch_bounds__(kSweepThreads, 3)
 // ---- forward projections of several projections in one sweep -----------------------
 // plane_forward_kernel for up to kSweepForward projections of one z direction, P
 // rows a workgroup, with fused multiply-adds (the fused kernels' fast arithmetic)
-// and the residual written.  A thread traces up to eight rays, (projection,
-// column) pairs, each through the P planes at once: 11 instructions a step for
-// the path and 1 for each plane's sum, where a ray a plane takes 12.  Where the
-// rows make too few workgroups, the projections of a sweep are spread over
-// several of them, which read the same planes on the same XCD.  512 x 512 x 256,
-// eight projections: 0.17 ms, of which the steps' VALU issue is 0.09.
-constexpr int kMaxSweepRays = 8;
+// and the residual written.  A thread traces up to eight ray columns, (projection,
+// column, sub-ray column) triples, each through the P planes at once: 11
+// instructions a step for the path and 1 for each plane's sum, where a ray a
+// plane takes 12.  kMask: the ray length sums the voxels' mask weights, staged
+// behind the P values of a voxel.  The columns are spread over several
+// workgroups (slices), which read the same planes on the same XCD.  512 x 512 x
+// 256, eight projections: 0.17 ms, of which the steps' VALU issue is 0.09; 250 x
+// 300 x 150 bf16 with a mask and 4 x 4 sub-rays: 0.042 ms (0.055 with an index
+// division for every staged voxel; reads of four steps in flight gained nothing).
+template <bool kMask, int P>
+struct SweepRay {
+    float rx, rz, stepx, stepz;
+    int at, left, dx, dz;
+    float acc[P], len[kMask ? P : 1];
+};
 
-template <typename S, bool kVec, int P, int R>
+struct SweepForward {
+    const ForwardView* views;
+    int n, zdir, nu, nv;
+    int sub, shift;      // sub-rays a pixel axis, log2 of the ray columns a pixel
+    const uint8_t* mask;
+    int band, groups;
+};
+
+template <typename S, bool kVec, bool kMask, int P, int R>
 __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
-    sweep_forward_kernel(SlabParams s, const ForwardView* __restrict__ views, int n, int per, int zdir, int nu, int nv,
-                         const typename S::T* vol, int band, int groups)
+    sweep_forward_kernel(SlabParams s, SweepForward a, const typename S::T* vol)
 {
     using Q = Quad<S>;
-    using L = Lanes<P>;
+    constexpr int W = kMask ? 2 * P : P;     // floats a voxel
+    using L = Lanes<W>;
+    constexpr int T = kFpThreads;
     __shared__ __attribute__((aligned(16))) float lds[kFpLds];
+    __shared__ float weights[kMask ? 256 : 1];
     const int tid = threadIdx.x;
-    const int group = blockIdx.x % groups, q0 = blockIdx.x / groups * per, nq = min(per, n - q0);
-    views += q0;
+    const int group = blockIdx.x % a.groups, slice0 = blockIdx.x / a.groups * (R * T);
+    const ForwardView* __restrict__ views = a.views;
+    const int nu = a.nu, nv = a.nv, zdir = a.zdir, band = a.band;
     const int row0 = group * P, rows = min(P, nv - row0);
     const int nx = s.res[0], nz = s.res[2];
-    const int chunks = (nu + kFpThreads - 1) / kFpThreads;   // rays of a thread and projection
+    const int columns = nu << a.shift;       // ray columns of a projection
+    const float sd = 1.0f / (float)a.sub, off = sd / 2.0f;
+    if constexpr (kMask) {
+        for (int i = tid; i < 256; i += T) weights[i] = (float)i / 255.0f;
+        __syncthreads();
+    }
     // the planes of the rows, the same for every projection (checked on the host)
     int plane[P];
     bool hit[P];
@@ -724,8 +750,8 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const ForwardView& f = views[0];
-        const float fy = (float)min(row0 + p, nv - 1) + 0.5f;
-        const float ru = f.h[1] * 0.5f, rv = f.v[1] * fy;
+        const float fy = (float)min(row0 + p, nv - 1) + off;
+        const float ru = f.h[1] * off, rv = f.v[1] * fy;
         const float src = f.source[1] + ru + rv;
         const float t0 = (s.bmin[1] - src) * -FLT_MAX, t1 = (s.bmax[1] - src) * -FLT_MAX;
         hit[p] = p < rows && fminf(t0, t1) < 0.0f && fmaxf(t0, t1) > 0.0f;
@@ -734,31 +760,41 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
         any = any || hit[p];
     }
 
-    ColumnRay<P> ray[R];
+    // ray column of slot r: false where there is none
+    auto column = [&](int r, int& q, int& u, int& si) {
+        const int id = slice0 + r * T + tid;
+        q = id / columns;
+        const int rem = id - q * columns;
+        u = rem >> a.shift;
+        si = rem & ((1 << a.shift) - 1);
+        return q < a.n && si < a.sub;
+    };
+    SweepRay<kMask, P> ray[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int q = r / chunks, u = (r - q * chunks) * kFpThreads + tid;
-        ColumnRay<P>& y = ray[r];
+        SweepRay<kMask, P>& y = ray[r];
         y.left = 0;
         y.at = 0;
         y.rx = y.rz = y.stepx = y.stepz = 0.0f;
         y.dx = y.dz = 0;
-        y.len = 0.0f;
 #pragma unroll
         for (int p = 0; p < P; ++p) y.acc[p] = 0.0f;
-        if (any && q < nq && u < nu) {
+#pragma unroll
+        for (int p = 0; p < (kMask ? P : 1); ++p) y.len[p] = 0.0f;
+        int q, u, si;
+        if (column(r, q, u, si) && any) {
             const ForwardView& f = views[q];
             RayParams g;
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                g.source[a] = f.source[a];
-                g.h[a] = f.h[a];
-                g.v[a] = f.v[a];
-                g.ray[a] = f.ray[a];
+            for (int k = 0; k < 3; ++k) {
+                g.source[k] = f.source[k];
+                g.h[k] = f.h[k];
+                g.v[k] = f.v[k];
+                g.ray[k] = f.ray[k];
             }
             const DdaConst c = dda_const(g.ray, s.vs);
             float src[3];
-            fp_ray_source(g, (uint32_t)u, (uint32_t)row0, 0, 0, 1.0f, 0.5f, src);
+            fp_ray_source(g, (uint32_t)u, (uint32_t)row0, (uint32_t)si, 0, sd, off, src);
             SlabParams flat = s;
             src[1] = 0.0f;
             flat.bmin[1] = -1.0f;
@@ -769,34 +805,63 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
             y.rz = d.res[2];
             y.stepx = c.step[0];
             y.stepz = c.step[2];
-            y.at = (d.vox[2] * nx + d.vox[0]) * P * 4;
+            y.at = (d.vox[2] * nx + d.vox[0]) * W * 4;
             y.left = !d.live ? 0 : c.sign[0] > 0 ? nx - d.vox[0] : c.sign[0] < 0 ? d.vox[0] + 1 : 0x7fffffff;
-            y.dx = c.sign[0] * P * 4;
-            y.dz = c.sign[2] * nx * P * 4;
+            y.dx = c.sign[0] * W * 4;
+            y.dz = c.sign[2] * nx * W * 4;
         }
     }
 
     if (any) {
         const size_t slice = (size_t)s.nx * s.ny;
         const typename S::T* base[P];
+        const uint8_t* mbase[P];
 #pragma unroll
-        for (int p = 0; p < P; ++p) base[p] = vol + s.first_voxel + (size_t)plane[p] * s.nx;
-        const int bands = (nz + band - 1) / band, quads = nx / 4;
-        constexpr int kItems = kVec ? kFpLds / (4 * P * kFpThreads) : 1;
-        typename Q::V pre[kItems][P];
+        for (int p = 0; p < P; ++p) {
+            base[p] = vol + s.first_voxel + (size_t)plane[p] * s.nx;
+            if constexpr (kMask) mbase[p] = a.mask + s.first_voxel + (size_t)plane[p] * s.nx;
+        }
+        const int bands = (nz + band - 1) / band;
+        // items of G voxels in x, P planes each: the next band's are in flight
+        // while the rays cross this one
+        constexpr int G = kVec ? 4 : 1, kItems = kFpLds / (G * W * T);
+        const int items_x = nx / G;
+        typename std::conditional<kVec, typename Q::V, typename S::T>::type pre[kItems][P];
+        typename std::conditional<kVec, uint32_t, uint8_t>::type mpre[kMask ? kItems : 1][P];
         auto range = [&](int b, int& z0, int& z1) {
             z0 = (zdir >= 0 ? b : bands - 1 - b) * band;
             z1 = min(z0 + band, nz);
         };
+        // item k T + tid of a band: its offset follows from the one before it (a
+        // band's offsets fit 32 bits: the host checks it)
+        const int first_z = tid / items_x, first_x = tid - first_z * items_x;
+        const uint32_t offset0 = (uint32_t)first_z * (uint32_t)slice + (uint32_t)(first_x * G);
+        const int next_x = T % items_x;
+        const uint32_t next = (uint32_t)(T / items_x) * (uint32_t)slice + (uint32_t)(next_x * G);
+        const uint32_t wrap = (uint32_t)slice - (uint32_t)nx;
         auto load = [&](int z0, int z1) {
-            if constexpr (kVec) {
-                const int m = (z1 - z0) * quads;
+            const uint32_t last = (uint32_t)(z1 - z0 - 1) * (uint32_t)slice + (uint32_t)(nx - G);
+            uint32_t offset = offset0;
+            int x = first_x;
 #pragma unroll
-                for (int k = 0; k < kItems; ++k) {
-                    const int i = min(k * kFpThreads + tid, m - 1), z = i / quads, x = (i - z * quads) * 4;
+            for (int k = 0; k < kItems; ++k) {
+                const uint32_t at = min(offset, last);   // (beyond the band: read again, not used)
 #pragma unroll
-                    for (int p = 0; p < P; ++p)
-                        pre[k][p] = *reinterpret_cast<const typename Q::V*>(base[p] + (size_t)(z0 + z) * slice + x);
+                for (int p = 0; p < P; ++p) {
+                    const typename S::T* from = base[p] + (size_t)z0 * slice;
+                    if constexpr (kVec) pre[k][p] = *reinterpret_cast<const typename Q::V*>(from + at);
+                    else pre[k][p] = from[at];
+                    if constexpr (kMask) {
+                        const uint8_t* mfrom = mbase[p] + (size_t)z0 * slice;
+                        if constexpr (kVec) mpre[k][p] = *reinterpret_cast<const uint32_t*>(mfrom + at);
+                        else mpre[k][p] = mfrom[at];
+                    }
+                }
+                x += next_x;
+                offset += next;
+                if (x >= items_x) {
+                    x -= items_x;
+                    offset += wrap;
                 }
             }
         };
@@ -805,25 +870,31 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
         load(z0, z1);
         for (int b = 0; b < bands; ++b) {
             range(b, z0, z1);
-            if constexpr (kVec) {
-                const int m = (z1 - z0) * quads;
+            const int m = (z1 - z0) * items_x;
 #pragma unroll
-                for (int k = 0; k < kItems; ++k) {
-                    const int i = k * kFpThreads + tid;
-                    if (i < m) {
-                        float v[P][4];
+            for (int k = 0; k < kItems; ++k) {
+                const int i = k * T + tid;
+                if (i < m) {
+                    if constexpr (kVec) {
+                        float v[W][4];
 #pragma unroll
-                        for (int p = 0; p < P; ++p) Q::unpack(pre[k][p], v[p]);
-                        interleave<P>(v, reinterpret_cast<f32x4*>(lds) + (size_t)i * P);
+                        for (int p = 0; p < P; ++p) {
+                            Q::unpack(pre[k][p], v[p]);
+                            if constexpr (kMask)
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) v[P + p][j] = weights[mpre[k][p] >> (8 * j) & 255u];
+                        }
+                        interleave<W>(v, reinterpret_cast<f32x4*>(lds) + (size_t)i * W);
+                    } else {
+                        typename L::V cell;
+                        float* to = reinterpret_cast<float*>(&cell);
+#pragma unroll
+                        for (int p = 0; p < P; ++p) {
+                            to[p] = S::load(&pre[k][p], 0);
+                            if constexpr (kMask) to[P + p] = weights[mpre[k][p]];
+                        }
+                        reinterpret_cast<typename L::V*>(lds)[i] = cell;
                     }
-                }
-            } else {
-                const int m = (z1 - z0) * nx;
-#pragma unroll 4
-                for (int i = tid; i < m; i += kFpThreads) {
-                    const int z = i / nx, x = i - z * nx;
-#pragma unroll
-                    for (int p = 0; p < P; ++p) lds[i * P + p] = S::load(base[p], (size_t)(z0 + z) * slice + x);
                 }
             }
             if (b + 1 < bands) {
@@ -832,12 +903,12 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
                 load(n0, n1);
             }
             __syncthreads();
-            const unsigned bytes = (unsigned)((z1 - z0) * nx * P) * 4u;
-            const int start = z0 * nx * P * 4;
+            const unsigned bytes = (unsigned)((z1 - z0) * nx * W) * 4u;
+            const int start = z0 * nx * W * 4;
             const char* rows_at = reinterpret_cast<const char*>(lds);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                ColumnRay<P>& y = ray[r];
+                SweepRay<kMask, P>& y = ray[r];
                 int at = y.at - start, left = y.left;
                 float rx = y.rx, rz = y.rz;
                 while (left != 0 && (unsigned)at < bytes) {
@@ -850,7 +921,12 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
                     left -= ix ? 1 : 0;
 #pragma unroll
                     for (int p = 0; p < P; ++p) y.acc[p] = fmaf(dt, L::get(v, p), y.acc[p]);
-                    y.len += dt;
+                    if constexpr (kMask) {
+#pragma unroll
+                        for (int p = 0; p < P; ++p) y.len[p] = fmaf(dt, L::get(v, P + p), y.len[p]);
+                    } else {
+                        y.len[0] += dt;
+                    }
                 }
                 y.at = at + start;
                 y.left = left;
@@ -863,14 +939,26 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
 
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int q = r / chunks, u = (r - q * chunks) * kFpThreads + tid;
-        if (q >= nq || u >= nu) continue;
-        const ForwardView& f = views[q];
+        int q, u, si;
+        const bool mine = column(r, q, u, si) && si == 0;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            if (p >= rows) continue;
+            // the pixel's sub-rays in the fused kernels' order: those of a column
+            // differ only in y and have equal sums
+            float acc = 0.0f, len = 0.0f;
+            const float ra = hit[p] ? ray[r].acc[p] : 0.0f, rl = hit[p] ? ray[r].len[kMask ? p : 0] : 0.0f;
+            for (int k = 0; k < a.sub; ++k) {
+                const float ka = a.sub > 1 ? __shfl_down(ra, k) : ra, kl = a.sub > 1 ? __shfl_down(rl, k) : rl;
+                for (int j = 0; j < a.sub; ++j) {
+                    acc += ka;
+                    len += kl;
+                }
+            }
+            if (!mine || p >= rows) continue;
+            const ForwardView& f = views[q];
             const size_t i = (size_t)(row0 + p) * nu + u;
-            float pv = 0.0f + (hit[p] ? ray[r].acc[p] : 0.0f) / 1.0f, l = 0.0f + (hit[p] ? ray[r].len : 0.0f) / 1.0f;
+            const float total = (float)(a.sub * a.sub);
+            float pv = 0.0f + acc / total, l = 0.0f + len / total;
             if (f.use_loc) {
                 pv = l > kEpsilon ? pv * f.loc_c / l : 0.0f;
                 l = f.loc_c;
@@ -885,44 +973,259 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
     }
 }
 
-template <typename S, bool kVec, int P>
-void launch_sweep_forward(const SlabParams& s, const ForwardView* views, int n, int zdir, int nu, int nv,
-                          const void* volume, hipStream_t stream)
+template <typename S, bool kVec, bool kMask, int P>
+void launch_sweep_forward(const SlabParams& s, SweepForward a, const void* volume, hipStream_t stream)
 {
+    constexpr int T = kFpThreads;
     const auto* vol = static_cast<const typename S::T*>(volume);
-    const int groups = (nv + P - 1) / P, chunks = (nu + kFpThreads - 1) / kFpThreads;
-    // projections a workgroup: as many as its rays hold, fewer where that
-    // leaves a CU fewer than two workgroups (512 x 512 x 256, eight
-    // projections: 167 us a sweep with two a CU, 175 with one)
-    int per = std::max(1, std::min(n, kMaxSweepRays / chunks));
-    while (per > 1 && groups * ((n + per - 1) / per) < 512) per = (per + 1) / 2;
-    const int band = std::max(1, std::min(s.res[2], kFpLds / (s.res[0] * P)));
-    const unsigned grid = (unsigned)(groups * ((n + per - 1) / per));
-    const int rays = per * chunks;
-    auto launch = [&](auto kernel) { kernel<<<grid, kFpThreads, 0, stream>>>(s, views, n, per, zdir, nu, nv, vol, band, groups); };
-    if (rays <= 1) launch(sweep_forward_kernel<S, kVec, P, 1>);
-    else if (rays <= 2) launch(sweep_forward_kernel<S, kVec, P, 2>);
-    else if (rays <= 4) launch(sweep_forward_kernel<S, kVec, P, 4>);
-    else launch(sweep_forward_kernel<S, kVec, P, 8>);
+    const int columns = a.n * (a.nu << a.shift);
+    a.groups = (a.nv + P - 1) / P;
+    // columns a thread: as many as there are, fewer where that leaves a CU fewer
+    // than two workgroups (512 x 512 x 256, eight projections: 167 us a sweep
+    // with two a CU, 175 with one)
+    int rays = 8;
+    while (rays > 1 && (rays / 2 * T >= columns || a.groups * ((columns + rays * T - 1) / (rays * T)) < 512)) rays /= 2;
+    a.band = std::max(1, std::min(s.res[2], kFpLds / (s.res[0] * P * (kMask ? 2 : 1))));
+    const unsigned grid = (unsigned)(a.groups * ((columns + rays * T - 1) / (rays * T)));
+    auto launch = [&](auto kernel) { kernel<<<grid, T, 0, stream>>>(s, a, vol); };
+    if (rays == 1) launch(sweep_forward_kernel<S, kVec, kMask, P, 1>);
+    else if (rays == 2) launch(sweep_forward_kernel<S, kVec, kMask, P, 2>);
+    else if (rays == 4) launch(sweep_forward_kernel<S, kVec, kMask, P, 4>);
+    else launch(sweep_forward_kernel<S, kVec, kMask, P, 8>);
 }
 
-template <typename S>
-void sweep_forward_typed(const SlabParams& s, const ForwardView* views, int n, int zdir, int nu, int nv,
-                         const void* volume, hipStream_t stream)
+template <typename S, bool kMask>
+void sweep_forward_typed(const SlabParams& s, const SweepForward& a, const void* volume, hipStream_t stream)
 {
-    const int nx = s.res[0];
-    const bool vec = nx % 4 == 0 && reinterpret_cast<uintptr_t>(volume) % (4 * sizeof(typename S::T)) == 0;
-    // planes a workgroup: four where they and the projections still make a
-    // workgroup for every CU (two planes: 240 us), fewer on small volumes
-    const int P = nx * 4 <= kFpLds && (nv + 3) / 4 * n >= 256 ? 4 : nx * 2 <= kFpLds && (nv + 1) / 2 * n >= 256 ? 2 : 1;
+    const int nx = s.res[0], w = kMask ? 2 : 1;
+    const bool vec = nx % 4 == 0 && reinterpret_cast<uintptr_t>(volume) % (4 * sizeof(typename S::T)) == 0 &&
+                     reinterpret_cast<uintptr_t>(a.mask) % 4 == 0;
+    // planes a workgroup: four where they and the columns still make a
+    // workgroup for every CU (two planes: 240 us), fewer on small volumes; a
+    // voxel's values and weights are one 16-byte read
+    auto fills = [&](int P) {
+        const int columns = a.n * (a.nu << a.shift);
+        return nx * P * w <= kFpLds &&
+               (a.nv + P - 1) / P * ((columns + kFpThreads - 1) / kFpThreads) >= 256;
+    };
+    const int P = !kMask && fills(4) ? 4 : fills(2) ? 2 : 1;
     auto launch = [&](auto v) {
         constexpr bool kVec = decltype(v)::value;
-        if (P == 4) launch_sweep_forward<S, kVec, 4>(s, views, n, zdir, nu, nv, volume, stream);
-        else if (P == 2) launch_sweep_forward<S, kVec, 2>(s, views, n, zdir, nu, nv, volume, stream);
-        else launch_sweep_forward<S, kVec, 1>(s, views, n, zdir, nu, nv, volume, stream);
+        if constexpr (!kMask) {
+            if (P == 4) return launch_sweep_forward<S, kVec, kMask, 4>(s, a, volume, stream);
+        }
+        if (P == 2) launch_sweep_forward<S, kVec, kMask, 2>(s, a, volume, stream);
+        else launch_sweep_forward<S, kVec, kMask, 1>(s, a, volume, stream);
     };
     if (vec) launch(std::true_type{});
     else launch(std::false_type{});
+}
+
+// ---- oversampled back projections in one sweep ------------------------------------
+// The per_dir x per_dir sample pattern (PD = per_dir) with the fused kernels' fast
+// lookups.  A sample's u does not depend on its pattern row, which only moves it
+// along y, nor on the plane: the PD samples of a pattern row give u, column and
+// weight for all PD rows of all four planes, so a sample costs its record read
+// and 11 instruction slots (19 on the fused kernels, which also leave CUs idle
+// where the planes are no multiple of them).  A workgroup owns four planes x 64
+// columns x 4 kSampleDepth slices in registers.  250 x 300 x 150 bf16 with a mask,
+// 3 x 3 samples: 0.052 ms, with the forward sweep 0.094 where a fused pass takes
+// 0.25; eight slices a wave 0.07 (fewer workgroups).
+constexpr int kSampleDepth = 4;      // slices a wave
+
+template <typename S, int PD>
+__global__ void __launch_bounds__(kSweepThreads, 4)
+    sweep_samples_kernel(SlabParams s, const SampleView* __restrict__ views, int n, typename S::T* vol,
+                         const uint8_t* __restrict__ mask, int nu, int nv)
+{
+    __shared__ f32x4 recs[kSweepPlanes * PD][kSweepColumns];
+    __shared__ float weights[256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int x0 = blockIdx.x * kSweepTile, y0 = blockIdx.y * kSweepPlanes, z0 = blockIdx.z * (4 * kSampleDepth);
+    const int x = x0 + lane, zw = z0 + wave * kSampleDepth;
+    const int planes = min(kSweepPlanes, s.res[1] - y0);
+    const bool xin = x < s.res[0];
+    const size_t slice = (size_t)s.nx * s.ny;
+    const size_t at0 = s.first_voxel + (size_t)zw * slice + (size_t)y0 * s.nx + (size_t)(uint32_t)x;
+    weights[tid] = (float)tid / 255.0f;
+
+    // (addresses are clamped into the volume: nothing waits for a single load)
+    float value[kSampleDepth][kSweepPlanes];
+    uint32_t mv[kSampleDepth];
+    auto clamped = [&](int j, int p) {
+        return s.first_voxel + (size_t)min(zw + j, s.res[2] - 1) * slice + (size_t)(y0 + min(p, planes - 1)) * s.nx +
+               (size_t)min(x, s.res[0] - 1);
+    };
+#pragma unroll
+    for (int j = 0; j < kSampleDepth; ++j)
+#pragma unroll
+        for (int p = 0; p < kSweepPlanes; ++p) value[j][p] = S::load(vol, clamped(j, p));
+    if (mask) {
+        uint32_t in[kSampleDepth][kSweepPlanes];
+#pragma unroll
+        for (int j = 0; j < kSampleDepth; ++j)
+#pragma unroll
+            for (int p = 0; p < kSweepPlanes; ++p) in[j][p] = mask[clamped(j, p)];
+#pragma unroll
+        for (int j = 0; j < kSampleDepth; ++j) mv[j] = in[j][0] | in[j][1] << 8 | in[j][2] << 16 | in[j][3] << 24;
+    } else {
+#pragma unroll
+        for (int j = 0; j < kSampleDepth; ++j) mv[j] = 0xffffffffu;
+    }
+    const float xc = s.bmin[0] + ((float)x + 0.5f) * s.vs[0];
+    // the tile's corners
+    const float cxa = s.bmin[0] + ((float)x0 + 0.5f) * s.vs[0], cxb = s.bmin[0] + ((float)(x0 + kSweepTile - 1) + 0.5f) * s.vs[0];
+    const float cza = s.bmin[2] + ((float)z0 + 0.5f) * s.vs[2];
+    const float czb = s.bmin[2] + ((float)(z0 + 4 * kSampleDepth - 1) + 0.5f) * s.vs[2];
+
+    for (int q = 0; q < n; ++q) {
+        const SampleView& v = views[q];
+        const float m0 = v.m0, m8 = v.m8, m12 = v.m12;
+        // the tile's smallest u, less one for its rounding
+        float sxa = v.sx[0], sxb = v.sx[0], sza = v.sz[0], szb = v.sz[0];
+#pragma unroll
+        for (int i = 1; i < PD; ++i) {
+            sxa = fminf(sxa, v.sx[i]);
+            sxb = fmaxf(sxb, v.sx[i]);
+            sza = fminf(sza, v.sz[i]);
+            szb = fmaxf(szb, v.sz[i]);
+        }
+        const float umin = (m0 >= 0.0f ? m0 * (cxa + sxa) : m0 * (cxb + sxb)) +
+                           (m8 >= 0.0f ? m8 * (cza + sza) : m8 * (czb + szb)) + m12 - 0.5f;
+        const int first = (int)floorf(umin) - 1;
+        __syncthreads();
+        // records {A, B, LA, LB} of a plane's pattern rows: R = A + B tx, L = LA + LB
+        // tx.  Thread (h, k) takes column k of rows h, h + 2, ...; the loads of PD of
+        // them are in flight together (clamped into the images, what lies outside
+        // zeroed afterwards)
+        const int k = tid % kSweepColumns, h = tid / kSweepColumns, u0 = first + k;
+        const bool c0 = (unsigned)u0 < (unsigned)nu, c1 = (unsigned)(u0 + 1) < (unsigned)nu;
+        const uint32_t k0 = (uint32_t)min(max(u0, 0), nu - 1), k1 = (uint32_t)min(max(u0 + 1, 0), nu - 1);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            float in[PD][8], ty[PD];
+            int r0[PD];
+#pragma unroll
+            for (int e = 0; e < PD; ++e) {
+                const int row = (half * PD + e) * 2 + h, p = row / PD;
+                const float py = s.bmin[1] + ((float)(y0 + p) + 0.5f) * s.vs[1];
+                float vp = v.m5 * (py + v.sy[row - p * PD]);
+                vp = vp + v.m13 * 1.0f;
+                float base_row;
+                ty[e] = cl_fract(vp - 0.5f, &base_row);
+                r0[e] = __builtin_amdgcn_readfirstlane((int)base_row);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const size_t at = (size_t)min(max(r0[e] + i, 0), nv - 1) * nu;
+                    in[e][2 * i] = (v.residual + at)[k0];
+                    in[e][2 * i + 1] = (v.residual + at)[k1];
+                    in[e][4 + 2 * i] = (v.length + at)[k0];
+                    in[e][5 + 2 * i] = (v.length + at)[k1];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < PD; ++e) {
+                float w[8];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const bool rin = (unsigned)(r0[e] + (t >> 1 & 1)) < (unsigned)nv;
+                    w[t] = (rin & (t & 1 ? c1 : c0)) ? in[e][t] : 0.0f;
+                }
+                const float dr0 = w[1] - w[0], dr1 = w[3] - w[2], dl0 = w[5] - w[4], dl1 = w[7] - w[6];
+                recs[(half * PD + e) * 2 + h][k] = f32x4{fmaf(w[2] - w[0], ty[e], w[0]), fmaf(dr1 - dr0, ty[e], dr0),
+                                                         fmaf(w[6] - w[4], ty[e], w[4]), fmaf(dl1 - dl0, ty[e], dl0)};
+            }
+        }
+        __syncthreads();
+        const f32x4* rec = recs[0] - first;
+#pragma unroll
+        for (int j = 0; j < kSampleDepth; ++j) {
+            const float zc = s.bmin[2] + ((float)(zw + j) + 0.5f) * s.vs[2];
+            float sum[kSweepPlanes];
+            int used[kSweepPlanes], full = 0;
+#pragma unroll
+            for (int p = 0; p < kSweepPlanes; ++p) {
+                sum[p] = 0.0f;
+                used[p] = 0;
+            }
+#pragma unroll 1
+            for (int i = 0; i < PD; ++i) {
+                float u = m0 * (xc + v.sx[i]) + 0.0f;
+                u = u + m8 * (zc + v.sz[i]);
+                u = u + m12 * 1.0f;
+                u = u - 0.5f;
+                const float tx = __builtin_amdgcn_fractf(u);
+                int column;
+                asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(column) : "v"(u));
+                const f32x4* c = rec + column;
+                const float lw = v.lambda * v.sw[i];
+                // the common case, every record with rays through it, decided for
+                // the whole wave: no test, count or select a sample
+                float R[PD][kSweepPlanes], L[PD][kSweepPlanes], least = FLT_MAX;
+#pragma unroll
+                for (int ys = 0; ys < PD; ++ys)
+#pragma unroll
+                    for (int p = 0; p < kSweepPlanes; ++p) {
+                        const f32x4 e = c[(p * PD + ys) * kSweepColumns];
+                        R[ys][p] = fmaf(e[1], tx, e[0]);
+                        L[ys][p] = fmaf(e[3], tx, e[2]);
+                        least = fminf(least, L[ys][p]);
+                    }
+                if (__all(least > kEpsilon)) {
+                    full += PD;
+#pragma unroll
+                    for (int p = 0; p < kSweepPlanes; ++p) {
+                        float part = 0.0f;
+#pragma unroll
+                        for (int ys = 0; ys < PD; ++ys) part = fmaf(R[ys][p], __builtin_amdgcn_rcpf(L[ys][p]), part);
+                        sum[p] = fmaf(part, lw, sum[p]);
+                    }
+                } else {
+#pragma unroll
+                    for (int p = 0; p < kSweepPlanes; ++p) {
+                        float part = 0.0f;
+#pragma unroll
+                        for (int ys = 0; ys < PD; ++ys) {
+                            const bool ok = L[ys][p] > kEpsilon;
+                            part = ok ? fmaf(R[ys][p], __builtin_amdgcn_rcpf(L[ys][p]), part) : part;
+                            used[p] += ok ? 1 : 0;
+                        }
+                        sum[p] = fmaf(part, lw, sum[p]);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int p = 0; p < kSweepPlanes; ++p) {
+                const int count = used[p] + full;
+                if (count != 0) value[j][p] += weights[mv[j] >> (8 * p) & 255u] * sum[p] / (float)count;
+            }
+            round_planes<S>(value[j]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kSampleDepth; ++j)
+#pragma unroll
+        for (int p = 0; p < kSweepPlanes; ++p)
+            if (zw + j < s.res[2] && p < planes && xin)
+                S::store(vol, at0 + (size_t)j * slice + (size_t)p * s.nx, value[j][p]);
+}
+
+template <typename S>
+void sweep_samples_typed(const SlabParams& s, const SampleView* views, int n, int per_dir, uint32_t nu, uint32_t nv,
+                         void* volume, const uint8_t* mask, hipStream_t stream)
+{
+    auto* vol = static_cast<typename S::T*>(volume);
+    const dim3 grid((s.res[0] + kSweepTile - 1) / kSweepTile, (s.res[1] + kSweepPlanes - 1) / kSweepPlanes,
+                    (s.res[2] + 4 * kSampleDepth - 1) / (4 * kSampleDepth));
+    auto launch = [&](auto kernel) {
+        kernel<<<grid, kSweepThreads, 0, stream>>>(s, views, n, vol, mask, (int)nu, (int)nv);
+    };
+    if (per_dir == 1) launch(sweep_samples_kernel<S, 1>);
+    else if (per_dir == 2) launch(sweep_samples_kernel<S, 2>);
+    else if (per_dir == 3) launch(sweep_samples_kernel<S, 3>);
+    else launch(sweep_samples_kernel<S, 4>);
 }
 
 }  // namespace
@@ -1025,7 +1328,7 @@ void sweep_back_project(const SlabParams& s, const SweepGroups& g, const BackVie
     hip_check(hipGetLastError(), "back projection sweep launch");
 }
 
-bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, uint32_t nv)
+bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, uint32_t nv, int sub, bool masked)
 {
     RayParams r{};
     for (int k = 0; k < 3; ++k) {
@@ -1037,18 +1340,72 @@ bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, u
     r.nu = nu;
     r.nv = nv;
     r.samples = 1;
-    return nu <= (uint32_t)(kMaxSweepRays * kFpThreads) && plane_geometry_fits(s, r);
+    if (sub < 1 || sub > 4 || nu > 1u << 20 || nv > 1u << 20 || s.res[1] > 65535) return false;
+    return s.res[0] * (masked ? 2 : 1) <= kFpLds && plane_geometry_fits(s, r, sub);
 }
 
 void sweep_forward_project(const SlabParams& s, const ForwardView* views, int n, int zdir, uint32_t nu, uint32_t nv,
-                           etn_voxel_type vt, const void* volume, hipStream_t stream)
+                           int sub, etn_voxel_type vt, const void* volume, const uint8_t* mask, hipStream_t stream)
 {
     if (n <= 0) return;
     if (n > kSweepForward) fail("forward projection sweep: at most eight projections");
-    if (vt == ETN_VOXEL_FLOAT16) sweep_forward_typed<F16>(s, views, n, zdir, (int)nu, (int)nv, volume, stream);
-    else if (vt == ETN_VOXEL_BFLOAT16) sweep_forward_typed<BF16>(s, views, n, zdir, (int)nu, (int)nv, volume, stream);
-    else sweep_forward_typed<F32>(s, views, n, zdir, (int)nu, (int)nv, volume, stream);
+    SweepForward a{};
+    a.views = views;
+    a.n = n;
+    a.zdir = zdir;
+    a.nu = (int)nu;
+    a.nv = (int)nv;
+    a.sub = sub;
+    while (1 << a.shift < sub) ++a.shift;
+    a.mask = mask;
+    auto launch = [&](auto type) {
+        using S = decltype(type);
+        if (mask) sweep_forward_typed<S, true>(s, a, volume, stream);
+        else sweep_forward_typed<S, false>(s, a, volume, stream);
+    };
+    if (vt == ETN_VOXEL_FLOAT16) launch(F16{});
+    else if (vt == ETN_VOXEL_BFLOAT16) launch(BF16{});
+    else launch(F32{});
     hip_check(hipGetLastError(), "forward projection sweep launch");
+}
+
+bool make_sample_view(const SlabParams& s, const BpParams& b, const float* residual, const float* length, SampleView* out)
+{
+    int pd = 1;
+    while (pd * pd < (int)b.nsamples) ++pd;
+    if (pd > 4 || pd * pd != (int)b.nsamples || !single_axis_matrix(s, b)) return false;
+    const float* m = b.m;
+    SampleView v{m[0], m[8], m[12], m[5], m[13], b.lambda, {}, {}, {}, {}, residual, length};
+    for (int t = 0; t < pd * pd; ++t) {
+        const float4 e = b.samples[t];
+        const int ys = t / pd, i = t - ys * pd;
+        if (i == 0) v.sy[ys] = e.y;
+        if (ys == 0) {
+            v.sx[i] = e.x;
+            v.sz[i] = e.z;
+            v.sw[i] = e.w;
+        }
+        // a pattern row only moves its samples along y
+        if (v.sy[ys] != e.y || v.sx[i] != e.x || v.sz[i] != e.z || v.sw[i] != e.w) return false;
+    }
+    const float spread = std::fabs(m[0]) * (*std::max_element(v.sx, v.sx + pd) - *std::min_element(v.sx, v.sx + pd)) +
+                         std::fabs(m[8]) * (*std::max_element(v.sz, v.sz + pd) - *std::min_element(v.sz, v.sz + pd));
+    const float columns = std::fabs(m[0]) * s.vs[0] * (float)(kSweepTile - 1) +
+                          std::fabs(m[8]) * s.vs[2] * (float)(4 * kSampleDepth - 1) + spread + 5.0f;
+    if (!(columns <= (float)kSweepColumns)) return false;
+    if ((s.res[1] + kSweepPlanes - 1) / kSweepPlanes > 65535 || s.res[2] / (4 * kSampleDepth) >= 65535) return false;
+    *out = v;
+    return true;
+}
+
+void sweep_samples_project(const SlabParams& s, const SampleView* views, int n, int per_dir, uint32_t nu, uint32_t nv,
+                           etn_voxel_type vt, void* volume, const uint8_t* mask, hipStream_t stream)
+{
+    if (n <= 0) return;
+    if (vt == ETN_VOXEL_FLOAT16) sweep_samples_typed<F16>(s, views, n, per_dir, nu, nv, volume, mask, stream);
+    else if (vt == ETN_VOXEL_BFLOAT16) sweep_samples_typed<BF16>(s, views, n, per_dir, nu, nv, volume, mask, stream);
+    else sweep_samples_typed<F32>(s, views, n, per_dir, nu, nv, volume, mask, stream);
+    hip_check(hipGetLastError(), "back projection sweep launch");
 }
 
 std::vector<uint8_t> row_classes(const SlabParams& s, const RayParams& r)

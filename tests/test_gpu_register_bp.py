@@ -150,8 +150,8 @@ def test_wbp_register_back_projection_equals_lds():
 # back projection: nx off a multiple of 4, rows beside the volume, one, two and
 # four planes a workgroup, several rays a thread, both z directions, more
 # projections in a block than in a sweep
-SWEEPS = [((61, 20, 33), 17, 4, 60.0, "float"), ((64, 70, 40), 23, 8, 60.0, "float"), ((64, 520, 12), 9, 3, 60.0, "float"),
-          ((520, 9, 16), 11, 8, 60.0, "bfloat16"), ((48, 33, 30), 40, 0, 60.0, "half"), ((40, 130, 24), 30, 5, 150.0, "float")]
+SWEEPS = [((135, 131, 120), 23, 8, 60.0, "float"), ((64, 522, 64), 9, 9, 60.0, "float"), ((300, 160, 180), 9, 4, 60.0, "float"),
+          ((520, 70, 64), 19, 8, 60.0, "bfloat16"), ((136, 130, 120), 40, 0, 60.0, "half"), ((130, 130, 128), 30, 12, 150.0, "float")]
 
 
 @pytest.mark.parametrize("shape,ntilts,block,reach,voxel", SWEEPS)
@@ -168,3 +168,31 @@ def test_block_sweeps_equal_the_fused_passes(shape, ntilts, block, reach, voxel,
     w, ref = run(case, flags=LDS)
     np.testing.assert_array_equal(v, w)
     assert norm == ref
+
+
+# sample patterns, sub-rays and masks in the sweeps.  They add a voxel's samples
+# in another order than the fused pass does: up to 16 terms of one rounding each,
+# so a relative 1e-6 of every update, below the 2e-5 that two reconstructions in
+# single precision may differ by; 16-bit storage rounds some voxels the other way
+# (half an ulp of the type at most, in the mean far less).
+@pytest.mark.parametrize("shape,ntilts,block,fp,bp,masked,voxel", [
+    ((90, 81, 77), 17, 0, 1, 1, True, "float"), ((88, 83, 76), 13, 8, 1, 1, True, "half"),
+    ((88, 81, 77), 9, 1, 2, 4, False, "float"), ((91, 82, 70), 9, 1, 4, 9, True, "float"),
+    ((92, 81, 72), 12, 4, 3, 16, True, "float"), ((88, 80, 79), 9, 1, 1, 9, True, "bfloat16")])
+def test_sampled_sweeps_match_the_fused_passes(shape, ntilts, block, fp, bp, masked, voxel):
+    nx, ny, nz = shape
+    rng = np.random.default_rng(ntilts)
+    case = dict(volume=E.VolumeGeometry.make(shape), base_geometry=E.ScannerGeometry.mrc_base(nx, ny),
+                tilt_angles=np.linspace(-60, 60, ntilts).astype(np.float32),
+                projections=torch.from_numpy(rng.normal(1.0, 0.3, (ntilts, ny, nx)).astype(np.float32)).cuda(),
+                algorithm="blockiterative" if block else "sirt", block_size=block, lam=0.3, voxel_type=voxel,
+                fp_samples=fp, bp_samples=bp)
+    if masked:
+        mask = rng.integers(0, 256, (nz, ny, nx)).astype(np.uint8)
+        mask[:, : ny // 3] = 0
+        case["mask"] = torch.from_numpy(mask).cuda()
+    v, norm = run(case)
+    w, ref = run(case, flags=LDS)
+    bound = 2e-5 if voxel == "float" else 1e-2
+    assert np.linalg.norm(v - w) <= bound * np.linalg.norm(w)
+    assert abs(norm - ref) <= bound * ref
