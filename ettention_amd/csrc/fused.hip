@@ -706,7 +706,7 @@ void FusedEngineImpl::enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* 
                                     b.back_count, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
         else
             dev::sweep_samples_project(split_slab_, split_back_.as<dev::SampleView>() + b.back_first, b.back_count,
-                                       m.rowsets, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, m.mask, stream);
+                                       m.rowsets, over_, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, m.mask, stream);
         for (const ForwardSweep& f : b.forward)
             dev::sweep_forward_project(split_slab_, split_forward_.as<dev::ForwardView>() + f.first, f.count, f.zdir,
                                        (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, vt_, volume, m.mask, stream);

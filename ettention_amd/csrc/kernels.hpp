@@ -111,10 +111,12 @@ struct SampleView {
     const float* length;
 };
 bool make_sample_view(const SlabParams& s, const BpParams& b, const float* residual, const float* length, SampleView* out);
-// Back-projects views[0 .. n) (device memory) in order, with a sample pattern, a
-// mask or both, rounding to the storage type after each.
-void sweep_samples_project(const SlabParams& s, const SampleView* views, int n, int per_dir, uint32_t nu, uint32_t nv,
-                           etn_voxel_type vt, void* volume, const uint8_t* mask, hipStream_t stream);
+// Back-projects views[0 .. n) (device memory) in order with the fused kernels' fast
+// arithmetic, operation for operation, rounding to the storage type after each.
+// over: their oversampled kernels' sample loop (forward or back projections
+// oversampled; mask or null), else (per_dir 1) their masked single-sample update.
+void sweep_samples_project(const SlabParams& s, const SampleView* views, int n, int per_dir, bool over, uint32_t nu,
+                           uint32_t nv, etn_voxel_type vt, void* volume, const uint8_t* mask, hipStream_t stream);
 void launch_compare(uint32_t n, const float* real, const float* virt, float* residual, hipStream_t stream);
 // real in its storage type (measured projections stored as f16 or bf16)
 void launch_compare(uint32_t n, const void* real, etn_voxel_type real_type, const float* virt, float* residual,

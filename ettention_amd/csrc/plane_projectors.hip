@@ -1021,23 +1021,27 @@ void sweep_forward_typed(const SlabParams& s, const SweepForward& a, const void*
     else launch(std::false_type{});
 }
 
-// ---- oversampled back projections in one sweep ------------------------------------
-// The per_dir x per_dir sample pattern (PD = per_dir) with the fused kernels' fast
-// lookups.  A sample's u does not depend on its pattern row, which only moves it
-// along y, nor on the plane: the PD samples of a pattern row give u, column and
-// weight for all PD rows of all four planes, so a sample costs its record read
-// and 11 instruction slots (19 on the fused kernels, which also leave CUs idle
+// ---- oversampled and masked back projections in one sweep -------------------------
+// The fused kernels' fast arithmetic, operation for operation and in their sample
+// order: with kOver the per_dir x per_dir pattern (PD = per_dir) of their sample
+// loop, without it their single-sample update with a mask weight (PD = 1).  A
+// sample's u does not depend on its pattern row, which only moves it along y, nor
+// on the plane: the columns and weights of a pattern row's PD samples are worked
+// out once for all PD rows of all four planes, so a sample costs its record read
+// and 9 instruction slots (19 on the fused kernels, which also leave CUs idle
 // where the planes are no multiple of them).  A workgroup owns four planes x 64
 // columns x 4 kSampleDepth slices in registers.  250 x 300 x 150 bf16 with a mask,
-// 3 x 3 samples: 0.052 ms, with the forward sweep 0.094 where a fused pass takes
-// 0.25; eight slices a wave 0.07 (fewer workgroups).
+// 3 x 3 samples: 0.068 ms, with the forward sweep 0.110 where a fused pass takes
+// 0.25 (0.052 with a pattern row's contributions added before their weight, a
+// different rounding).
 constexpr int kSampleDepth = 4;      // slices a wave
 
-template <typename S, int PD>
+template <typename S, int PD, bool kOver>
 __global__ void __launch_bounds__(kSweepThreads, 4)
     sweep_samples_kernel(SlabParams s, const SampleView* __restrict__ views, int n, typename S::T* vol,
                          const uint8_t* __restrict__ mask, int nu, int nv)
 {
+    constexpr int kPlanes = PD >= 3 ? 2 : kSweepPlanes;   // planes whose reads are in flight together
     __shared__ f32x4 recs[kSweepPlanes * PD][kSweepColumns];
     __shared__ float weights[256];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1133,7 +1137,9 @@ __global__ void __launch_bounds__(kSweepThreads, 4)
                     w[t] = (rin & (t & 1 ? c1 : c0)) ? in[e][t] : 0.0f;
                 }
                 const float dr0 = w[1] - w[0], dr1 = w[3] - w[2], dl0 = w[5] - w[4], dl1 = w[7] - w[6];
-                recs[(half * PD + e) * 2 + h][k] = f32x4{fmaf(w[2] - w[0], ty[e], w[0]), fmaf(dr1 - dr0, ty[e], dr0),
+                // (a single sample's A and B carry lambda times the chord)
+                const float lc = kOver ? 1.0f : v.lambda * v.sw[0];
+                recs[(half * PD + e) * 2 + h][k] = f32x4{lc * fmaf(w[2] - w[0], ty[e], w[0]), lc * fmaf(dr1 - dr0, ty[e], dr0),
                                                          fmaf(w[6] - w[4], ty[e], w[4]), fmaf(dl1 - dl0, ty[e], dl0)};
             }
         }
@@ -1142,64 +1148,83 @@ __global__ void __launch_bounds__(kSweepThreads, 4)
 #pragma unroll
         for (int j = 0; j < kSampleDepth; ++j) {
             const float zc = s.bmin[2] + ((float)(zw + j) + 0.5f) * s.vs[2];
-            float sum[kSweepPlanes];
-            int used[kSweepPlanes], full = 0;
+            // the columns and weights of a pattern row's samples
+            const f32x4* at[PD];
+            float tx[PD];
 #pragma unroll
-            for (int p = 0; p < kSweepPlanes; ++p) {
-                sum[p] = 0.0f;
-                used[p] = 0;
-            }
-#pragma unroll 1
             for (int i = 0; i < PD; ++i) {
                 float u = m0 * (xc + v.sx[i]) + 0.0f;
                 u = u + m8 * (zc + v.sz[i]);
                 u = u + m12 * 1.0f;
                 u = u - 0.5f;
-                const float tx = __builtin_amdgcn_fractf(u);
                 int column;
-                asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(column) : "v"(u));
-                const f32x4* c = rec + column;
-                const float lw = v.lambda * v.sw[i];
-                // the common case, every record with rays through it, decided for
-                // the whole wave: no test, count or select a sample
-                float R[PD][kSweepPlanes], L[PD][kSweepPlanes], least = FLT_MAX;
-#pragma unroll
-                for (int ys = 0; ys < PD; ++ys)
-#pragma unroll
-                    for (int p = 0; p < kSweepPlanes; ++p) {
-                        const f32x4 e = c[(p * PD + ys) * kSweepColumns];
-                        R[ys][p] = fmaf(e[1], tx, e[0]);
-                        L[ys][p] = fmaf(e[3], tx, e[2]);
-                        least = fminf(least, L[ys][p]);
-                    }
-                if (__all(least > kEpsilon)) {
-                    full += PD;
-#pragma unroll
-                    for (int p = 0; p < kSweepPlanes; ++p) {
-                        float part = 0.0f;
-#pragma unroll
-                        for (int ys = 0; ys < PD; ++ys) part = fmaf(R[ys][p], __builtin_amdgcn_rcpf(L[ys][p]), part);
-                        sum[p] = fmaf(part, lw, sum[p]);
-                    }
+                if constexpr (kOver) {
+                    const float base = floorf(u);
+                    tx[i] = u - base;
+                    column = (int)base;
                 } else {
+                    tx[i] = __builtin_amdgcn_fractf(u);
+                    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(column) : "v"(u));
+                }
+                at[i] = rec + column;
+            }
+            if constexpr (kOver) {
+                float sum[kSweepPlanes];
+                int used[kSweepPlanes];
 #pragma unroll
-                    for (int p = 0; p < kSweepPlanes; ++p) {
-                        float part = 0.0f;
+                for (int p = 0; p < kSweepPlanes; ++p) {
+                    sum[p] = 0.0f;
+                    used[p] = 0;
+                }
+#pragma unroll 1
+                for (int ys = 0; ys < PD; ++ys) {
 #pragma unroll
-                        for (int ys = 0; ys < PD; ++ys) {
-                            const bool ok = L[ys][p] > kEpsilon;
-                            part = ok ? fmaf(R[ys][p], __builtin_amdgcn_rcpf(L[ys][p]), part) : part;
-                            used[p] += ok ? 1 : 0;
+                    for (int p0 = 0; p0 < kSweepPlanes; p0 += kPlanes) {
+                        float R[PD][kPlanes], L[PD][kPlanes], least = FLT_MAX;
+#pragma unroll
+                        for (int i = 0; i < PD; ++i)
+#pragma unroll
+                            for (int p = 0; p < kPlanes; ++p) {
+                                const f32x4 e = at[i][((p0 + p) * PD + ys) * kSweepColumns];
+                                R[i][p] = fmaf(e[1], tx[i], e[0]);
+                                L[i][p] = fmaf(e[3], tx[i], e[2]);
+                                least = __builtin_elementwise_minimum(least, L[i][p]);   // (a NaN stays)
+                            }
+                        // the common case, every record with rays through it, decided for
+                        // the whole wave: no test, count or select a sample
+                        const bool all = __all(least > kEpsilon);
+#pragma unroll
+                        for (int p = 0; p < kPlanes; ++p) used[p0 + p] += all ? PD : 0;
+#pragma unroll
+                        for (int i = 0; i < PD; ++i) {
+                            const float lw = v.lambda * v.sw[i];
+#pragma unroll
+                            for (int p = 0; p < kPlanes; ++p) {
+                                const float contrib = R[i][p] * lw * __builtin_amdgcn_rcpf(L[i][p]);
+                                if (all) {
+                                    sum[p0 + p] += contrib;
+                                } else {
+                                    const bool ok = L[i][p] > kEpsilon;
+                                    sum[p0 + p] += ok ? contrib : 0.0f;
+                                    used[p0 + p] += ok ? 1 : 0;
+                                }
+                            }
                         }
-                        sum[p] = fmaf(part, lw, sum[p]);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                __builtin_amdgcn_sched_barrier(0);
-            }
 #pragma unroll
-            for (int p = 0; p < kSweepPlanes; ++p) {
-                const int count = used[p] + full;
-                if (count != 0) value[j][p] += weights[mv[j] >> (8 * p) & 255u] * sum[p] / (float)count;
+                for (int p = 0; p < kSweepPlanes; ++p) {
+                    if (used[p] != 0) value[j][p] += weights[mv[j] >> (8 * p) & 255u] * sum[p] / (float)used[p];
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < kSweepPlanes; ++p) {
+                    const f32x4 e = at[0][p * kSweepColumns];
+                    const float R = fmaf(e[1], tx[0], e[0]), L = fmaf(e[3], tx[0], e[2]);
+                    const float next = fmaf(weights[mv[j] >> (8 * p) & 255u], R * __builtin_amdgcn_rcpf(L), value[j][p]);
+                    value[j][p] = L > kEpsilon ? next : value[j][p];
+                }
             }
             round_planes<S>(value[j]);
         }
@@ -1213,8 +1238,8 @@ __global__ void __launch_bounds__(kSweepThreads, 4)
 }
 
 template <typename S>
-void sweep_samples_typed(const SlabParams& s, const SampleView* views, int n, int per_dir, uint32_t nu, uint32_t nv,
-                         void* volume, const uint8_t* mask, hipStream_t stream)
+void sweep_samples_typed(const SlabParams& s, const SampleView* views, int n, int per_dir, bool over, uint32_t nu,
+                         uint32_t nv, void* volume, const uint8_t* mask, hipStream_t stream)
 {
     auto* vol = static_cast<typename S::T*>(volume);
     const dim3 grid((s.res[0] + kSweepTile - 1) / kSweepTile, (s.res[1] + kSweepPlanes - 1) / kSweepPlanes,
@@ -1222,10 +1247,11 @@ void sweep_samples_typed(const SlabParams& s, const SampleView* views, int n, in
     auto launch = [&](auto kernel) {
         kernel<<<grid, kSweepThreads, 0, stream>>>(s, views, n, vol, mask, (int)nu, (int)nv);
     };
-    if (per_dir == 1) launch(sweep_samples_kernel<S, 1>);
-    else if (per_dir == 2) launch(sweep_samples_kernel<S, 2>);
-    else if (per_dir == 3) launch(sweep_samples_kernel<S, 3>);
-    else launch(sweep_samples_kernel<S, 4>);
+    if (!over) launch(sweep_samples_kernel<S, 1, false>);
+    else if (per_dir == 1) launch(sweep_samples_kernel<S, 1, true>);
+    else if (per_dir == 2) launch(sweep_samples_kernel<S, 2, true>);
+    else if (per_dir == 3) launch(sweep_samples_kernel<S, 3, true>);
+    else launch(sweep_samples_kernel<S, 4, true>);
 }
 
 }  // namespace
@@ -1398,13 +1424,14 @@ bool make_sample_view(const SlabParams& s, const BpParams& b, const float* resid
     return true;
 }
 
-void sweep_samples_project(const SlabParams& s, const SampleView* views, int n, int per_dir, uint32_t nu, uint32_t nv,
-                           etn_voxel_type vt, void* volume, const uint8_t* mask, hipStream_t stream)
+void sweep_samples_project(const SlabParams& s, const SampleView* views, int n, int per_dir, bool over, uint32_t nu,
+                           uint32_t nv, etn_voxel_type vt, void* volume, const uint8_t* mask, hipStream_t stream)
 {
     if (n <= 0) return;
-    if (vt == ETN_VOXEL_FLOAT16) sweep_samples_typed<F16>(s, views, n, per_dir, nu, nv, volume, mask, stream);
-    else if (vt == ETN_VOXEL_BFLOAT16) sweep_samples_typed<BF16>(s, views, n, per_dir, nu, nv, volume, mask, stream);
-    else sweep_samples_typed<F32>(s, views, n, per_dir, nu, nv, volume, mask, stream);
+    if (!over && per_dir != 1) fail("back projection sweep: a sample pattern is oversampled");
+    if (vt == ETN_VOXEL_FLOAT16) sweep_samples_typed<F16>(s, views, n, per_dir, over, nu, nv, volume, mask, stream);
+    else if (vt == ETN_VOXEL_BFLOAT16) sweep_samples_typed<BF16>(s, views, n, per_dir, over, nu, nv, volume, mask, stream);
+    else sweep_samples_typed<F32>(s, views, n, per_dir, over, nu, nv, volume, mask, stream);
     hip_check(hipGetLastError(), "back projection sweep launch");
 }
 

@@ -170,11 +170,8 @@ def test_block_sweeps_equal_the_fused_passes(shape, ntilts, block, reach, voxel,
     assert norm == ref
 
 
-# sample patterns, sub-rays and masks in the sweeps.  They add a voxel's samples
-# in another order than the fused pass does: up to 16 terms of one rounding each,
-# so a relative 1e-6 of every update, below the 2e-5 that two reconstructions in
-# single precision may differ by; 16-bit storage rounds some voxels the other way
-# (half an ulp of the type at most, in the mean far less).
+# sample patterns, sub-rays and masks in the sweeps, within what two
+# reconstructions in single precision may differ by
 @pytest.mark.parametrize("shape,ntilts,block,fp,bp,masked,voxel", [
     ((90, 81, 77), 17, 0, 1, 1, True, "float"), ((88, 83, 76), 13, 8, 1, 1, True, "half"),
     ((88, 81, 77), 9, 1, 2, 4, False, "float"), ((91, 82, 70), 9, 1, 4, 9, True, "float"),
@@ -196,3 +193,36 @@ def test_sampled_sweeps_match_the_fused_passes(shape, ntilts, block, fp, bp, mas
     bound = 2e-5 if voxel == "float" else 1e-2
     assert np.linalg.norm(v - w) <= bound * np.linalg.norm(w)
     assert abs(norm - ref) <= bound * ref
+
+
+# the same bit for bit, also with shapes that take two planes a workgroup (nx in
+# fours and odd) and with a tile set between two iterations, which leaves the
+# sweeps for the fused passes
+@pytest.mark.parametrize("shape,ntilts,block,fp,bp,masked,voxel", [
+    ((90, 81, 77), 17, 0, 1, 1, True, "float"), ((88, 83, 76), 13, 8, 1, 1, True, "half"),
+    ((88, 81, 77), 9, 1, 2, 4, False, "float"), ((91, 82, 70), 9, 1, 4, 9, True, "float"),
+    ((92, 81, 72), 12, 4, 3, 16, True, "float"), ((88, 80, 79), 9, 1, 1, 9, True, "bfloat16"),
+    ((250, 300, 16), 5, 1, 4, 9, True, "bfloat16"), ((252, 300, 16), 5, 1, 4, 4, True, "float"),
+    ((252, 260, 130), 3, 1, 3, 1, False, "half")])
+def test_sampled_sweeps_equal_the_fused_passes(shape, ntilts, block, fp, bp, masked, voxel):
+    nx, ny, nz = shape
+    rng = np.random.default_rng(ntilts)
+    case = dict(volume=E.VolumeGeometry.make(shape), base_geometry=E.ScannerGeometry.mrc_base(nx, ny),
+                tilt_angles=np.linspace(-60, 60, ntilts).astype(np.float32),
+                projections=torch.from_numpy(rng.normal(1.0, 0.3, (ntilts, ny, nx)).astype(np.float32)).cuda(),
+                algorithm="blockiterative" if block else "sirt", block_size=block, lam=0.3, voxel_type=voxel,
+                fp_samples=fp, bp_samples=bp)
+    if masked:
+        mask = rng.integers(0, 256, (nz, ny, nx)).astype(np.uint8)
+        mask[:, : ny // 3] = 0
+        case["mask"] = torch.from_numpy(mask).cuda()
+    print("sampled sweeps", shape, block, fp, bp, masked, voxel, flush=True)
+    v, norm = run(case)
+    w, ref = run(case, flags=LDS)
+    np.testing.assert_array_equal(v, w)
+    assert norm == ref
+    r = A.BlockIterativeReconstructionOperator(**case)
+    r.run_iterations(1)
+    r.set_tile(*r.tile())
+    r.run_iterations(1)
+    np.testing.assert_array_equal(r.get_reconstructed_volume(dtype=torch.float32).cpu().numpy(), w)
