@@ -191,7 +191,8 @@ def main():
     # the committed PMC traffic summaries cover the 512^3 metric workload (f32 and bf16; f32 masked)
     plain = args.fp_samples == 1 and args.bp_samples == 1
     roofline = kernel_roofline(r, args.voxel_type, fused, V, P, block, masked=mask is not None,
-                               pmc=args.workload == "metric" and plain, gpu_ms_per_step=gpu_ms_per_step, N=N)
+                               pmc=args.workload == "metric" and plain, gpu_ms_per_step=gpu_ms_per_step, N=N,
+                               over=not plain)
     if args.fp_samples != 1 or args.bp_samples != 1:
         roofline["kernel"] += ", FP %dx%d sub-rays, BP %d samples" % (args.fp_samples, args.fp_samples,
                                                                      args.bp_samples)
@@ -482,9 +483,10 @@ def run_wbp(args):
     projection filtered, its ray length computed and back-projected with
     lambda / N).  GUPS = V x N / seconds per reconstruction.  The dominant
     kernel is the back projection sweep (up to 64 projections per volume
-    sweep), timed with HIP events around its launches in one more run; its
-    algorithmic bytes are those of one sweep for its B projections, 2 s V + 8 P B
-    (the volume read and written once, residual and length images read)."""
+    sweep; the library reports which kernel ran), timed with HIP events around
+    its launches in one more run; its algorithmic bytes are those of one launch
+    for the B projections it carries on average, 2 s V + 8 P B (the volume read
+    and written once, residual and length images read)."""
     import torch
     import ettention_amd as E
     from ettention_amd import api as A
@@ -532,11 +534,11 @@ def run_wbp(args):
     kernel, bp_ms, launches = r.time_kernels()
     del r
     torch.cuda.empty_cache()
-    if kernel == 0:
-        # a sweep carries up to 64 projections; launches of the fused kernels eight
-        B = N / launches if launches * 8 < N else 8
+    if kernel in (0, 3):
+        # (of the fused launches those carrying eight projections are timed)
+        B = N / launches if kernel == 3 else 8
         name = "%s (back projections only, %g projections per launch)" % (
-            "sweep_back_kernel" if launches * 8 < N else "fused_plane_kernel", B)
+            "sweep_back_kernel" if kernel == 3 else "fused_plane_kernel", B)
     else:
         B = 1
         name = "back_project_kernel (generic, one projection with lambda / N)"
@@ -574,7 +576,7 @@ def run_wbp(args):
         "dtype": "f32",
         "data": "synthetic (seeded ellipsoid phantom, FP projections + 2% Gaussian noise)",
         "config": {"workload": wl["name"], "volume": [nx, ny, nz], "detector": [nu, nv], "projections": N,
-                   "algorithm": "wbp", "kernels": "fused-plane" if kernel == 0 else "generic",
+                   "algorithm": "wbp", "kernels": {0: "fused-plane", 3: "sweeps"}.get(kernel, "generic"),
                    "parallelism": "single GPU"},
         "roofline": roofline,
         "cpu_baseline": cpu,
@@ -728,14 +730,15 @@ def run_learned(args):
         "result": {k: (round(v, 6) if isinstance(v, float) else v) for k, v in res.items() if k != "plain_norms"},
         "roofline": {"bound": "mfma", "achieved": round(tflops, 1), "peak": 2500.0, "unit": "TFLOP/s",
                      "frac": round(tflops / 2500.0, 4), "traffic": None,
-                     "kernel": "conv3_fwd_kernel (whole network forward at %d^3)" % n,
+                     "kernel": "conv3_brick_kernel (whole network forward at %d^3)" % n,
                      "avg_launch_ms": round(fwd_ms, 4), "flops_per_forward": flops},
         "cpu_baseline": None,
     }
     print(json.dumps(out), flush=True)
 
 
-def kernel_roofline(r, voxel_type, fused, V, P, block=1, masked=False, pmc=True, gpu_ms_per_step=None, N=1):
+def kernel_roofline(r, voxel_type, fused, V, P, block=1, masked=False, pmc=True, gpu_ms_per_step=None, N=1,
+                    over=False):
     """The dominant kernel's algorithmic bytes against its measured time.
 
     Fused plane kernel: an iteration's launches are all this kernel.  Its
@@ -751,6 +754,11 @@ def kernel_roofline(r, voxel_type, fused, V, P, block=1, masked=False, pmc=True,
     itself (B' projections each way: the compulsory bytes); the rocprofv3
     counters give the measured traffic.
 
+    Separate sweeps (blocks of several projections, oversampling or a mask,
+    where the library takes them): the same algorithmic bytes over the launches
+    of the back and the forward projection sweeps together; an iteration's
+    compulsory bytes are (2 s) V a back sweep, s V a forward sweep and 20 P N.
+
     Generic kernels (FP: s V + 8 P; BP: 2 s V + 8 P per launch) share the
     timed region with the residual kernels, so their duration comes from one
     extra eager iteration with HIP events around every launch.  A mask adds
@@ -759,7 +767,7 @@ def kernel_roofline(r, voxel_type, fused, V, P, block=1, masked=False, pmc=True,
     m = 1 if masked else 0
     kernel, eager_ms, launches = r.time_kernels()
     if fused:
-        assert kernel == 0
+        assert kernel in (0, 3)
         blocks = -(-N // block)
         alg_iter = blocks * (3 * s + 2 * m) * V + 20 * P * N
         dur_ms = gpu_ms_per_step / launches
@@ -769,6 +777,11 @@ def kernel_roofline(r, voxel_type, fused, V, P, block=1, masked=False, pmc=True,
                   % launches)
         name = ("fused_plane_kernel (BP of projection k-1 + FP/residual of projection k)" if block == 1 else
                 "fused_plane_kernel (BPs of block b-1 + FPs/residuals of block b, %d projections per block)" % block)
+        if kernel == 3:
+            pmc = False
+            kernel_bytes = (blocks * (2 * s + m) * V + (launches - blocks) * (s + m) * V + 20 * P * N) / launches
+            name = "%s + sweep_forward_kernel (%d projections per block)" % (
+                "sweep_samples_kernel" if masked or over else "sweep_back_kernel", block)
     else:
         dur_ms = eager_ms
         source = "one extra eager iteration, HIP events around every launch"

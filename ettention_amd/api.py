@@ -330,7 +330,7 @@ class BlockIterativeReconstructionOperator:
 
     def time_kernels(self):
         """(kernel id, average ms, launches) of the dominant kernel over one extra
-        eagerly launched iteration (0 fused, 1 generic FP, 2 generic BP)."""
+        eagerly launched iteration (0 fused, 1 generic FP, 2 generic BP, 3 separate sweeps)."""
         k = C.c_int()
         ms = C.c_double()
         n = C.c_uint32()

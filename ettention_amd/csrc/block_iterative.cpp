@@ -315,9 +315,10 @@ void BlockIterativeReconstructionOperator::synchronize()
 double BlockIterativeReconstructionOperator::timeKernels(int* kernel, uint32_t* launches)
 {
     if (fused_) {
-        // average over the launches that carry both a back and a forward projection
+        // average over the launches that carry both a back and a forward
+        // projection, or over the separate sweeps
         ensureTuned();
-        *kernel = 0;
+        *kernel = fused_->sweeps() ? 3 : 0;
         double total = 0.0;
         uint32_t n = 0, all = 0;
         for (const auto& t : fused_->timeIteration(stream_)) {

@@ -511,6 +511,7 @@ public:
     void tile(size_t member, int* planes, int* band) const override;
     void setThreads(int threads, hipStream_t stream) override;
     int threads() const override { return threads_; }
+    bool sweeps() const override { return !split_.empty() && !split_off_; }
     size_t memberCount() const override { return members_.size(); }
     double residualNorm(size_t member, double* scratch, hipStream_t stream) override;
 
@@ -542,6 +543,7 @@ private:
     float timeSchedule(const Schedule& s, hipStream_t stream) const;
     void plan_split(hipStream_t stream);
     void enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* ev) const;
+    size_t splitLaunches() const;
 
     // An iteration as separate sweeps (blocks of several projections): per block
     // the back projections of the block before it, all in one sweep, then the
@@ -698,19 +700,30 @@ void FusedEngineImpl::enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* 
 {
     const MemberPlan& m = members_[0];
     void* volume = m.op->getReconstructedVolume()->data();
-    for (size_t k = 0; k < split_.size(); ++k) {
-        const SplitBlock& b = split_[k];
+    size_t k = 0;   // launches so far
+    auto timed = [&](auto&& launch) {
         if (ev) ETN_HIP(hipEventRecord((*ev)[2 * k], stream));
-        if (!over_ && !m.mask)
-            dev::sweep_back_project(split_slab_, split_groups_, split_back_.as<dev::BackView>() + b.back_first,
-                                    b.back_count, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
-        else
-            dev::sweep_samples_project(split_slab_, split_back_.as<dev::SampleView>() + b.back_first, b.back_count,
-                                       m.rowsets, over_, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, m.mask, stream);
-        for (const ForwardSweep& f : b.forward)
-            dev::sweep_forward_project(split_slab_, split_forward_.as<dev::ForwardView>() + f.first, f.count, f.zdir,
-                                       (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, vt_, volume, m.mask, stream);
+        launch();
         if (ev) ETN_HIP(hipEventRecord((*ev)[2 * k + 1], stream));
+        ++k;
+    };
+    for (const SplitBlock& b : split_) {
+        if (b.back_count > 0)
+            timed([&] {
+                if (!over_ && !m.mask)
+                    dev::sweep_back_project(split_slab_, split_groups_, split_back_.as<dev::BackView>() + b.back_first,
+                                            b.back_count, (uint32_t)m.nu, (uint32_t)m.nv, vt_, volume, stream);
+                else
+                    dev::sweep_samples_project(split_slab_, split_back_.as<dev::SampleView>() + b.back_first,
+                                               b.back_count, m.rowsets, over_, (uint32_t)m.nu, (uint32_t)m.nv, vt_,
+                                               volume, m.mask, stream);
+            });
+        for (const ForwardSweep& f : b.forward)
+            timed([&] {
+                dev::sweep_forward_project(split_slab_, split_forward_.as<dev::ForwardView>() + f.first, f.count,
+                                           f.zdir, (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, vt_, volume, m.mask,
+                                           stream);
+            });
     }
 }
 
@@ -932,9 +945,16 @@ void FusedEngineImpl::enqueue(const Schedule& s, size_t first, size_t last, hipS
     }
 }
 
+size_t FusedEngineImpl::splitLaunches() const
+{
+    size_t n = 0;
+    for (const SplitBlock& b : split_) n += (b.back_count > 0 ? 1 : 0) + b.forward.size();
+    return n;
+}
+
 void FusedEngineImpl::enqueueIteration(hipStream_t stream)
 {
-    if (!split_.empty() && !split_off_) enqueueSplit(stream, nullptr);
+    if (sweeps()) enqueueSplit(stream, nullptr);
     else enqueue(sched_, 0, sched_.launches.size(), stream, nullptr);
 }
 
@@ -1026,8 +1046,8 @@ void FusedEngineImpl::check(hipStream_t stream)
 
 std::vector<FusedPlaneEngine::LaunchTime> FusedEngineImpl::timeIteration(hipStream_t stream)
 {
-    const bool split = !split_.empty() && !split_off_;
-    const size_t n = split ? split_.size() : sched_.launches.size();
+    const bool split = sweeps();
+    const size_t n = split ? splitLaunches() : sched_.launches.size();
     std::vector<hipEvent_t> ev(2 * n);
     for (auto& e : ev) ETN_HIP(hipEventCreate(&e));
     if (split) enqueueSplit(stream, &ev);
@@ -1038,8 +1058,7 @@ std::vector<FusedPlaneEngine::LaunchTime> FusedEngineImpl::timeIteration(hipStre
         if (!split && sched_.launches[k].groups == 0) continue;
         float ms = 0.0f;
         ETN_HIP(hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]));
-        // (a block's sweeps count as one launch)
-        out.push_back({ms, split ? split_[k].back_count > 0 && !split_[k].forward.empty() : sched_.launches[k].steady});
+        out.push_back({ms, split || sched_.launches[k].steady});
     }
     for (auto& e : ev) (void)hipEventDestroy(e);
     return out;
@@ -1162,7 +1181,7 @@ void FusedEngineImpl::tuneTiles(hipStream_t stream)
 // the engine's whole schedule; keep the fastest shape with its tiles.
 void FusedEngineImpl::autotune(hipStream_t stream)
 {
-    if (!split_.empty() && !split_off_) return;   // the sweeps have no tiles
+    if (sweeps()) return;   // they have no tiles
     // Candidates: workgroup shape x cap on the rays per thread.  A lower cap
     // needs fewer registers per thread (more waves per SIMD: two rays take
     // about 120 VGPRs, eight about 190) but splits a block's forward

@@ -53,7 +53,7 @@ public:
     };
     struct LaunchTime {
         float ms;
-        bool steady;            // every member pass of the launch carries a back and a forward projection
+        bool steady;            // a sweep, or every member pass of the launch carries a back and a forward projection
     };
 
     // Builds an engine over the members that have a fused form (geometry,
@@ -67,6 +67,10 @@ public:
                                                     hipStream_t stream, std::vector<bool>* taken);
     virtual ~FusedPlaneEngine() = default;
     virtual void enqueueIteration(hipStream_t stream) = 0;
+    // Whether an iteration is separate back and forward projection sweeps (one
+    // member: blocks of several projections, oversampling or a mask, where they
+    // are the faster) instead of fused passes; the volumes are the same bit for bit.
+    virtual bool sweeps() const = 0;
     // Throws when a kernel found a live ray outside the plane its row was assigned to.
     virtual void check(hipStream_t stream) = 0;
     // One eager iteration with an event pair around every launch.
@@ -79,6 +83,7 @@ public:
     // Index is the member's position among the engine's members (in the order
     // given to create).  Throws ETN_ERROR_INVALID_ARGUMENT for a tile that
     // does not fit; reallocates the launch tables (no captured graph may use them).
+    // A tile and a workgroup shape are the fused passes': setting one leaves the sweeps.
     virtual void setTile(size_t member, int planes, int band, hipStream_t stream) = 0;
     virtual void tile(size_t member, int* planes, int* band) const = 0;
     // Workgroup shape of every launch: 512 threads (64 KiB LDS, two workgroups

@@ -245,7 +245,7 @@ double WeightedBackProjection::timeKernels(int* kernel, uint32_t* launches)
 {
     std::vector<float> ms;
     if (usesFusedPath()) {
-        *kernel = 0;
+        *kernel = views_.get() ? 3 : 0;
         launch_ms_ = &ms;
         try {
             run();

@@ -36,8 +36,8 @@ public:
     // arithmetic are asked for.
     bool usesFusedPath() const override { return fused_ != nullptr || views_.get() != nullptr; }
     // One more run() with HIP events around the back projections: the average
-    // sweep, or fused launch carrying eight projections (*kernel = 0), or the
-    // generic back projection (*kernel = 2).  Adds to the volume.
+    // sweep (*kernel = 3), fused launch carrying eight projections (0) or
+    // generic back projection (2).  Adds to the volume.
     double timeKernels(int* kernel, uint32_t* launches) override;
 
     // GenerateRamLakKernel.cl: value at position p = i - resolution / 2 is 1/4

@@ -276,8 +276,10 @@ etn_status etn_reconstruction_uses_fused_path(etn_reconstruction* r, int* out);
  * average duration of the kernel that dominates it: *kernel = 0 fused plane
  * kernel (average over the launches carrying a back and a forward projection;
  * *launches = every launch of the iteration), 1 generic forward projection,
- * 2 generic back projection (*launches = that kernel's launches).  Advances
- * the reconstruction. */
+ * 2 generic back projection (*launches = that kernel's launches), 3 separate
+ * back and forward projection sweeps (average over all of them, *launches
+ * their number; "wbp": back projection sweeps only).  Advances the
+ * reconstruction. */
 etn_status etn_reconstruction_time_kernels(etn_reconstruction* r, int* kernel, double* average_ms,
                                            uint32_t* launches);
 /* Extension (no reference counterpart): the fused kernels' tile, i.e. volume

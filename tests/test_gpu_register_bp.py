@@ -56,6 +56,16 @@ def run(case, flags=0, threads=None, tile=None, iterations=2):
     return r.get_reconstructed_volume(dtype=torch.float32).cpu().numpy(), r.residual_norm()
 
 
+FUSED, SWEEPING = 0, 3      # the library's own report of what it timed
+
+
+def timed_kernel(case, flags=0):
+    kernel, ms, launches = A.BlockIterativeReconstructionOperator(
+        flags=flags | E.ETN_RECON_FLAG_NO_AUTOTUNE, **case).time_kernels()
+    assert launches > 0 and (kernel != SWEEPING or ms > 0.0)   # (a single block has no steady fused pass)
+    return kernel
+
+
 CASES = {
     "sart": ((64, 64, 64), 41, {}),
     "block4": ((48, 48, 40), 61, dict(algorithm="blockiterative", block_size=4, projection_iteration="maxangle")),
@@ -170,6 +180,32 @@ def test_block_sweeps_equal_the_fused_passes(shape, ntilts, block, reach, voxel,
     assert norm == ref
 
 
+def test_time_kernels_tells_sweeps_from_fused_passes():
+    # 16 projections in blocks of 8: per block one back sweep and a forward sweep
+    # for each z direction among its projections
+    shape = (130, 130, 128)
+    case = dict(volume=E.VolumeGeometry.make(shape), base_geometry=E.ScannerGeometry.mrc_base(130, 130),
+                tilt_angles=np.linspace(0, 60, 16).astype(np.float32),
+                projections=torch.ones((16, 130, 130), device="cuda"), algorithm="blockiterative", block_size=8,
+                projection_iteration="identity")
+    kernel, ms, launches = A.BlockIterativeReconstructionOperator(**case).time_kernels()
+    assert (kernel, launches) == (SWEEPING, 4) and ms > 0.0
+    assert timed_kernel(case, LDS) == FUSED
+    r = A.BlockIterativeReconstructionOperator(**case)
+    r.set_tile(*r.tile())                       # a tile is one of the fused passes'
+    assert r.time_kernels()[0] == FUSED
+
+
+def test_wbp_time_kernels_tells_sweeps_from_fused_passes():
+    n, count = 40, 70                           # two chunks of up to 64 projections, a sweep each
+    case = dict(volume=E.VolumeGeometry.make((n, n, n)), base_geometry=E.ScannerGeometry.mrc_base(n, n),
+                tilt_angles=np.linspace(-60, 60, count).astype(np.float32),
+                projections=torch.ones((count, n, n), device="cuda"))
+    assert A.WeightedBackProjection(**case).time_kernels()[::2] == (SWEEPING, 2)
+    assert A.WeightedBackProjection(flags=LDS, **case).time_kernels()[0] == FUSED
+    assert A.WeightedBackProjection(flags=E.ETN_RECON_FLAG_GENERIC_KERNELS, **case).time_kernels()[0] == 2
+
+
 # sample patterns, sub-rays and masks in the sweeps, within what two
 # reconstructions in single precision may differ by
 @pytest.mark.parametrize("shape,ntilts,block,fp,bp,masked,voxel", [
@@ -221,6 +257,7 @@ def test_sampled_sweeps_equal_the_fused_passes(shape, ntilts, block, fp, bp, mas
     w, ref = run(case, flags=LDS)
     np.testing.assert_array_equal(v, w)
     assert norm == ref
+    assert timed_kernel(case) == SWEEPING and timed_kernel(case, LDS) == FUSED
     r = A.BlockIterativeReconstructionOperator(**case)
     r.run_iterations(1)
     r.set_tile(*r.tile())
