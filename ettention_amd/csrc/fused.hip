@@ -542,6 +542,7 @@ private:
     void tuneTiles(hipStream_t stream);
     float timeSchedule(const Schedule& s, hipStream_t stream) const;
     void plan_split(hipStream_t stream);
+    bool sweepsPay(const MemberPlan& m, bool plain) const;
     void enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* ev) const;
     size_t splitLaunches() const;
 
@@ -589,6 +590,59 @@ FusedEngineImpl::FusedEngineImpl(std::vector<MemberPlan> members, etn_voxel_type
     plan_split(stream);
 }
 
+// Where the sweeps are the faster (fused passes against sweeps, us for 31 tilts,
+// f32 unless 16 bits are named).  They are two or three launches a block of 10 to
+// 20 us each, whose workgroups own whole tiles of 64 columns and 64 slices (16
+// with samples or a mask): small volumes do not fill the launches, narrow and flat
+// ones the tiles.  A fused pass lasts as long as a CU's planes do.
+bool FusedEngineImpl::sweepsPay(const MemberPlan& m, bool plain) const
+{
+    const size_t voxels = (size_t)m.nx * m.ny * m.nz;
+    const double cu_work = (double)m.nx * m.nz * std::max(1.0, m.ny / 256.0);
+    const bool half = vt_ != ETN_VOXEL_FLOAT32;
+    if (plain) {
+        // up to 128 columns: 64 x 256 x 128 167 / 236, 128 x 160 x 128 245 / 279,
+        // 128^3 244 / 244, 64 x 512 x 256 314 / 306, 128 x 128 x 256 413 / 304; beyond,
+        // where the fused passes' rows are no power of two or fill a workgroup with
+        // one plane: 132 x 1000 x 20 302 / 229, 256 x 256 x 64 270 / 238
+        if (m.nx <= 128 && cu_work <= 16384.0) return false;
+        // blocks of 8: 256^3 780 / 542; 32 x 512 x 256 195 / 245, 48 x 512 x 256 297 / 260,
+        // 512 x 512 x 16 360 / 354.  16-bit volumes: a sweep's loads and stores are half
+        // as wide and every projection rounds: blocks of 8: 256^3 800 / 651,
+        // 64 x 512 x 256 330 / 349, 96 x 512 x 256 685 / 593, 112 x 200 x 200 436 / 350,
+        // 512 x 512 x 32 503 / 509, x 48 647 / 542, 520 x 70 x 64 801 / 285;  of 16:
+        // 64 x 512 x 256 348 / 300, 512 x 512 x 16 398 / 391
+        if (m.bmax >= (half ? 16u : 8u)) return m.nx >= 48 && m.nz >= 16 && voxels >= (size_t)1 << 21;
+        if (m.bmax >= 8) return m.nx >= 96 && m.nz >= 48 && voxels >= (size_t)2200000;
+        // blocks of 4: 256^3 841 / 718, 128 x 512 x 256 630 / 688 (of 5 698 / 664),
+        // 512 x 512 x 32 480 / 493, x 48 612 / 566; 256^3 on a detector of 128^2 616 / 657
+        // (the fused pass traces fewer rays);  of 2: 256^3 1115 / 1328.  16 bits, of 4:
+        // 256^3 874 / 919;  of 5: 256^3 912 / 875, 512 x 512 x 128 1350 / 1346;  of 6:
+        // 128 x 512 x 256 669 / 778, 512 x 512 x 48 636 / 685, x 64 774 / 732
+        if (m.bmax < 4 || voxels < (size_t)1 << 23 || 4 * (size_t)m.nu < 3 * (size_t)m.nx) return false;
+        if (!half) return m.nx >= (m.bmax < 5 ? 129 : 96) && m.nz >= 48;
+        return m.bmax >= 5 && m.nx > 128 && m.nz >= (m.bmax < 6 ? 128 : 64);
+    }
+    // masked, blocks of 8: 96^3 408 / 279, 256^3 1053 / 937, 32 x 512 x 256 220 / 267,
+    // 40 x 200 x 200 234 / 150, 64 x 128 x 64 120 / 128, 128 x 512 x 8 108 / 113, 512 x 512 x 8 287 / 196;
+    // of 4: 128^3 409 / 430
+    if (!over_)
+        return m.bmax >= 8 && m.nx >= 40 && voxels > (size_t)1 << (m.nz < 16 ? 20 : 19);
+    // tiles at least 5/8 full: 32 x 512 x 256, 4 samples, 863 / 1388;
+    // 132 x 1000 x 20, 9 samples, 1297 / 1773 (0.43 full)
+    const size_t tiles = (size_t)((m.nx + 63) / 64 * 64) * ((m.nz + 15) / 16 * 16) * m.ny;
+    if (8 * voxels < 5 * tiles) return false;
+    // forward sub-rays alone: 4 x 4 96^3 684 / 718, 204^3 1987 / 1803;
+    // 2 x 2 204^3 1500 / 1584, 256^3 2009 / 1958, in blocks of 8 204^3 1299 / 588
+    if (m.bp_samples == 1) return voxels >= (size_t)1 << (m.fp_n == 2 && m.bmax == 1 ? 24 : 23);
+    if (voxels < 500000) return false;
+    // 9 samples: 80^3 with a mask 1009 / 884;  4 samples, blocks of 2: 96^3 554 / 510
+    if (m.bp_samples > 4 || m.bmax > 1) return true;
+    // 4 samples, SART: 96^3 745 / 752, 104^3 845 / 809, 128^3 1119 / 917;
+    // 200 x 400 x 32 737 / 860, 512 x 512 x 16 966 / 917
+    return cu_work > (m.ny <= 256 ? 10000.0 : 13000.0);
+}
+
 // The fused pass reads the volume once for a block's back and forward
 // projections, but works out every voxel's column and every ray's steps in
 // every plane: with several projections a pass it is bound by that (512 x 512 x
@@ -602,21 +656,7 @@ void FusedEngineImpl::plan_split(hipStream_t stream)
     if (members_.size() != 1 || exact_ || sr_ || cap_ || !reg_bp_) return;
     const MemberPlan& m = members_[0];
     const bool plain = !over_ && !m.mask;
-    // Where the sweeps are the faster (fused passes against sweeps, 31 tilts, n^3
-    // f32 voxels).  They are two launches a block, of fewer workgroups:
-    //   blocks of 8: 96^3 318 / 326 us, 128^3 356 / 348, 256^3 928 / 697
-    //   blocks of 4: 128^3 387 / 455, 256^3 1000 / 889;  of 2: 256^3 1115 / 1328
-    //   masked, 8: 96^3 408 / 279, 256^3 1053 / 937;  masked, 4: 128^3 409 / 430
-    //   2 x 2 sub-rays, 4 samples: 64^3 587 / 637, 80^3 730 / 699, 96^3 841 / 788
-    //   4 x 4 sub-rays, 1 sample: 96^3 684 / 718
-    const size_t voxels = (size_t)m.nx * m.ny * m.nz;
-    if (over_) {
-        if (voxels < (m.bp_samples > 1 ? (size_t)500000 : (size_t)1 << 23)) return;
-    } else if (m.mask) {
-        if (m.bmax < 8 || voxels < (size_t)1 << 19) return;
-    } else {
-        if (m.bmax < 4 || voxels < (size_t)1 << (m.bmax < 8 ? 23 : 21)) return;
-    }
+    if (!sweepsPay(m, plain)) return;
     BlockIterativeReconstructionOperator& op = *m.op;
     GpuVolume* vol = op.getReconstructedVolume();
     const VolumeProperties vp = whole_volume(vol->properties());

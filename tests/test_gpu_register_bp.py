@@ -196,6 +196,32 @@ def test_time_kernels_tells_sweeps_from_fused_passes():
     assert r.time_kernels()[0] == FUSED
 
 
+# which reconstructions are swept: sizes on both sides of the lines that
+# measurements drew (FusedEngineImpl::sweepsPay)
+@pytest.mark.parametrize("shape,block,voxel,fp,bp,masked,kernel", [
+    ((128, 160, 128), 8, "float", 1, 1, False, FUSED), ((128, 128, 132), 8, "float", 1, 1, False, SWEEPING),
+    ((32, 512, 300), 8, "float", 1, 1, False, FUSED), ((48, 400, 300), 8, "float", 1, 1, False, SWEEPING),
+    ((256, 256, 32), 8, "float", 1, 1, False, SWEEPING), ((512, 512, 8), 8, "float", 1, 1, False, FUSED),
+    ((80, 256, 256), 8, "half", 1, 1, False, FUSED), ((112, 200, 200), 8, "half", 1, 1, False, SWEEPING),
+    ((512, 256, 32), 8, "bfloat16", 1, 1, False, FUSED), ((512, 256, 48), 8, "bfloat16", 1, 1, False, SWEEPING),
+    ((64, 256, 300), 16, "bfloat16", 1, 1, False, SWEEPING), ((128, 256, 256), 4, "float", 1, 1, False, FUSED),
+    ((256, 512, 64), 4, "float", 1, 1, False, SWEEPING), ((256, 512, 64), 4, "bfloat16", 1, 1, False, FUSED),
+    ((256, 512, 64), 6, "bfloat16", 1, 1, False, SWEEPING), ((32, 512, 64), 8, "float", 1, 1, True, FUSED),
+    ((96, 96, 96), 8, "float", 1, 1, True, SWEEPING), ((96, 96, 96), 1, "float", 2, 4, False, FUSED),
+    ((104, 104, 104), 1, "float", 2, 4, False, SWEEPING), ((132, 1000, 20), 1, "float", 1, 9, False, FUSED),
+    ((200, 400, 32), 1, "float", 1, 4, False, FUSED), ((204, 204, 204), 1, "float", 2, 1, False, FUSED),
+    ((204, 204, 204), 1, "float", 3, 1, False, SWEEPING)])
+def test_sweeps_where_they_pay(shape, block, voxel, fp, bp, masked, kernel):
+    nx, ny, nz = shape
+    case = dict(volume=E.VolumeGeometry.make(shape), base_geometry=E.ScannerGeometry.mrc_base(nx, ny),
+                tilt_angles=np.linspace(-60, 60, 16).astype(np.float32),
+                projections=torch.ones((16, ny, nx), device="cuda"), algorithm="blockiterative", block_size=block,
+                voxel_type=voxel, fp_samples=fp, bp_samples=bp)
+    if masked:
+        case["mask"] = torch.full((nz, ny, nx), 255, dtype=torch.uint8, device="cuda")
+    assert timed_kernel(case) == kernel
+
+
 def test_wbp_time_kernels_tells_sweeps_from_fused_passes():
     n, count = 40, 70                           # two chunks of up to 64 projections, a sweep each
     case = dict(volume=E.VolumeGeometry.make((n, n, n)), base_geometry=E.ScannerGeometry.mrc_base(n, n),
@@ -236,9 +262,9 @@ def test_sampled_sweeps_match_the_fused_passes(shape, ntilts, block, fp, bp, mas
 # sweeps for the fused passes
 @pytest.mark.parametrize("shape,ntilts,block,fp,bp,masked,voxel", [
     ((90, 81, 77), 17, 0, 1, 1, True, "float"), ((88, 83, 76), 13, 8, 1, 1, True, "half"),
-    ((88, 81, 77), 9, 1, 2, 4, False, "float"), ((91, 82, 70), 9, 1, 4, 9, True, "float"),
+    ((104, 81, 98), 9, 1, 2, 4, False, "float"), ((91, 82, 76), 9, 1, 4, 9, True, "float"),
     ((92, 81, 72), 12, 4, 3, 16, True, "float"), ((88, 80, 79), 9, 1, 1, 9, True, "bfloat16"),
-    ((250, 300, 16), 5, 1, 4, 9, True, "bfloat16"), ((252, 300, 16), 5, 1, 4, 4, True, "float"),
+    ((250, 300, 16), 5, 1, 4, 9, True, "bfloat16"), ((252, 300, 16), 5, 1, 4, 9, True, "float"),
     ((252, 260, 130), 3, 1, 3, 1, False, "half")])
 def test_sampled_sweeps_equal_the_fused_passes(shape, ntilts, block, fp, bp, masked, voxel):
     nx, ny, nz = shape
