@@ -545,6 +545,7 @@ private:
     bool sweepsPay(const MemberPlan& m, bool plain) const;
     void enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* ev) const;
     size_t splitLaunches() const;
+    bool sweepResidualNorm(double* scratch, hipStream_t stream) const;
 
     // An iteration as separate sweeps (blocks of several projections): per block
     // the back projections of the block before it, all in one sweep, then the
@@ -643,6 +644,22 @@ bool FusedEngineImpl::sweepsPay(const MemberPlan& m, bool plain) const
     return cu_work > (m.ny <= 256 ? 10000.0 : 13000.0);
 }
 
+dev::ForwardView forward_view(const BlockIterativeReconstructionOperator& op, uint32_t phys, float* residual,
+                              float* length)
+{
+    const ParallelScannerGeometry& g = op.geometry(phys);
+    dev::ForwardView f{};
+    g.ray_direction().store(f.ray);
+    g.source_base().store(f.source);
+    g.horizontal_pitch().store(f.h);
+    g.vertical_pitch().store(f.v);
+    f.measured = op.realProjection(phys);
+    f.measured_type = op.projectionType();
+    f.residual = residual;
+    f.length = length;
+    return f;
+}
+
 // The fused pass reads the volume once for a block's back and forward
 // projections, but works out every voxel's column and every ray's steps in
 // every plane: with several projections a pass it is bound by that (512 x 512 x
@@ -684,16 +701,8 @@ void FusedEngineImpl::plan_split(hipStream_t stream)
             for (uint32_t p = 0; p < bs; ++p) {
                 const uint32_t phys = op.getPhysicalProjectionIndex(b, p);
                 const ParallelScannerGeometry& g = op.geometry(phys);
-                dev::ForwardView f{};
-                g.ray_direction().store(f.ray);
+                dev::ForwardView f = forward_view(op, phys, image(parity, p, 0), image(parity, p, 1));
                 if ((f.ray[2] > 0.0f) != (zdir > 0)) continue;
-                g.source_base().store(f.source);
-                g.horizontal_pitch().store(f.h);
-                g.vertical_pitch().store(f.v);
-                f.measured = op.realProjection(phys);
-                f.measured_type = op.projectionType();
-                f.residual = image(parity, p, 0);
-                f.length = image(parity, p, 1);
                 f.loc_c = loc_c;
                 f.use_loc = m.use_loc ? 1 : 0;
                 if (!dev::forward_view_fits(slab, f, (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, m.mask != nullptr)) return;
@@ -998,10 +1007,70 @@ void FusedEngineImpl::enqueueIteration(hipStream_t stream)
     else enqueue(sched_, 0, sched_.launches.size(), stream, nullptr);
 }
 
+// ||A x - b||_2 of a swept reconstruction by forward sweeps of up to kSweepForward
+// projections (the fused passes keep an untuned tile here: 256^3, 41 tilts, 1.83 ms,
+// 1.14 tuned, 0.70 in sweeps).  False where a measured projection does not fit.
+bool FusedEngineImpl::sweepResidualNorm(double* scratch, hipStream_t stream) const
+{
+    const MemberPlan& m = members_[0];
+    BlockIterativeReconstructionOperator& op = *m.op;
+    const std::vector<uint32_t>& measured = op.measuredProjections();
+    constexpr size_t kChunk = dev::kSweepForward;
+    DeviceBuffer images(sizeof(float) * m.pixels * 2 * kChunk);
+    auto slot = [&](size_t k, int which) { return images.as<float>() + m.pixels * (2 * k + which); };
+    // chunk by chunk, the projections of one z direction after the other's
+    std::vector<dev::ForwardView> views;
+    std::vector<ForwardSweep> sweeps;
+    std::vector<size_t> chunk_end;     // sweeps of chunk c end at chunk_end[c]
+    for (size_t c0 = 0; c0 < measured.size(); c0 += kChunk) {
+        for (const int zdir : {-1, 1}) {
+            const size_t first = views.size();
+            for (size_t k = c0; k < std::min(measured.size(), c0 + kChunk); ++k) {
+                dev::ForwardView f = forward_view(op, measured[k], slot(k - c0, 0), slot(k - c0, 1));
+                if ((f.ray[2] > 0.0f) != (zdir > 0)) continue;
+                f.raw = 1;
+                if (!dev::forward_view_fits(split_slab_, f, (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, m.mask != nullptr))
+                    return false;
+                views.push_back(f);
+            }
+            if (views.size() > first) sweeps.push_back({(int)first, (int)(views.size() - first), zdir});
+        }
+        chunk_end.push_back(sweeps.size());
+    }
+    DeviceBuffer table(sizeof(dev::ForwardView) * std::max<size_t>(views.size(), 1));
+    ETN_HIP(hipMemcpyAsync(table.get(), views.data(), sizeof(dev::ForwardView) * views.size(), hipMemcpyHostToDevice,
+                           stream));
+    const void* volume = op.getReconstructedVolume()->data();
+    size_t at = 0;
+    for (size_t c = 0; c < chunk_end.size(); ++c) {
+        for (; at < chunk_end[c]; ++at)
+            dev::sweep_forward_project(split_slab_, table.as<dev::ForwardView>() + sweeps[at].first, sweeps[at].count,
+                                       sweeps[at].zdir, (uint32_t)m.nu, (uint32_t)m.nv, m.fp_n, vt_, volume, m.mask,
+                                       stream);
+        // squared differences in projection order, as the unfused norm adds them
+        const size_t c0 = c * kChunk;
+        for (size_t k = c0; k < std::min(measured.size(), c0 + kChunk); ++k)
+            dev::launch_sum_squared_difference(op.realProjection(measured[k]), op.projectionType(), slot(k - c0, 0),
+                                               m.pixels, scratch, scratch + dev::kSsdBlocks, stream);
+    }
+    ETN_HIP(hipStreamSynchronize(stream));   // the images and the table go
+    return true;
+}
+
 double FusedEngineImpl::residualNorm(size_t member, double* scratch, hipStream_t stream)
 {
     if (member >= members_.size()) fail("member index out of range");
     const MemberPlan& m = members_[member];
+    if (sweeps()) {
+        double* total = scratch + dev::kSsdBlocks;
+        ETN_HIP(hipMemsetAsync(total, 0, sizeof(double), stream));
+        if (sweepResidualNorm(scratch, stream)) {
+            double host = 0.0;
+            ETN_HIP(hipMemcpyAsync(&host, total, sizeof(double), hipMemcpyDeviceToHost, stream));
+            ETN_HIP(hipStreamSynchronize(stream));
+            return std::sqrt(host);
+        }
+    }
     BlockIterativeReconstructionOperator& op = *m.op;
     const std::vector<uint32_t>& measured = op.measuredProjections();
     const size_t M = members_.size();

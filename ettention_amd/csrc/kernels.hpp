@@ -80,7 +80,7 @@ void sweep_back_project(const SlabParams& s, const SweepGroups& g, const BackVie
                         uint32_t nv, etn_voxel_type vt, void* volume, hipStream_t stream);
 // One forward projection of sweep_forward_project (device table entries); the
 // residual measured - line integral (with long-object compensation when
-// use_loc) and the ray length are written.
+// use_loc), or the line integral itself (raw), and the ray length are written.
 struct ForwardView {
     float source[3], h[3], v[3], ray[3];
     const void* measured;       // nv x nu in measured_type
@@ -89,6 +89,7 @@ struct ForwardView {
     float* length;
     float loc_c;
     int use_loc;
+    int raw;
 };
 constexpr int kSweepForward = 8;    // projections of a sweep
 // Whether sweep_forward_project takes a projection (a plane per detector row,

@@ -963,6 +963,11 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
                 pv = l > kEpsilon ? pv * f.loc_c / l : 0.0f;
                 l = f.loc_c;
             }
+            if (f.raw) {
+                f.residual[i] = pv;
+                f.length[i] = l;
+                continue;
+            }
             float b;
             if (f.measured_type == ETN_VOXEL_FLOAT16) b = F16::load(static_cast<const __half*>(f.measured), i);
             else if (f.measured_type == ETN_VOXEL_BFLOAT16) b = BF16::load(static_cast<const uint16_t*>(f.measured), i);

@@ -264,8 +264,8 @@ etn_status etn_reconstruction_volume(etn_reconstruction* r, void** device_volume
 /* Replace the working volume (volume.initFile): device source of the same type and size. */
 etn_status etn_reconstruction_set_volume(etn_reconstruction* r, const void* device_volume);
 /* ||A x - b||_2 over every used projection, FP64 accumulation; synchronises.
- * On the fused path the forward projections run as forward-only fused passes
- * (bit-identical to the generic kernels' norm with exact arithmetic). */
+ * On the fused path the forward projections run as forward-only fused passes or
+ * sweeps, whichever the iterations take (bit-identical to the generic kernels' norm with exact arithmetic). */
 etn_status etn_reconstruction_residual_norm(etn_reconstruction* r, double* out);
 etn_status etn_reconstruction_synchronize(etn_reconstruction* r);
 /* 1 when the fused plane kernels run this reconstruction, 0 for the generic kernels. */

@@ -196,6 +196,28 @@ def test_time_kernels_tells_sweeps_from_fused_passes():
     assert r.time_kernels()[0] == FUSED
 
 
+# the residual norm of a swept reconstruction runs in forward sweeps (of up to 8
+# projections, both z directions in a chunk) and is the fused passes' bit for bit
+@pytest.mark.parametrize("shape,block,fp,masked,voxel", [((130, 131, 140), 8, 1, False, "float"), ((97, 96, 96), 9, 1, True, "half"),
+                                                         ((104, 80, 98), 2, 2, False, "bfloat16")])
+def test_residual_norm_of_sweeps(shape, block, fp, masked, voxel):
+    nx, ny, nz = shape
+    rng = np.random.default_rng(block)
+    case = dict(volume=E.VolumeGeometry.make(shape), base_geometry=E.ScannerGeometry.mrc_base(nx, ny),
+                tilt_angles=np.linspace(-150, 150, 21).astype(np.float32),
+                projections=torch.from_numpy(rng.normal(1.0, 0.3, (21, ny, nx)).astype(np.float32)).cuda(),
+                algorithm="blockiterative", block_size=block, lam=0.3, voxel_type=voxel, fp_samples=fp,
+                bp_samples=4 if fp > 1 else 1, skip_projections=(0, 7, 8), use_long_object_compensation=True)
+    if masked:
+        case["mask"] = torch.from_numpy(rng.integers(0, 256, (nz, ny, nx)).astype(np.uint8)).cuda()
+    r = A.BlockIterativeReconstructionOperator(**case)
+    r.run_iterations(1)
+    norm = r.residual_norm()
+    assert timed_kernel(case) == SWEEPING
+    r.set_tile(*r.tile())
+    assert norm == r.residual_norm() and norm > 0.0
+
+
 # which reconstructions are swept: sizes on both sides of the lines that
 # measurements drew (FusedEngineImpl::sweepsPay)
 @pytest.mark.parametrize("shape,block,voxel,fp,bp,masked,kernel", [
