@@ -56,7 +56,10 @@ __device__ __forceinline__ uint32_t gated(uint32_t pair, uint32_t act)
 // input row it starts at and serves every output row whose taps it holds:
 //   F1(r): taps dx = 0 and 1 of input row r,     used with dy = 0, 1, 2;
 //   F2(r): tap dx = 2 of input rows r and r + 1, used with dy = 0 and 1 (P)
-//          and, its first row weighted 0, with dy = 2 (Q).
+//          and with dy = 1 and 2 (Q).
+// The weight of dx = 2, dy = 1, which both hold, is halved in each (exact: a power
+// of two; a zero in one of them would turn an infinite voxel into NaN, and the ReLU
+// that into 0).
 // That is 5 steps per dz and output row (15 for the 27 taps, 0.9 of the
 // products wanted) and 7 LDS reads for 10 MFMAs; a step of four arbitrary taps
 // of 8 channels took one read per MFMA.  What bounds it besides the MFMAs is
@@ -587,11 +590,11 @@ __global__ void pack_weights_kernel(const float* w, int wci, int cin, int cout, 
     const int co = tile % (cout / 16) * 16 + (lane & 15), kg = lane >> 4;
     const int ci = tile / (cout / 16) * 16 + (kg & 1) * 8 + e;
     const int dz = frag / 5, f = frag % 5, second = kg >> 1;
-    // F1: row f, dx 0 or 1; P: dx 2, rows 0 and 1; Q: dx 2, row 2 from the second
-    const int dy = f < 3 ? f : f == 3 ? second : 2, dx = f < 3 ? second : 2;
+    // F1: row f, dx 0 or 1; P: dx 2, rows 0 and 1; Q: dx 2, rows 1 and 2
+    const int dy = f < 3 ? f : f - 3 + second, dx = f < 3 ? second : 2;
     const int tap = (dz * 3 + dy) * 3 + dx;
     float v = transposed ? w[((size_t)ci * 27 + (26 - tap)) * wci + co] : w[((size_t)co * 27 + tap) * wci + ci];
-    if (f == 4 && !second) v = 0.0f;
+    if (f >= 3 && dy == 1) v *= 0.5f;   // (in P and in Q)
     wt[i] = f2bf(v);
 }
 

@@ -71,6 +71,19 @@ def test_forward_matches_oracle(shape):
     assert err < 3e-2, err
 
 
+def test_infinite_activations_stay_infinite():
+    """One voxel whose first activations overflow, all weights positive: every
+    activation that sees it is +infinity (16^3 voxels: all of the prediction),
+    none NaN, which the ReLU would turn into 0."""
+    shape = (16, 16, 16)
+    params = np.full(Lrn.parameter_count(), 0.01, np.float32)
+    params[:16 * 27 * 2] = 100.0
+    x = np.zeros(shape, np.float32)
+    x[8, 8, 8] = 1e38
+    y = Lrn.CorrectionNet(shape, params).predict(torch.from_numpy(x).cuda(), None, 1.0)
+    assert bool((y == float("inf")).all())
+
+
 def test_scale_only_rescales():
     shape = (8, 8, 8)
     params, x, d, _ = setup_case(shape, 12)
