@@ -93,16 +93,16 @@ WeightedBackProjection::WeightedBackProjection(const etn_reconstruction_desc& d,
     taps_.allocate(k.size() * sizeof(float));
     ETN_HIP(hipMemcpyAsync(taps_.get(), k.data(), taps_.bytes(), hipMemcpyHostToDevice, stream_));
     ETN_HIP(hipStreamSynchronize(stream_));
+    slots_ = chunkSize();
     if ((d.flags & (ETN_RECON_FLAG_GENERIC_KERNELS | ETN_RECON_FLAG_EXACT_ARITHMETIC)) == 0) {
         // the sweep takes every projection or none; the whole volume is one slab
         const uint32_t samples = d.bp_samples ? d.bp_samples : 1;
         std::vector<dev::BackView> views(geometries_.size());
         const VolumeProperties whole = wholeVolume();
         bool sweep = samples == 1 && (d.flags & ETN_RECON_FLAG_LDS_BACK_PROJECTION) == 0;
-        const uint32_t slots = std::min(count_, kChunk);
-        if (sweep) chunk_.allocate(sizeof(float) * 2 * pixels_ * slots);
+        if (sweep) chunk_.allocate(sizeof(float) * 2 * pixels_ * slots_);
         for (size_t i = 0; sweep && i < views.size(); ++i) {
-            const float* image = chunk_.as<float>() + 2 * pixels_ * (i % kChunk);
+            const float* image = chunk_.as<float>() + 2 * pixels_ * (i % slots_);
             sweep = dev::make_back_view(make_slab_params(whole, 0),
                                         make_bp_params(geometries_[i], whole, samples, lambda_ / (float)count_), image,
                                         image + pixels_, &views[i]);
@@ -164,6 +164,12 @@ VolumeProperties WeightedBackProjection::wholeVolume() const
     return VolumeProperties(g);
 }
 
+uint32_t WeightedBackProjection::chunkSize() const
+{
+    const size_t fit = kChunkBytes / (sizeof(float) * 2 * pixels_);
+    return std::max(1u, std::min(count_, (uint32_t)std::min<size_t>(kChunk, std::max<size_t>(fit, 8))));
+}
+
 // Filtered images and ray lengths of projections first .. first + count - 1
 // into the slots of chunk_, one launch each (one launch per image had cost 13
 // and 4 us each, most of it launch and ramp-up).
@@ -185,11 +191,11 @@ void WeightedBackProjection::runNiterations(uint32_t n)
 {
     if (n > count_) fail("WBP: more projections requested than the stack holds");
     if (views_.get()) {
-        // filtered images and ray lengths of up to kChunk projections, then
+        // filtered images and ray lengths of a chunk of projections, then
         // their back projections in stack order in one sweep of the volume
         const dev::SlabParams slab = make_slab_params(wholeVolume(), 0);
-        for (uint32_t i0 = 0; i0 < n; i0 += kChunk) {
-            const uint32_t k = std::min(n - i0, kChunk);
+        for (uint32_t i0 = 0; i0 < n; i0 += slots_) {
+            const uint32_t k = std::min(n - i0, slots_);
             filterChunk(i0, k);
             hipEvent_t ev[2] = {nullptr, nullptr};
             if (launch_ms_) {
@@ -211,11 +217,11 @@ void WeightedBackProjection::runNiterations(uint32_t n)
     }
     if (fused_) {
         // the same chunks, eight projections per volume sweep
-        if (!chunk_.get()) chunk_.allocate(sizeof(float) * 2 * pixels_ * std::min(count_, kChunk));
-        for (uint32_t i0 = 0; i0 < n; i0 += kChunk) {
+        if (!chunk_.get()) chunk_.allocate(sizeof(float) * 2 * pixels_ * slots_);
+        for (uint32_t i0 = 0; i0 < n; i0 += slots_) {
             std::vector<uint32_t> idx;
             std::vector<const float*> res, len;
-            const uint32_t i1 = std::min(n, i0 + kChunk);
+            const uint32_t i1 = std::min(n, i0 + slots_);
             filterChunk(i0, i1 - i0);
             for (uint32_t i = i0; i < i1; ++i) {
                 float* f = chunk_.as<float>() + 2 * pixels_ * (i - i0);

@@ -30,8 +30,8 @@ public:
     GpuVolume* getReconstructedVolume() override { return volume_.get(); }
     void synchronize() override;
     hipStream_t stream() const override { return stream_; }
-    // Single-axis tilt geometries back-project up to kChunk projections per
-    // volume sweep, or on the fused kernels eight (oversampled, the LDS back
+    // Single-axis tilt geometries back-project a chunk of up to kChunk projections
+    // per volume sweep, or on the fused kernels eight (oversampled, the LDS back
     // projection), with fast arithmetic, unless the generic kernels or exact
     // arithmetic are asked for.
     bool usesFusedPath() const override { return fused_ != nullptr || views_.get() != nullptr; }
@@ -50,7 +50,12 @@ public:
     void filter(const float* src, float* dst);
 
 private:
+    // Projections of a chunk: their filtered images and ray lengths stay allocated
+    // with the object, within kChunkBytes as long as that holds eight (64 of 1024^2,
+    // 16 of 2048^2, 8 of 4096^2: 1 GiB).
     static constexpr uint32_t kChunk = 64;
+    static constexpr size_t kChunkBytes = (size_t)512 << 20;
+    uint32_t chunkSize() const;
     void filterChunk(uint32_t first, uint32_t count);
     VolumeProperties wholeVolume() const;
 
@@ -74,7 +79,8 @@ private:
     DeviceBuffer rays_;   // fused paths: every projection's ray geometry, for the batched ray lengths
     DeviceBuffer views_;  // sweep path: every projection's table entry (its images: a slot of chunk_)
     dev::SweepGroups groups_;
-    DeviceBuffer chunk_;  // filtered images and ray lengths of up to kChunk projections
+    uint32_t slots_ = 0;  // projections of a chunk
+    DeviceBuffer chunk_;  // their filtered images and ray lengths
     std::vector<float>* launch_ms_ = nullptr;    // set while timeKernels runs
 };
 

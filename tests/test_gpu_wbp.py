@@ -184,3 +184,23 @@ def test_wbp_sweep_matches_the_other_paths(size, det, count, voxel):
         np.testing.assert_array_equal(vols["sweep"], vols["lds"])
     if voxel == "float":
         assert rel_l2(vols["sweep"], vols["generic"]) < 1e-6
+
+
+def test_wbp_keeps_a_bounded_chunk():
+    """The filtered images that stay allocated between runs: 16 of 2048^2 (512 MiB),
+    so 20 projections take two sweeps; the volume is the LDS path's bit for bit."""
+    count, size = 20, (64, 8, 8)
+    projs = torch.rand((count, 2048, 2048), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+    args = dict(volume=E.VolumeGeometry.make(size), base_geometry=E.ScannerGeometry.mrc_base(2048, 2048),
+                tilt_angles=np.linspace(-60.0, 60.0, count).astype(np.float32), projections=projs, lam=1.0)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    r = A.WeightedBackProjection(**args)
+    r.run()
+    r.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 640 << 20
+    got = r.get_reconstructed_volume().cpu().numpy()
+    assert r.time_kernels()[::2] == (3, 2)
+    r = A.WeightedBackProjection(flags=E.ETN_RECON_FLAG_LDS_BACK_PROJECTION, **args)
+    r.run()
+    np.testing.assert_array_equal(got, r.get_reconstructed_volume().cpu().numpy())
