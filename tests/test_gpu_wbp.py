@@ -204,3 +204,12 @@ def test_wbp_keeps_a_bounded_chunk():
     r = A.WeightedBackProjection(flags=E.ETN_RECON_FLAG_LDS_BACK_PROJECTION, **args)
     r.run()
     np.testing.assert_array_equal(got, r.get_reconstructed_volume().cpu().numpy())
+
+
+@pytest.mark.parametrize("size,count,kernel", [((32, 32, 32), 41, 0), ((32, 32, 32), 40, 3), ((24, 24, 24), 64, 3),
+                                               ((16, 16, 16), 64, 0), ((32, 16, 36), 64, 3), ((36, 16, 32), 64, 3)])
+def test_wbp_of_small_volumes_takes_the_faster_path(size, count, kernel):
+    r = A.WeightedBackProjection(volume=E.VolumeGeometry.make(size), base_geometry=E.ScannerGeometry.mrc_base(*size[:2]),
+                                 tilt_angles=np.linspace(-60.0, 60.0, count).astype(np.float32),
+                                 projections=torch.ones((count, size[1], size[0]), device="cuda"), lam=1.0)
+    assert r.time_kernels()[0] == kernel
