@@ -317,13 +317,28 @@ bool plane_geometry_fits(const SlabParams& s, const RayParams& r, int sub = 1)
     if (!(size > 0.5f)) return false;   // (a unit vector without y) the larger of x and z bounds the times
     const float inv = -FLT_MAX;
     const float sd = 1.0f / (float)sub, off = sd / 2.0f;
-    for (uint32_t y = 0; y < r.nv * (uint32_t)sub; ++y) {
+    const uint32_t rows = r.nv * (uint32_t)sub;
+    auto source_y = [&](uint32_t y) {
         const float fy = (float)(y / sub) + off + sd * (float)(y % sub);
         const float rv = r.v[1] * fy;
-        const float src = r.source[1] + 0.0f + rv;
-        const float t0 = (s.bmin[1] - src) * inv, t1 = (s.bmax[1] - src) * inv;
-        const float lo = std::fmin(t0, t1), hi = std::fmax(t0, t1);
-        if (!((lo < -1e30f && hi > 1e30f) || hi < -1e30f || lo > 1e30f)) return false;
+        return r.source[1] + 0.0f + rv;
+    };
+    if (!std::isfinite(source_y(0)) || !std::isfinite(source_y(rows - 1))) return false;
+    // a row's source moves one way with the row (each operation rounds
+    // monotonically), so if any row lies too near a face of the box, the first, the
+    // last or one beside the face does
+    for (const float face : {s.bmin[1], s.bmax[1]}) {
+        const bool above = face - source_y(0) > 0.0f;
+        uint32_t lo = 0, hi = rows;     // first row on the other side of the face than row 0
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) / 2;
+            if ((face - source_y(mid) > 0.0f) == above) lo = mid + 1;
+            else hi = mid;
+        }
+        for (const uint32_t y : {0u, lo > 0 ? lo - 1 : 0u, std::min(lo, rows - 1), rows - 1}) {
+            const float t = (face - source_y(y)) * inv;
+            if (!(std::fabs(t) > 1e30f)) return false;
+        }
     }
     return true;
 }

@@ -85,3 +85,18 @@ def test_slabs_add_up(subvolumes):
         O.forward_project(ov, vol, og, slab=i, proj=op, length=ol)
     np.testing.assert_array_equal(p.cpu().numpy(), op)
     np.testing.assert_array_equal(l.cpu().numpy(), ol)
+
+
+# rows whose rays run along a face of the volume (not this path's): the first and
+# the last one, ones in between, one of a coarser detector, none
+@pytest.mark.parametrize("nv,pitch", [(7, 1.0), (9, 1.0), (4, 2.0), (13, 0.5), (8, 1.0)])
+def test_rows_on_a_face_equal_the_oracle(nv, pitch):
+    size = (48, 6, 40)
+    vg, ov, g, og, rng = case(size, (48, nv), (1.0, pitch), 25.0, 6)
+    vol = rng.uniform(0, 1, size[::-1]).astype(np.float32)
+    p = torch.zeros((nv, 48), device="cuda")
+    l = torch.zeros_like(p)
+    A.forward_project(vg, torch.from_numpy(vol).cuda(), g, p, l)
+    op, ol = O.forward_project(ov, vol, og)
+    np.testing.assert_array_equal(p.cpu().numpy(), op)
+    np.testing.assert_array_equal(l.cpu().numpy(), ol)
