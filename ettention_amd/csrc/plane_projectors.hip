@@ -280,12 +280,18 @@ void launch_forward_cols(const SlabParams& s, const RayParams& r, const void* vo
         plane_forward_kernel<S, kVec, P, 4><<<grid, kFpThreads, 0, stream>>>(s, r, v, proj, len, band);
 }
 
+// rows read four voxels at a time
+bool vector_rows(const SlabParams& s, const void* vol, size_t voxel)
+{
+    return s.res[0] % 4 == 0 && s.nx % 4 == 0 && reinterpret_cast<uintptr_t>(vol) % (4 * voxel) == 0;
+}
+
 template <typename S>
 void launch_forward_typed(const SlabParams& s, const RayParams& r, const void* vol, float* proj, float* len,
                           hipStream_t stream)
 {
     const int nx = s.res[0];
-    const bool vec = nx % 4 == 0 && s.nx % 4 == 0 && reinterpret_cast<uintptr_t>(vol) % (4 * sizeof(typename S::T)) == 0;
+    const bool vec = vector_rows(s, vol, sizeof(typename S::T));
     // two rows a workgroup halve the steps' instructions; one row gives twice
     // the workgroups, where two would not reach every CU (256 of them)
     const bool two = r.nv >= 512 && nx * 2 <= kFpLds;
@@ -1280,6 +1286,19 @@ bool plane_forward_project(const SlabParams& s, const RayParams& r, etn_voxel_ty
                            float* projection, float* traversal_length, hipStream_t stream)
 {
     if (!plane_forward_fits(s, r)) return false;
+    // A row's whole plane is staged however few rays cross it: us for the planes
+    // (less a voxel where several rows share one) and for one ray after another's
+    // steps on the generic kernel, which also slows down with the rays in flight.
+    // Staged / generic: 1000^3 10 columns 590 / 521, 32 columns 590 / 653; 850^3
+    // (single voxels) 64 columns 687 / 582, 128 columns 691 / 665; 1000 x 128 x 1000
+    // 128 columns x 2048 rows 838 / 571; 700^3 10 columns 254 / 358
+    const size_t voxel = vt == ETN_VOXEL_FLOAT32 ? 4 : 2;
+    const double rate = !vector_rows(s, volume, voxel) ? 1.12e-6
+                        : r.nv >= 2u * (uint32_t)s.res[1] ? 0.42e-6
+                        : voxel == 4 ? 0.59e-6 : 0.36e-6;
+    const double staged = rate * r.nv * s.res[0] * s.res[2];
+    const double rays = (double)r.nu * std::min(r.nv, (uint32_t)s.res[1]);
+    if (staged > 0.25 * (s.res[0] + s.res[2]) * (1.0 + rays * 1e-5)) return false;
     if (vt == ETN_VOXEL_FLOAT16) launch_forward_typed<F16>(s, r, volume, projection, traversal_length, stream);
     else if (vt == ETN_VOXEL_BFLOAT16) launch_forward_typed<BF16>(s, r, volume, projection, traversal_length, stream);
     else launch_forward_typed<F32>(s, r, volume, projection, traversal_length, stream);
