@@ -100,3 +100,11 @@ def test_rows_on_a_face_equal_the_oracle(nv, pitch):
     op, ol = O.forward_project(ov, vol, og)
     np.testing.assert_array_equal(p.cpu().numpy(), op)
     np.testing.assert_array_equal(l.cpu().numpy(), ol)
+
+
+# workgroups of 256, 128 and 64 columns (one, two and four rows of waves for the
+# slices), one column more than those, fewer slices than waves
+@pytest.mark.parametrize("nx", [64, 65, 128, 129, 192, 193, 256, 257, 260, 320, 321])
+@pytest.mark.parametrize("nz,tilt,dtype", [(3, 10.0, "float"), (37, 60.0, "bfloat16"), (130, -35.0, "half")])
+def test_back_of_every_row_width_equals_the_oracle(nx, nz, tilt, dtype):
+    test_back_equals_the_oracle((nx, 5, nz), (nx, 5), (1.0, 1.0), tilt, dtype)
