@@ -157,9 +157,9 @@ def test_wbp_register_back_projection_equals_lds():
 
 
 # blocks as separate sweeps (the default) against the fused passes on the LDS
-# back projection: nx off a multiple of 4, rows beside the volume, one, two and
-# four planes a workgroup, several rays a thread, both z directions, more
-# projections in a block than in a sweep
+# back projection: nx off a multiple of 4, one and two planes a workgroup, both z
+# directions, more projections in a block than in a sweep (other detectors, four
+# planes and several rays a thread: test_gpu_sweep_geometries.py)
 SWEEPS = [((135, 131, 120), 23, 8, 60.0, "float"), ((64, 522, 64), 9, 9, 60.0, "float"), ((300, 160, 180), 9, 4, 60.0, "float"),
           ((520, 70, 64), 19, 8, 60.0, "bfloat16"), ((136, 130, 120), 40, 0, 60.0, "half"), ((130, 130, 128), 30, 12, 150.0, "float")]
 
