@@ -812,7 +812,8 @@ size_t wgrad_partial_floats(int D, int H, int W, int cin, int cout)
 void conv3_weight_grad(const ConvSrc& src, int D, int H, int W, const uint16_t* gy, int cin, int cout, float* partial,
                        float* dw, float* db, hipStream_t stream)
 {
-    if (cout % 16 || cout > kMaxCout || cout == 48 || src.ca % 8 || src.cb % 8 || cin > src.ca + src.cb)
+    // (16 input channels a workgroup, all of them from a or from b)
+    if (cout % 16 || cout > kMaxCout || cout == 48 || src.ca % (src.cb ? 16 : 8) || src.cb % 8 || cin > src.ca + src.cb)
         fail("conv3 weight gradient: channel counts");
     const int cin16 = (src.ca + src.cb + 15) / 16 * 16, chunks = wgrad_chunks(D, H, W, src.ca + src.cb);
     const int nbx = (W + kWX - 1) / kWX, nby = (H + kWY - 1) / kWY, nbz = (D + kWZ - 1) / kWZ;
