@@ -1,5 +1,5 @@
 // Device-side building blocks of the projectors: storage conversion, the DDA
-// ray traversal and the software bilinear lookup.  Every file including this
+// ray traversal and the fract of the bilinear lookups.  Every file including this
 // is compiled with -ffp-contract=off: the expressions below round exactly as
 // the OpenCL C source of the reference writes them, so the traversal takes
 // the same voxel sequence and the same segment lengths.
@@ -171,7 +171,7 @@ __device__ __forceinline__ DdaConst dda_const(const float ray[3], const float vs
     return c;
 }
 
-// Traversal state of one ray; suspends at band boundaries and resumes.
+// Traversal state of one ray.
 struct DdaRay {
     int vox[3];
     float res[3];
@@ -219,44 +219,6 @@ __device__ __forceinline__ void dda_begin(const SlabParams& s, const DdaConst& c
     }
 }
 
-// Advances the ray while its voxel lies inside the subvolume and its z index
-// inside [zlo, zhi).  `sample(x, y, z, &value, &maskv)` reads the voxel.  The
-// loop condition is the reference's (in range, then ++breakVar < 4096, with a
-// second ++breakVar in the body: at most 2048 steps); a ray that leaves the
-// band with its condition not yet evaluated resumes unchanged.
-template <typename Sampler>
-__device__ __forceinline__ void dda_advance(const SlabParams& s, const DdaConst& c, DdaRay& r, int zlo, int zhi,
-                                            const Sampler& sample)
-{
-    while (r.live) {
-        if (!(r.vox[0] >= 0 && r.vox[1] >= 0 && r.vox[2] >= 0 && r.vox[0] < s.res[0] && r.vox[1] < s.res[1] &&
-              r.vox[2] < s.res[2])) {
-            r.live = 0;
-            break;
-        }
-        if (r.vox[2] < zlo || r.vox[2] >= zhi) break;
-        if (!(++r.brk < 4096u)) {
-            r.live = 0;
-            break;
-        }
-        const float dt = fminf(fminf(r.res[0], r.res[1]), r.res[2]);
-        float value, maskv;
-        sample(r.vox[0], r.vox[1], r.vox[2], value, maskv);
-        r.acc += dt * value;
-        r.accl += dt * maskv;
-        const int ix = (r.res[0] <= r.res[1] && r.res[0] <= r.res[2]) ? 1 : 0;
-        const int iy = (r.res[1] < r.res[0] && r.res[1] <= r.res[2]) ? 1 : 0;
-        const int iz = (r.res[2] < r.res[0] && r.res[2] < r.res[1]) ? 1 : 0;
-        r.res[0] = ix ? c.step[0] : r.res[0] - dt;
-        r.res[1] = iy ? c.step[1] : r.res[1] - dt;
-        r.res[2] = iz ? c.step[2] : r.res[2] - dt;
-        r.vox[0] += ix * c.sign[0];
-        r.vox[1] += iy * c.sign[1];
-        r.vox[2] += iz * c.sign[2];
-        ++r.brk;
-    }
-}
-
 // Sub-ray origin (ParallelBeamsForwardProjection.cl:12-24).
 __device__ __forceinline__ void fp_ray_source(const RayParams& g, uint32_t x, uint32_t y, uint32_t si, uint32_t sj,
                                               float sd, float off, float src[3])
@@ -270,66 +232,12 @@ __device__ __forceinline__ void fp_ray_source(const RayParams& g, uint32_t x, ui
     }
 }
 
-// ---- bilinear lookup with zero border (ocl_src/ImageHandler.hl:20-40) ------
+// ---- fract of the bilinear lookups (ocl_src/ImageHandler.hl:20-29) ----------
 __device__ __forceinline__ float cl_fract(float x, float* base)
 {
     const float fl = floorf(x);
     *base = fl;
     return fminf(x - fl, 0x1.fffffep-1f);
-}
-__device__ __forceinline__ float lerp_row(const float* row, int n, float c)
-{
-    float b;
-    const float t = cl_fract(c - 0.5f, &b);
-    const int i0 = (int)b, i1 = i0 + 1;
-    const float v0 = (i0 >= 0 && i0 < n) ? row[i0] : 0.0f;
-    const float v1 = (i1 >= 0 && i1 < n) ? row[i1] : 0.0f;
-    return v0 + (v1 - v0) * t;
-}
-__device__ __forceinline__ float bilinear(const float* img, int nu, int nv, float cx, float cy)
-{
-    float b;
-    const float t = cl_fract(cy - 0.5f, &b);
-    const int j0 = (int)b, j1 = j0 + 1;
-    const float v0 = (j0 >= 0 && j0 < nv) ? lerp_row(img + (size_t)j0 * nu, nu, cx) : 0.0f;
-    const float v1 = (j1 >= 0 && j1 < nv) ? lerp_row(img + (size_t)j1 * nu, nu, cx) : 0.0f;
-    return v0 + (v1 - v0) * t;
-}
-
-// Detector coordinate of a point (TransformCoordG, Matrix4x4.hl:38-58).
-__device__ __forceinline__ void project_point(const float* m, const float p[3], float& u, float& v)
-{
-    float r[4];
-    for (int row = 0; row < 4; ++row) {
-        float a = m[0 * 4 + row] * p[0] + m[1 * 4 + row] * p[1];
-        a = a + m[2 * 4 + row] * p[2];
-        r[row] = a + m[3 * 4 + row] * 1.0f;
-    }
-    u = r[0] / r[3];
-    v = r[1] / r[3];
-}
-
-// One voxel's correction: the sample loop of ParallelBeamsBackProjection.cl:26-44.
-// Returns the used-sample count; *sum receives the summed contributions.
-__device__ __forceinline__ uint32_t bp_voxel_sum(const BpParams& b, const float center[3], const float* residual,
-                                                 const float* ray_length, float* sum)
-{
-    float acc = 0.0f;
-    uint32_t used = 0;
-    for (uint32_t si = 0; si < b.nsamples; ++si) {
-        const float4 smp = b.samples[si];
-        const float p[3] = {center[0] + smp.x, center[1] + smp.y, center[2] + smp.z};
-        float u, v;
-        project_point(b.m, p, u, v);
-        const float L = bilinear(ray_length, (int)b.nu, (int)b.nv, u, v);
-        const float R = bilinear(residual, (int)b.nu, (int)b.nv, u, v);
-        const float w = smp.w / L;
-        const float contrib = R * b.lambda * w;
-        acc += (L > kEpsilon) ? contrib : 0.0f;
-        used += (L > kEpsilon) ? 1u : 0u;
-    }
-    *sum = acc;
-    return used;
 }
 
 }  // namespace dev

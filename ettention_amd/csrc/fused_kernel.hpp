@@ -964,7 +964,7 @@ __global__ void __launch_bounds__(kThreads, kRes == 2 || kRes == 3 ? 2
                                     L = fmaf(c.w, tx, c.z);
                                     contrib = Rv * lw * __builtin_amdgcn_rcpf(L);
                                 } else {
-                                    // bp_voxel_sum's bilinear lookups and weight, operation for operation
+                                    // the generic kernel's bilinear lookups and weight, operation for operation
                                     float bu;
                                     const float tx = cl_fract(u - 0.5f, &bu);
                                     const int k = padded_index((int)bu, nu);

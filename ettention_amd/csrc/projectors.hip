@@ -58,8 +58,10 @@ __global__ void __launch_bounds__(256) forward_project_kernel(SlabParams s, RayP
             float src[3];
             fp_ray_source(g, x, y, k / n, k % n, sd, off, src);
             dda_begin(s, c, src, r);
-            // the loop's condition as the steps left on each axis until the ray
-            // leaves the volume, and 2048 in all (dda_advance)
+            // the reference's loop condition (voxel in range, then ++breakVar < 4096,
+            // with a second ++breakVar in the body: at most 2048 steps,
+            // DDARaytracer.hl:20-110) as the steps left on each axis until the ray
+            // leaves the volume, and in all
             uint32_t left = r.live ? 2048u : 0u;
             int lx = c.sign[0] > 0 ? s.res[0] - r.vox[0] : c.sign[0] < 0 ? r.vox[0] + 1 : 0x7fffffff;
             int ly = c.sign[1] > 0 ? s.res[1] - r.vox[1] : c.sign[1] < 0 ? r.vox[1] + 1 : 0x7fffffff;
@@ -124,7 +126,8 @@ __global__ void __launch_bounds__(256) forward_project_kernel(SlabParams s, RayP
     len[i] += accl / total;
 }
 
-// ParallelBeamsBackProjection.cl:correct for kBpDepth voxels of a column: the
+// ParallelBeamsBackProjection.cl:correct for kBpDepth voxels of a column (its
+// sample loop, :26-44: a sample with a ray length up to 1e-4 is not used): the
 // x and y terms of the projected point serve all of them, and their image reads
 // are in flight together.  kUnit: the matrix's last row is (0, 0, 0, 1), so that
 // u and v are divided by exactly 1.  Residual and ray length are looked up at
@@ -159,7 +162,8 @@ __global__ void __launch_bounds__(256) back_project_kernel(SlabParams s, BpParam
     for (uint32_t si = 0; si < b.nsamples; ++si) {
         const float4 smp = b.samples[si];
         const float px = cx + smp.x, py = cy + smp.y;
-        // project_point's rows, their x and y terms first
+        // detector coordinates (TransformCoordG, Matrix4x4.hl:38-58): the x and y
+        // terms of the rows first
         const float ux = b.m[0] * px + b.m[4] * py, vx = b.m[1] * px + b.m[5] * py, wx = b.m[3] * px + b.m[7] * py;
 #pragma unroll
         for (int d = 0; d < kBpDepth; ++d) {
@@ -173,7 +177,7 @@ __global__ void __launch_bounds__(256) back_project_kernel(SlabParams s, BpParam
                 u = u / w;
                 v = v / w;
             }
-            // bilinear() of both images
+            // bilinear lookups with a zero border in both images (ImageHandler.hl:20-40)
             float bu, bv;
             const float tx = cl_fract(u - 0.5f, &bu), ty = cl_fract(v - 0.5f, &bv);
             const int i = (int)bu, j = (int)bv;
