@@ -204,7 +204,8 @@ enum {
     ETN_RECON_FLAG_LDS_BACK_PROJECTION = 1u << 6 /* fast fused kernels: apply the back projections to the band in
                                                    LDS, one projection after another, instead of in registers as
                                                    the band arrives from HBM (the default where it applies: nx a
-                                                   multiple of 4, no oversampling).  Same volumes bit for bit;
+                                                   multiple of 4, no oversampling), and no separate sweeps.
+                                                   Same volumes bit for bit;
                                                    for comparison and measurement */
 };
 
@@ -286,7 +287,11 @@ etn_status etn_reconstruction_time_kernels(etn_reconstruction* r, int* kernel, d
  * planes per workgroup and z rows per LDS band.  The first run times the
  * candidate tiles on the reconstruction's own data unless
  * ETN_RECON_FLAG_NO_AUTOTUNE is set; setting a tile skips that.  Tiles never
- * change results.  ETN_ERROR_UNSUPPORTED on the generic path,
+ * change results.  Reconstructions that run as separate sweeps (time_kernels
+ * reports 3) use no tile and tune none: tile() then reports the default one, and
+ * setting a tile, also that one, moves the reconstruction from the sweeps to the
+ * fused passes for good (the same volumes, slower).
+ * ETN_ERROR_UNSUPPORTED on the generic path,
  * ETN_ERROR_INVALID_ARGUMENT for a tile that does not fit (planes must be
  * 1, 2, 4 or 8 and divide ny; band and detector rows must fit the LDS array
  * of the workgroup shape: 64 KiB at 512 threads, 40 KiB at 256). */
@@ -296,7 +301,7 @@ etn_status etn_reconstruction_tile(etn_reconstruction* r, int* planes, int* band
  * kernels, 512 (two workgroups per CU) or 256 (four per CU, half the band).
  * The autotuner chooses it with the tile; setting it skips the autotuner, and
  * a tile that no longer fits reverts to the default tile.  Never changes
- * results.  ETN_ERROR_UNSUPPORTED on the generic path,
+ * results; leaves the sweeps as set_tile does.  ETN_ERROR_UNSUPPORTED on the generic path,
  * ETN_ERROR_INVALID_ARGUMENT for another size or one the volume does not fit. */
 etn_status etn_reconstruction_set_workgroup_threads(etn_reconstruction* r, int threads);
 etn_status etn_reconstruction_workgroup_threads(etn_reconstruction* r, int* threads);
