@@ -199,8 +199,9 @@ std::vector<Tile> candidate_tiles(const MemberPlan& m)
 // The fused kernels sweep the whole volume.  A z-slab split
 // (hardware.subVolumeCount) restarts the reference's forward projection at
 // every slab face and sums the slab parts; sweeping the volume in one pass
-// takes the same steps and only regroups those sums and the voxel-centre
-// arithmetic, so it is allowed with fast arithmetic and left to the generic
+// regroups those sums and the voxel-centre arithmetic, and a ray that a restart
+// at a face would round into the neighbouring voxel keeps its steps, as on the
+// whole volume.  So it is allowed with fast arithmetic and left to the generic
 // kernels with exact arithmetic.
 VolumeProperties whole_volume(const VolumeProperties& vp)
 {

@@ -523,8 +523,9 @@ BackTile plane_back_tile(const SlabParams& s, const BpParams& b)
 // shared and 3 instructions per update and plane remain.
 // A projection's columns (the 64 x 64 tile reaches at most 97 at unit pitch) are
 // loaded while the one before it is applied and staged in alternating buffers.
-// Bound by VALU issue: 0.071 ms a projection at 512^3 on the fused kernels (eight
-// a sweep), 0.039 here (the VALU's issue time is 0.032).
+// Bound by VALU issue (busy 0.67 of the time by its counter) and the record reads
+// together: 0.071 ms a projection at 512^3 on the fused kernels (eight a sweep),
+// 0.037 to 0.039 here.
 constexpr int kSweepThreads = 256;
 constexpr int kSweepPlanes = 4;
 constexpr int kSweepDepth = 16;      // slices a wave
@@ -741,8 +742,8 @@ __global__ void __launch_bounds__(kSweepThreads, 3)
 // plane takes 12.  kMask: the ray length sums the voxels' mask weights, staged
 // behind the P values of a voxel.  The columns are spread over several
 // workgroups (slices), which read the same planes on the same XCD.  512 x 512 x
-// 256, eight projections: 0.17 ms, of which the steps' VALU issue is 0.09; 250 x
-// 300 x 150 bf16 with a mask and 4 x 4 sub-rays: 0.042 ms (0.055 with an index
+// 256, eight projections: 0.17 ms, VALU busy 0.54 of it, LDS bank conflicts 0.36;
+// 250 x 300 x 150 bf16 with a mask and 4 x 4 sub-rays: 0.042 ms (0.055 with an index
 // division for every staged voxel; reads of four steps in flight gained nothing).
 template <bool kMask, int P>
 struct SweepRay {
@@ -1071,7 +1072,7 @@ void sweep_forward_typed(const SlabParams& s, const SweepForward& a, const void*
 // sample's u does not depend on its pattern row, which only moves it along y, nor
 // on the plane: the columns and weights of a pattern row's PD samples are worked
 // out once for all PD rows of all four planes, so a sample costs its record read
-// and 9 instruction slots (19 on the fused kernels, which also leave CUs idle
+// and 10 instruction slots (19 on the fused kernels, which also leave CUs idle
 // where the planes are no multiple of them).  A workgroup owns four planes x 64
 // columns x 4 kSampleDepth slices in registers.  250 x 300 x 150 bf16 with a mask,
 // 3 x 3 samples: 0.068 ms, with the forward sweep 0.110 where a fused pass takes

@@ -269,7 +269,8 @@ etn_status etn_reconstruction_set_volume(etn_reconstruction* r, const void* devi
  * sweeps, whichever the iterations take (bit-identical to the generic kernels' norm with exact arithmetic). */
 etn_status etn_reconstruction_residual_norm(etn_reconstruction* r, double* out);
 etn_status etn_reconstruction_synchronize(etn_reconstruction* r);
-/* 1 when the fused plane kernels run this reconstruction, 0 for the generic kernels. */
+/* 1 when the fused plane kernels or the separate sweeps run this reconstruction, 0
+ * for the generic kernels. */
 etn_status etn_reconstruction_uses_fused_path(etn_reconstruction* r, int* out);
 /* Extension (profiling; the reference's CL-event PerformanceReport,
  * CLAbstractionLayer.cpp:295-329): runs ONE more iteration eagerly with HIP
