@@ -543,7 +543,11 @@ private:
     void tuneTiles(hipStream_t stream);
     float timeSchedule(const Schedule& s, hipStream_t stream) const;
     void plan_split(hipStream_t stream);
-    bool sweepsPay(const MemberPlan& m, bool plain) const;
+    struct SplitCost {
+        double passes, sweeps;
+    };
+    SplitCost splitCost(const MemberPlan& m) const;
+    bool sweepsPay(const MemberPlan& m) const;
     void enqueueSplit(hipStream_t stream, std::vector<hipEvent_t>* ev) const;
     size_t splitLaunches() const;
     bool sweepResidualNorm(double* scratch, hipStream_t stream) const;
@@ -592,17 +596,92 @@ FusedEngineImpl::FusedEngineImpl(std::vector<MemberPlan> members, etn_voxel_type
     plan_split(stream);
 }
 
+// Microseconds of an iteration as fused passes and as sweeps: what each path's
+// kernels do, at rates fitted to 730 reconstructions of 24 to 1100 columns, rows and
+// slices and 0.3 to 70 million voxels, and 350 at chosen sizes, each measured both
+// ways (31 projections in blocks of 1 to 31; the fits scatter by 12 to 20%).
+FusedEngineImpl::SplitCost FusedEngineImpl::splitCost(const MemberPlan& m) const
+{
+    const double n = (double)m.op->measuredProjections().size(), B = std::min((double)m.bmax, n), blocks = std::ceil(n / B);
+    const double nx = m.nx, ny = m.ny, nz = m.nz, samples = m.bp_samples, mega = 1e-6 * nx * ny * nz;
+    const bool mask = m.mask != nullptr, sampled = over_ || mask;
+    SplitCost c;
+
+    // A fused pass lasts as long as a CU's planes, a workgroup each: voxels' columns
+    // worked out in every plane for every projection (cheaper where a thread keeps
+    // one x), rays' steps.  More planes than CUs overlap by a third.
+    const double cu_planes = 1.0 + 0.7 * std::max(0.0, ny / 256.0 - 1.0), plane = nx * nz * cu_planes;
+    const int max_fp = std::max(1, std::min(dev::kMaxFusedFp, dev::kMaxThreads * dev::kMaxRaysPerThread /
+                                                                  ((m.rows_per_plane * m.nu) << m.fp_shift)));
+    const double passes = blocks * (std::ceil(B / max_fp) + std::ceil(B / dev::kMaxFusedBp) - 1.0) + 1.0;
+    const double rays = n * m.rows_per_plane * m.nu * m.fp_n * (nx + nz) * cu_planes;
+    if (over_) {
+        c.passes = vec_ ? 11.0 * passes + plane * n * (8.3e-4 + 1.9e-4 * samples) + 5e-6 * rays
+                        : 10.5 * passes + plane * (3e-4 * passes + n * (8e-4 + 3.5e-4 * samples)) + 1.5e-5 * rays +
+                              0.8 * passes * mega;
+    } else {
+        const bool one_x = vec_ && dev::kMaxThreads % (m.nx / 4) == 0;
+        c.passes = 12.5 * passes + plane * n * (one_x ? (mask ? 3.6e-4 : 3.1e-4) : (mask ? 8.3e-4 : 5.8e-4)) +
+                   1e-5 * rays + (one_x ? 0.0 : 0.7 * passes * mega);
+    }
+
+    // The sweeps: launches; rounds of the workgroups that the CUs hold, back (tiles of
+    // 64 columns, 4 planes and 64 slices, 16 with samples or a mask) for every
+    // projection, forward for their staged planes and their rays' steps; the planes
+    // read for the detector's rows.
+    auto rounds = [](double workgroups, int held) {
+        const double r = workgroups / held;
+        return r < 3.0 ? std::max(1.0, std::ceil(r)) : r + 0.5;
+    };
+    const int slices = sampled ? 16 : 64;
+    const double back = rounds((double)((m.nx + 63) / 64) * ((m.ny + 3) / 4) * ((m.nz + slices - 1) / slices),
+                               (sampled ? 4 : 3) * 256);
+    const double sweeps = blocks * std::ceil(B / dev::kSweepForward);
+    const int rows = std::max(1, m.nv - m.ndead);
+    const dev::ForwardShape f = dev::sweep_forward_shape(m.nx, (int)std::ceil(n / sweeps), (uint32_t)m.nu, (uint32_t)rows,
+                                                         m.fp_n, mask);
+    const double forward = sweeps * rounds(f.workgroups, f.rays > 4 ? 256 : 512);
+    const double staged = forward * f.planes * nx * nz, steps = forward * f.rays * (nx + nz);
+    const double read = 1e-6 * sweeps * nx * nz * rows * (mask ? 2.0 : 1.0);
+    if (over_)
+        c.sweeps = 1.5 * blocks + 8.0 * sweeps + n * back * (3.2 + 1.33 * samples) + 1.47e-4 * staged + 0.012 * steps +
+                   1.28 * read;
+    else if (mask)
+        c.sweeps = 6.5 * blocks + 4.8 * sweeps + 2.55 * n * back + 2.6e-4 * staged + 0.0035 * steps + 0.85 * read;
+    else if (vt_ != ETN_VOXEL_FLOAT32)   // (half as wide loads and stores, a rounding a projection)
+        c.sweeps = 18.0 * blocks + 2.9 * sweeps + back * (4.5 * n + 2.1 * blocks) + 1e-4 * staged + 0.0038 * steps +
+                   2.45 * read;
+    else
+        c.sweeps = 7.4 * blocks + 8.5 * sweeps + 4.2 * n * back + 1.47e-4 * staged + 0.0029 * steps + 1.26 * read;
+    return c;
+}
+
 // Where the sweeps are the faster (fused passes against sweeps, us for 31 tilts,
 // f32 unless 16 bits are named).  They are two or three launches a block of 10 to
 // 20 us each, whose workgroups own whole tiles of 64 columns and 64 slices (16
 // with samples or a mask): small volumes do not fill the launches, narrow and flat
 // ones the tiles.  A fused pass lasts as long as a CU's planes do.
-bool FusedEngineImpl::sweepsPay(const MemberPlan& m, bool plain) const
+bool FusedEngineImpl::sweepsPay(const MemberPlan& m) const
 {
     const size_t voxels = (size_t)m.nx * m.ny * m.nz;
+    // below these no estimate is asked
+    if (over_ ? voxels < (m.bp_samples > 1 ? (size_t)500000 : (size_t)1 << 23)
+        : m.mask ? m.bmax < 8 || voxels < (size_t)1 << 19
+                 : m.bmax < 4 || voxels < (size_t)1 << (m.bmax < 8 ? 23 : 21))
+        return false;
+    // Fused workgroups with more than two rays a thread (four without samples) fall
+    // far behind: 512 x 384 x 32 on 768 x 768 rows of half pitch, 9 samples 48.0 / 5.4 ms
+    if ((m.rows_per_plane * m.nu) << m.fp_shift > dev::kMaxThreads * (over_ ? 2 : 4)) return true;
+    // estimates that are further apart than they scatter decide (200 x 69 x 614 half in
+    // blocks of 4 2216 / 858, 384 x 300 x 384 3882 / 1851; 32 x 96 x 512, 9 samples in one
+    // block 1269 / 631), the lines below where they are closer: with 1.3 for 1.4,
+    // 1000 x 1000 x 16 bf16 in blocks of 4 1498 / 1972
+    const SplitCost c = splitCost(m);
+    if (c.passes > 1.4 * c.sweeps) return true;
+    if (over_ && c.sweeps > 1.25 * c.passes) return false;
     const double cu_work = (double)m.nx * m.nz * std::max(1.0, m.ny / 256.0);
     const bool half = vt_ != ETN_VOXEL_FLOAT32;
-    if (plain) {
+    if (!over_ && !m.mask) {
         // up to 128 columns: 64 x 256 x 128 167 / 236, 128 x 160 x 128 245 / 279,
         // 128^3 244 / 244, 64 x 512 x 256 314 / 306, 128 x 128 x 256 413 / 304; beyond,
         // where the fused passes' rows are no power of two or fill a workgroup with
@@ -614,30 +693,28 @@ bool FusedEngineImpl::sweepsPay(const MemberPlan& m, bool plain) const
         // 64 x 512 x 256 330 / 349, 96 x 512 x 256 685 / 593, 112 x 200 x 200 436 / 350,
         // 512 x 512 x 32 503 / 509, x 48 647 / 542, 520 x 70 x 64 801 / 285;  of 16:
         // 64 x 512 x 256 348 / 300, 512 x 512 x 16 398 / 391
-        if (m.bmax >= (half ? 16u : 8u)) return m.nx >= 48 && m.nz >= 16 && voxels >= (size_t)1 << 21;
+        if (m.bmax >= (half ? 16u : 8u)) return m.nx >= 48 && m.nz >= 16;
         if (m.bmax >= 8) return m.nx >= 96 && m.nz >= 48 && voxels >= (size_t)2200000;
         // blocks of 4: 256^3 841 / 718, 128 x 512 x 256 630 / 688 (of 5 698 / 664),
         // 512 x 512 x 32 480 / 493, x 48 612 / 566; 256^3 on a detector of 128^2 616 / 657
         // (the fused pass traces fewer rays);  of 2: 256^3 1115 / 1328.  16 bits, of 4:
         // 256^3 874 / 919;  of 5: 256^3 912 / 875, 512 x 512 x 128 1350 / 1346;  of 6:
         // 128 x 512 x 256 669 / 778, 512 x 512 x 48 636 / 685, x 64 774 / 732
-        if (m.bmax < 4 || voxels < (size_t)1 << 23 || 4 * (size_t)m.nu < 3 * (size_t)m.nx) return false;
+        if (4 * (size_t)m.nu < 3 * (size_t)m.nx) return false;
         if (!half) return m.nx >= (m.bmax < 5 ? 129 : 96) && m.nz >= 48;
         return m.bmax >= 5 && m.nx > 128 && m.nz >= (m.bmax < 6 ? 128 : 64);
     }
     // masked, blocks of 8: 96^3 408 / 279, 256^3 1053 / 937, 32 x 512 x 256 220 / 267,
     // 40 x 200 x 200 234 / 150, 64 x 128 x 64 120 / 128, 128 x 512 x 8 108 / 113, 512 x 512 x 8 287 / 196;
     // of 4: 128^3 409 / 430
-    if (!over_)
-        return m.bmax >= 8 && m.nx >= 40 && voxels > (size_t)1 << (m.nz < 16 ? 20 : 19);
+    if (!over_) return m.nx >= 40 && voxels > (size_t)1 << (m.nz < 16 ? 20 : 19);
     // tiles at least 5/8 full: 32 x 512 x 256, 4 samples, 863 / 1388;
     // 132 x 1000 x 20, 9 samples, 1297 / 1773 (0.43 full)
     const size_t tiles = (size_t)((m.nx + 63) / 64 * 64) * ((m.nz + 15) / 16 * 16) * m.ny;
     if (8 * voxels < 5 * tiles) return false;
     // forward sub-rays alone: 4 x 4 96^3 684 / 718, 204^3 1987 / 1803;
     // 2 x 2 204^3 1500 / 1584, 256^3 2009 / 1958, in blocks of 8 204^3 1299 / 588
-    if (m.bp_samples == 1) return voxels >= (size_t)1 << (m.fp_n == 2 && m.bmax == 1 ? 24 : 23);
-    if (voxels < 500000) return false;
+    if (m.bp_samples == 1) return m.fp_n > 2 || m.bmax > 1 || voxels >= (size_t)1 << 24;
     // 9 samples: 80^3 with a mask 1009 / 884;  4 samples, blocks of 2: 96^3 554 / 510
     if (m.bp_samples > 4 || m.bmax > 1) return true;
     // 4 samples, SART: 96^3 745 / 752, 104^3 845 / 809, 128^3 1119 / 917;
@@ -674,7 +751,7 @@ void FusedEngineImpl::plan_split(hipStream_t stream)
     if (members_.size() != 1 || exact_ || sr_ || cap_ || !reg_bp_) return;
     const MemberPlan& m = members_[0];
     const bool plain = !over_ && !m.mask;
-    if (!sweepsPay(m, plain)) return;
+    if (!sweepsPay(m)) return;
     BlockIterativeReconstructionOperator& op = *m.op;
     GpuVolume* vol = op.getReconstructedVolume();
     const VolumeProperties vp = whole_volume(vol->properties());

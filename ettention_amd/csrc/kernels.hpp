@@ -96,6 +96,12 @@ constexpr int kSweepForward = 8;    // projections of a sweep
 // the same steps in every row, rays below the 2048-step limit); sub: sub-rays
 // along each pixel axis.
 bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, uint32_t nv, int sub, bool masked);
+// Launch of a forward sweep of n views: volume planes (detector rows) a workgroup,
+// ray columns a thread, workgroups.
+struct ForwardShape {
+    int planes, rays, workgroups;
+};
+ForwardShape sweep_forward_shape(int nx, int n, uint32_t nu, uint32_t nv, int sub, bool masked);
 // Forward-projects n <= kSweepForward views (device memory) whose rays move in
 // the z direction zdir (or stay in z) in one sweep of the volume, with the fused
 // kernels' fast arithmetic, operation for operation.  mask: prior-knowledge mask

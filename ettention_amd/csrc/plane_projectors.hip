@@ -1018,20 +1018,15 @@ __global__ void __launch_bounds__(kFpThreads, R <= 4 ? 4 : 2)
 }
 
 template <typename S, bool kVec, bool kMask, int P>
-void launch_sweep_forward(const SlabParams& s, SweepForward a, const void* volume, hipStream_t stream)
+void launch_sweep_forward(const SlabParams& s, SweepForward a, const ForwardShape& shape, const void* volume,
+                          hipStream_t stream)
 {
     constexpr int T = kFpThreads;
     const auto* vol = static_cast<const typename S::T*>(volume);
-    const int columns = a.n * (a.nu << a.shift);
     a.groups = (a.nv + P - 1) / P;
-    // columns a thread: as many as there are, fewer where that leaves a CU fewer
-    // than two workgroups (512 x 512 x 256, eight projections: 167 us a sweep
-    // with two a CU, 175 with one)
-    int rays = 8;
-    while (rays > 1 && (rays / 2 * T >= columns || a.groups * ((columns + rays * T - 1) / (rays * T)) < 512)) rays /= 2;
     a.band = std::max(1, std::min(s.res[2], kFpLds / (s.res[0] * P * (kMask ? 2 : 1))));
-    const unsigned grid = (unsigned)(a.groups * ((columns + rays * T - 1) / (rays * T)));
-    auto launch = [&](auto kernel) { kernel<<<grid, T, 0, stream>>>(s, a, vol); };
+    auto launch = [&](auto kernel) { kernel<<<(unsigned)shape.workgroups, T, 0, stream>>>(s, a, vol); };
+    const int rays = shape.rays;
     if (rays == 1) launch(sweep_forward_kernel<S, kVec, kMask, P, 1>);
     else if (rays == 2) launch(sweep_forward_kernel<S, kVec, kMask, P, 2>);
     else if (rays == 4) launch(sweep_forward_kernel<S, kVec, kMask, P, 4>);
@@ -1041,25 +1036,16 @@ void launch_sweep_forward(const SlabParams& s, SweepForward a, const void* volum
 template <typename S, bool kMask>
 void sweep_forward_typed(const SlabParams& s, const SweepForward& a, const void* volume, hipStream_t stream)
 {
-    const int nx = s.res[0], w = kMask ? 2 : 1;
-    const bool vec = nx % 4 == 0 && reinterpret_cast<uintptr_t>(volume) % (4 * sizeof(typename S::T)) == 0 &&
+    const bool vec = s.res[0] % 4 == 0 && reinterpret_cast<uintptr_t>(volume) % (4 * sizeof(typename S::T)) == 0 &&
                      reinterpret_cast<uintptr_t>(a.mask) % 4 == 0;
-    // planes a workgroup: four where they and the columns still make a
-    // workgroup for every CU (two planes: 240 us), fewer on small volumes; a
-    // voxel's values and weights are one 16-byte read
-    auto fills = [&](int P) {
-        const int columns = a.n * (a.nu << a.shift);
-        return nx * P * w <= kFpLds &&
-               (a.nv + P - 1) / P * ((columns + kFpThreads - 1) / kFpThreads) >= 256;
-    };
-    const int P = !kMask && fills(4) ? 4 : fills(2) ? 2 : 1;
+    const ForwardShape shape = sweep_forward_shape(s.res[0], a.n, (uint32_t)a.nu, (uint32_t)a.nv, a.sub, kMask);
     auto launch = [&](auto v) {
         constexpr bool kVec = decltype(v)::value;
         if constexpr (!kMask) {
-            if (P == 4) return launch_sweep_forward<S, kVec, kMask, 4>(s, a, volume, stream);
+            if (shape.planes == 4) return launch_sweep_forward<S, kVec, kMask, 4>(s, a, shape, volume, stream);
         }
-        if (P == 2) launch_sweep_forward<S, kVec, kMask, 2>(s, a, volume, stream);
-        else launch_sweep_forward<S, kVec, kMask, 1>(s, a, volume, stream);
+        if (shape.planes == 2) launch_sweep_forward<S, kVec, kMask, 2>(s, a, shape, volume, stream);
+        else launch_sweep_forward<S, kVec, kMask, 1>(s, a, shape, volume, stream);
     };
     if (vec) launch(std::true_type{});
     else launch(std::false_type{});
@@ -1427,6 +1413,26 @@ bool forward_view_fits(const SlabParams& s, const ForwardView& v, uint32_t nu, u
     r.samples = 1;
     if (sub < 1 || sub > 4 || nu > 1u << 20 || nv > 1u << 20 || s.res[1] > 65535) return false;
     return s.res[0] * (masked ? 2 : 1) <= kFpLds && plane_geometry_fits(s, r, sub);
+}
+
+ForwardShape sweep_forward_shape(int nx, int n, uint32_t nu, uint32_t nv, int sub, bool masked)
+{
+    int shift = 0;
+    while (1 << shift < sub) ++shift;
+    const int columns = n * (int)(nu << shift), w = masked ? 2 : 1;
+    auto groups = [&](int planes) { return ((int)nv + planes - 1) / planes; };
+    auto slices = [&](int rays) { return (columns + rays * kFpThreads - 1) / (rays * kFpThreads); };
+    // planes a workgroup: four where they and the columns still make a
+    // workgroup for every CU (two planes: 240 us), fewer on small volumes; a
+    // voxel's values and weights are one 16-byte read
+    auto fills = [&](int planes) { return nx * planes * w <= kFpLds && groups(planes) * slices(1) >= 256; };
+    ForwardShape f{!masked && fills(4) ? 4 : fills(2) ? 2 : 1, 8, 0};
+    // columns a thread: as many as there are, fewer where that leaves a CU fewer
+    // than two workgroups (512 x 512 x 256, eight projections: 167 us a sweep
+    // with two a CU, 175 with one)
+    while (f.rays > 1 && (f.rays / 2 * kFpThreads >= columns || groups(f.planes) * slices(f.rays) < 512)) f.rays /= 2;
+    f.workgroups = groups(f.planes) * slices(f.rays);
+    return f;
 }
 
 void sweep_forward_project(const SlabParams& s, const ForwardView* views, int n, int zdir, uint32_t nu, uint32_t nv,

@@ -224,7 +224,7 @@ def test_residual_norm_of_sweeps(shape, block, fp, masked, voxel):
     ((128, 160, 128), 8, "float", 1, 1, False, FUSED), ((128, 128, 132), 8, "float", 1, 1, False, SWEEPING),
     ((32, 512, 300), 8, "float", 1, 1, False, FUSED), ((48, 400, 300), 8, "float", 1, 1, False, SWEEPING),
     ((256, 256, 32), 8, "float", 1, 1, False, SWEEPING), ((512, 512, 8), 8, "float", 1, 1, False, FUSED),
-    ((80, 256, 256), 8, "half", 1, 1, False, FUSED), ((112, 200, 200), 8, "half", 1, 1, False, SWEEPING),
+    ((64, 512, 256), 8, "half", 1, 1, False, FUSED), ((112, 200, 200), 8, "half", 1, 1, False, SWEEPING),
     ((512, 256, 32), 8, "bfloat16", 1, 1, False, FUSED), ((512, 256, 48), 8, "bfloat16", 1, 1, False, SWEEPING),
     ((64, 256, 300), 16, "bfloat16", 1, 1, False, SWEEPING), ((128, 256, 256), 4, "float", 1, 1, False, FUSED),
     ((256, 512, 64), 4, "float", 1, 1, False, SWEEPING), ((256, 512, 64), 4, "bfloat16", 1, 1, False, FUSED),
@@ -232,7 +232,10 @@ def test_residual_norm_of_sweeps(shape, block, fp, masked, voxel):
     ((96, 96, 96), 8, "float", 1, 1, True, SWEEPING), ((96, 96, 96), 1, "float", 2, 4, False, FUSED),
     ((104, 104, 104), 1, "float", 2, 4, False, SWEEPING), ((132, 1000, 20), 1, "float", 1, 9, False, FUSED),
     ((200, 400, 32), 1, "float", 1, 4, False, FUSED), ((204, 204, 204), 1, "float", 2, 1, False, FUSED),
-    ((204, 204, 204), 1, "float", 3, 1, False, SWEEPING)])
+    ((204, 204, 204), 1, "float", 3, 1, False, SWEEPING),
+    # estimates far apart, more than two rays a thread
+    ((200, 69, 614), 4, "half", 1, 1, False, SWEEPING), ((32, 96, 512), 16, "float", 3, 9, False, SWEEPING),
+    ((132, 1000, 20), 1, "bfloat16", 4, 9, True, FUSED), ((512, 96, 48), 1, "half", 3, 16, False, SWEEPING)])
 def test_sweeps_where_they_pay(shape, block, voxel, fp, bp, masked, kernel):
     nx, ny, nz = shape
     case = dict(volume=E.VolumeGeometry.make(shape), base_geometry=E.ScannerGeometry.mrc_base(nx, ny),
